@@ -1,0 +1,48 @@
+"""GPU parity of the CDM kernels at the edges of their tiles and of the size
+ranges their launches choose between, against the oracle."""
+import numpy as np
+import pytest
+
+from conftest import smooth_volume
+
+pytestmark = pytest.mark.gpu
+
+
+def _field(shape, seed, scale=2.0, zero_frac=0.2):
+    from scipy.ndimage import gaussian_filter
+    r = np.random.default_rng(seed)
+    d = gaussian_filter(r.standard_normal(shape + (3,)), (2, 2, 2, 0)).astype(np.float32) * scale
+    d[r.random(shape) < zero_frac] = 0.0
+    return d
+
+
+def _bits_equal(a, b):
+    return np.array_equal(np.asarray(a, np.float32).view(np.uint32),
+                          np.asarray(b, np.float32).view(np.uint32))
+
+
+@pytest.mark.parametrize("shape", [(1, 1, 1), (4, 4, 16), (5, 5, 17), (3, 3, 15), (9, 4, 33),
+                                   (2, 11, 31), (6, 7, 2), (13, 12, 66)])
+def test_gradient_tile_edges(ctx, oracle, shape):
+    """Shapes that end on, before and after a 16 x 4 x 4 tile, rows that start
+    at every alignment, full-range bytes: bit for bit the oracle's."""
+    r = np.random.default_rng(sum(shape))
+    Js = r.integers(0, 256, shape).astype(np.uint8)
+    It = np.clip(Js.astype(int) + r.integers(-60, 61, shape), 0, 255).astype(np.uint8)
+    nd, c = ctx.gradient(Js, It, "r")
+    nd_o, c_o = oracle.gradient(Js, It, "r")
+    assert _bits_equal(nd, nd_o)
+    # the cost is a sum of at most n terms in another order, rounded to float
+    assert abs(c - c_o) <= 2.0 ** -23 * max(abs(c_o), 1e-30)
+
+
+def test_cdm_odd_levels_two_modalities(ctx, oracle):
+    """A pyramid whose second modality's half-size images start at an odd
+    multiple of two bytes."""
+    shape = (33, 37, 41)
+    A = [smooth_volume(shape, s) for s in (1, 2)]
+    B = [smooth_volume(shape, s) for s in (3, 4)]
+    ok, want, _ = oracle.cdm(A, B)
+    rc, got, _ = ctx.cdm([ctx.volume(v) for v in A], [ctx.volume(v) for v in B])
+    assert ok and rc == 0
+    assert float(np.sqrt(((got - want) ** 2).sum(-1).mean())) <= 0.01
