@@ -46,3 +46,28 @@ def test_cdm_odd_levels_two_modalities(ctx, oracle):
     rc, got, _ = ctx.cdm([ctx.volume(v) for v in A], [ctx.volume(v) for v in B])
     assert ok and rc == 0
     assert float(np.sqrt(((got - want) ** 2).sum(-1).mean())) <= 0.01
+
+
+@pytest.mark.parametrize("shape", [(1, 1, 1), (8, 8, 8), (9, 7, 17), (1, 3, 40), (40, 2, 1), (16, 24, 8),
+                                   (33, 20, 25)])
+def test_poisson_four_sweep_tiles(ctx, oracle, shape):
+    """Volumes around the 8 x 8 x 8 tile of the four-sweep launch, thinner than
+    its halo, and with rows shorter than it: 4, 8 and 12 sweeps, and
+    remainders after four-sweep launches."""
+    nd = _field(shape, 21, 1.0, 0.0)
+    for sweeps in (4, 12, 5, 6, 8, 11):
+        out, ml = ctx.poisson(nd, sweeps)
+        want = oracle.poisson(nd, sweeps)
+        assert _bits_equal(out, want), sweeps
+        assert ml == oracle.max_length(want)
+
+
+def test_poisson_sweeps_per_launch_by_size(ctx, oracle):
+    """The largest volume that takes four sweeps a launch and the next one
+    that takes two."""
+    for shape in ((64, 128, 128), (64, 128, 129)):
+        nd = np.random.default_rng(5).standard_normal(shape + (3,)).astype(np.float32)
+        out, ml = ctx.poisson(nd, 12)
+        want = oracle.poisson(nd, 12)
+        assert _bits_equal(out, want)
+        assert ml == oracle.max_length(want)

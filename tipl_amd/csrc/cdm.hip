@@ -464,6 +464,10 @@ __global__ __launch_bounds__(1024) void max_reduce_kernel(const float* __restric
 // ---------------------------------------------------------------------------
 constexpr float kInvD2 = -0.5f / 3.0f;
 
+// Volumes of at most this many voxels take four sweeps a launch
+// (poisson4_kernel), larger ones two (poisson2_kernel).
+constexpr size_t kPoisson4Voxels = size_t(1) << 20;
+
 template <bool FIRST, bool MAXLEN>
 __global__ __launch_bounds__(256) void poisson_kernel(const float* __restrict__ nd,
                                                       const float* __restrict__ a, FieldGeo g,
@@ -801,6 +805,129 @@ __global__ __launch_bounds__(kQX * kQY) void poisson2_kernel(const float* __rest
                                                              float* __restrict__ maxparts)
 {
     poisson2_body<FIRST, MAXLEN>(nd, a, g, zq, b, maxparts, logical_block());
+}
+
+// ---------------------------------------------------------------------------
+// Four Jacobi sweeps per launch for small volumes.  The three components of
+// the field are independent in cdm_solve_poisson, so a workgroup takes one
+// component of one 8 x 8 x 8 tile, grown by 4 on every side to 16 x 16 x 16.
+// Thread (lx, ly) holds its 16-voxel z column of the iterate and of new_d in
+// registers: the p-+wh neighbours are its own registers, p-+1 come from the
+// neighbouring lanes of its 16-lane row (DPP), p-+w from an LDS copy of the
+// planes.  A sweep spoils one layer of the grown tile, so after four the
+// 8 x 8 x 8 core is exact.  Offsets are flat-index offsets as in
+// poisson2_kernel (row and plane wrap included); positions outside [0, n)
+// read 0 through the buffer's range check and are kept 0, which is the
+// reference's dropped neighbour.
+// What bounds it is latency -- one round of loads, four barriers -- where
+// poisson2_kernel chains a barrier pair and a load per plane.  Twelve sweeps:
+// 44 -> 17 us at 32x32x32 and below, 45 -> 21 at 40x48x40, 75 -> 68 at
+// 80x96x80, where the halo's work (eight times the core's) takes over.
+// ---------------------------------------------------------------------------
+constexpr int kCT = 8, kCH = 4, kCL = kCT + 2 * kCH;  // tile, halo (= sweeps), grown tile
+constexpr int kCThreads = kCL * kCL;
+static_assert(kCL == 16, "a tile row is one DPP row");
+
+inline bool poisson4_fits(const FieldGeo& g) { return g.n <= kPoisson4Voxels; }
+
+uint32_t poisson4_blocks(const FieldGeo& g)
+{
+    return 3u * uint32_t((g.w + kCT - 1) / kCT) * uint32_t((g.h + kCT - 1) / kCT) *
+           uint32_t((g.d + kCT - 1) / kCT);
+}
+
+template <bool FIRST>
+__device__ __forceinline__ void poisson4_body(const float* __restrict__ nd, const float* __restrict__ a,
+                                              const FieldGeo& g, float* __restrict__ b, uint32_t blk)
+{
+    __shared__ float plane[2][kCL][kCL + 2][kCL];  // rows -1 .. 16 of every plane
+    const int tid = int(threadIdx.x), lx = tid & (kCL - 1), ly = tid / kCL;
+    const uint32_t gx = uint32_t((g.w + kCT - 1) / kCT), gy = uint32_t((g.h + kCT - 1) / kCT);
+    const uint32_t comp = blk % 3u, tile = blk / 3u;
+    const int x0 = int(tile % gx) * kCT, y0 = int((tile / gx) % gy) * kCT, z0 = int(tile / (gx * gy)) * kCT;
+    const int w = g.w, wh = int(g.wh), n = int(g.n);
+    const int q0 = (z0 - kCH) * wh + (y0 - kCH) * w + (x0 - kCH);  // the grown tile's first voxel
+    const int q = q0 + ly * w + lx;
+    const __amdgpu_buffer_rsrc_t rn = make_rsrc(nd, g.n * 12u);
+    const __amdgpu_buffer_rsrc_t ra = make_rsrc(FIRST ? nd : a, g.n * 12u);
+    auto load = [&](__amdgpu_buffer_rsrc_t rs, int k) {
+        return __uint_as_float(
+            __builtin_amdgcn_raw_buffer_load_b32(rs, (q + k * wh) * 12 + int(comp) * 4, 0, 0));
+    };
+    float r[kCL], v[kCL];
+#pragma unroll
+    for (int k = 0; k < kCL; ++k) r[k] = load(rn, k);
+    if constexpr (FIRST) {
+#pragma unroll
+        for (int k = 0; k < kCL; ++k) v[k] = r[k] * kInvD2;
+    } else {
+#pragma unroll
+        for (int k = 0; k < kCL; ++k) v[k] = load(ra, k);
+    }
+    // tiles that reach past either end of the array keep those positions 0
+    const bool ends = q0 < 0 || q0 + (kCL - 1) * (1 + w + wh) >= n;
+    uint32_t inside = 0;
+#pragma unroll
+    for (int k = 0; k < kCL; ++k) inside |= uint32_t(q + k * wh >= 0 && q + k * wh < n) << k;
+#pragma unroll
+    for (int s = 1; s <= kCH; ++s) {
+        float(*pl)[kCL + 2][kCL] = plane[s & 1];
+#pragma unroll
+        for (int k = s; k < kCL - s; ++k) pl[k][ly + 1][lx] = v[k];
+        __syncthreads();
+        float below = v[s - 1];
+#pragma unroll
+        for (int k = s; k < kCL - s; ++k) {
+            const float c = v[k];
+            const float xm = dpp_prev(c), xp = dpp_next(c);
+            float t = r[k] - xm;
+            t = t - xp;
+            t = t - pl[k][ly][lx];
+            t = t - pl[k][ly + 2][lx];
+            t = t - below;
+            t = t - v[k + 1];
+            t = t * kInvD2;
+            below = c;
+            v[k] = t;
+        }
+        if (ends) {
+#pragma unroll
+            for (int k = s; k < kCL - s; ++k) v[k] = (inside >> k) & 1u ? v[k] : 0.0f;
+        }
+    }
+    if (lx < kCH || lx >= kCH + kCT || ly < kCH || ly >= kCH + kCT) return;
+    if (x0 + lx - kCH >= w || y0 + ly - kCH >= g.h) return;
+#pragma unroll
+    for (int k = kCH; k < kCH + kCT; ++k)
+        if (z0 + k - kCH < g.d) b[3 * size_t(q + k * wh) + comp] = v[k];
+}
+
+template <bool FIRST>
+__global__ __launch_bounds__(kCThreads) void poisson4_kernel(const float* __restrict__ nd,
+                                                             const float* __restrict__ a, FieldGeo g,
+                                                             float* __restrict__ b)
+{
+    poisson4_body<FIRST>(nd, a, g, b, xcd_remap(blockIdx.x, gridDim.x));
+}
+
+// cdm_max_displacement_length of a whole field: per-block maxima.
+constexpr uint32_t kMaxLenBlocks = 128;
+
+__global__ __launch_bounds__(256) void max_length_kernel(const float* __restrict__ d, uint32_t n,
+                                                         float* __restrict__ maxparts)
+{
+    float m = 0.0f;
+    for (uint32_t p = blockIdx.x * 256u + threadIdx.x; p < n; p += gridDim.x * 256u) {
+        const float3 r = ld3(d, p);
+        float s2 = r.x * r.x + r.y * r.y;
+        s2 = s2 + r.z * r.z;
+        m = fmaxf(m, float(sqrt(double(s2))));
+    }
+    m = wave_max_f32(m);
+    __shared__ float part[4];
+    if ((threadIdx.x & 63u) == 0) part[threadIdx.x >> 6] = m;
+    __syncthreads();
+    if (threadIdx.x == 0) maxparts[blockIdx.x] = fmaxf(fmaxf(part[0], part[1]), fmaxf(part[2], part[3]));
 }
 
 // ---------------------------------------------------------------------------
@@ -1221,10 +1348,12 @@ void launch_gradient(tiplhip_ctx* ctx, const uint8_t* Js, const uint8_t* It, con
     TIPLHIP_CHECK(hipGetLastError());
 }
 
-// `sweeps` Jacobi sweeps, two per launch (poisson2_kernel) and a single
+// `sweeps` Jacobi sweeps: four per launch while the volume is small
+// (poisson4_kernel), two per launch (poisson2_kernel) otherwise, and a single
 // z-marching sweep for an odd remainder; returns the buffer holding the
-// result.  With maxlen, the last launch also forms per-block maxima of the
-// displacement length and max_reduce_kernel writes their maximum.
+// result.  With maxlen, per-block maxima of the displacement length (from the
+// last launch, or a pass of their own after a four-sweep one) are reduced by
+// max_reduce_kernel.
 float* launch_poisson(tiplhip_ctx* ctx, const float* nd, float* a, float* b, const FieldGeo& g,
                       int sweeps, unsigned int* maxlen, float* maxparts)
 {
@@ -1234,6 +1363,23 @@ float* launch_poisson(tiplhip_ctx* ctx, const float* nd, float* a, float* b, con
     int done = 0;
     while (done < sweeps) {
         const bool first = done == 0;
+        if (sweeps - done >= kCH && poisson4_fits(g)) {
+            const dim3 grid(poisson4_blocks(g)), block(kCThreads);
+            if (first)
+                hipLaunchKernelGGL(poisson4_kernel<true>, grid, block, 0, ctx->stream, nd, src, g, dst);
+            else
+                hipLaunchKernelGGL(poisson4_kernel<false>, grid, block, 0, ctx->stream, nd, src, g, dst);
+            TIPLHIP_CHECK(hipGetLastError());
+            done += kCH;
+            if (done == sweeps && maxlen) {
+                last_blocks = std::min(kMaxLenBlocks, block_count(g));
+                hipLaunchKernelGGL(max_length_kernel, dim3(last_blocks), dim3(256), 0, ctx->stream, dst,
+                                   g.n, maxparts);
+                TIPLHIP_CHECK(hipGetLastError());
+            }
+            std::swap(src, dst);
+            continue;
+        }
         const bool pair = sweeps - done >= 2;
         const bool last = done + (pair ? 2 : 1) == sweeps && maxlen;
         if (pair) {

@@ -271,6 +271,16 @@ __device__ inline uint32_t xcd_remap(uint32_t b, uint32_t total)
     return xcd * q + (xcd < r ? xcd : r) + slot;
 }
 
+// The value of the previous / next lane of a 16-lane row (0 past its ends).
+__device__ inline float dpp_prev(float v)
+{
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x111, 0xf, 0xf, true));
+}
+__device__ inline float dpp_next(float v)
+{
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x101, 0xf, 0xf, true));
+}
+
 __device__ inline uint64_t wave_sum_u64(uint64_t v)
 {
     for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, kWave);
