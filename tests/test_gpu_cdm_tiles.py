@@ -62,12 +62,26 @@ def test_poisson_four_sweep_tiles(ctx, oracle, shape):
         assert ml == oracle.max_length(want)
 
 
-def test_poisson_sweeps_per_launch_by_size(ctx, oracle):
-    """The largest volume that takes four sweeps a launch and the next one
-    that takes two."""
-    for shape in ((64, 128, 128), (64, 128, 129)):
-        nd = np.random.default_rng(5).standard_normal(shape + (3,)).astype(np.float32)
-        out, ml = ctx.poisson(nd, 12)
-        want = oracle.poisson(nd, 12)
+@pytest.mark.parametrize("shape", [(64, 64, 64), (64, 64, 65), (3, 300, 301), (300, 3, 301), (301, 300, 3),
+                                   (70, 57, 113), (90, 48, 112)])
+def test_poisson_marched_tiles(ctx, oracle, shape):
+    """The largest volume on 8 x 8 x 8 tiles and larger ones that march z:
+    thinner than the halo along each axis, and with rows and planes ending on
+    and inside the 56 x 24 core of a column.  13 sweeps end in a single one."""
+    nd = np.random.default_rng(5).standard_normal(shape + (3,)).astype(np.float32)
+    for sweeps in (12, 13):
+        out, ml = ctx.poisson(nd, sweeps)
+        want = oracle.poisson(nd, sweeps)
         assert _bits_equal(out, want)
         assert ml == oracle.max_length(want)
+
+
+@pytest.mark.parametrize("shape", [(21, 30, 27), (61, 67, 71)])
+def test_level_iterations_by_size(ctx, oracle, shape):
+    """The loop's planar gradient fields, on each side of the size where the
+    Poisson kernel changes: the oracle's step functions in the loop's order."""
+    from test_gpu_cdm import _pair, oracle_level_iterations
+    It, Is = _pair(shape, 31)
+    want = oracle_level_iterations(oracle, It, Is, 4)
+    got = ctx.cdm_level_iterations(ctx.volume(It), ctx.volume(Is), 4, want_field=True)
+    assert _bits_equal(got, want)

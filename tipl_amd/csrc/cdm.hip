@@ -41,6 +41,32 @@
 namespace tiplhip {
 namespace {
 
+// Where a gradient field (new_d and its Jacobi iterates) keeps component c of
+// voxel p: element p * ps + c * cs.  The loops keep these fields planar (one
+// array per component), so that kernels which take one component each read
+// whole lines: twelve sweeps 269 -> 204 us at 182x218x182, 120 against 216 at
+// 160x192x160.  Packed like the displacement fields where a caller's buffer
+// is, and where 12 n reaches 2^31.
+struct Lay {
+    uint32_t ps, cs;
+};
+inline Lay packed_layout() { return Lay{3u, 1u}; }
+inline bool planar_fits(const FieldGeo& g) { return size_t(g.n) * 12 < (size_t(1) << 31); }
+inline Lay grad_layout(const FieldGeo& g) { return planar_fits(g) ? Lay{1u, g.n} : packed_layout(); }
+
+__device__ inline float3 ld_lay(const float* f, uint32_t p, const Lay& l)
+{
+    const size_t i = size_t(p) * l.ps;
+    return make_float3(f[i], f[i + l.cs], f[i + 2 * size_t(l.cs)]);
+}
+__device__ inline void st_lay(float* f, uint32_t p, const Lay& l, float3 v)
+{
+    const size_t i = size_t(p) * l.ps;
+    f[i] = v.x;
+    f[i + l.cs] = v.y;
+    f[i + 2 * size_t(l.cs)] = v.z;
+}
+
 // ---------------------------------------------------------------------------
 // compose_displacement: Js(x) = Is(x + d(x)); exact copy where d(x) == 0.
 // ---------------------------------------------------------------------------
@@ -78,7 +104,7 @@ __global__ __launch_bounds__(256) void compose_kernel(const uint8_t* __restrict_
 template <char TYPE>
 __global__ __launch_bounds__(256) void gradient_kernel(const uint8_t* __restrict__ Js,
                                                        const uint8_t* __restrict__ It, FieldGeo g,
-                                                       int accumulate, float* __restrict__ nd,
+                                                       int accumulate, float* __restrict__ nd, Lay lay,
                                                        double* __restrict__ partials)
 {
     const Vox v = this_voxel(g);
@@ -147,13 +173,13 @@ __global__ __launch_bounds__(256) void gradient_kernel(const uint8_t* __restrict
             gr.z = 0.0f + gz * s;
         }
         if (accumulate) {
-            float3 o = ld3(nd, v.p);
+            float3 o = ld_lay(nd, v.p, lay);
             o.x = o.x + gr.x;
             o.y = o.y + gr.y;
             o.z = o.z + gr.z;
-            st3(nd, v.p, o);
+            st_lay(nd, v.p, lay, o);
         } else {
-            st3(nd, v.p, gr);
+            st_lay(nd, v.p, lay, gr);
         }
     }
     // deterministic per-block partial sum of the cost map
@@ -226,7 +252,7 @@ template <int TY, int TZ, int NT>
 __device__ __forceinline__ void gradient_r_box_body(const uint8_t* __restrict__ Js,
                                                     const uint8_t* __restrict__ It,
                                                     const FieldGeo& g, int accumulate,
-                                                    float* __restrict__ nd,
+                                                    float* __restrict__ nd, const Lay& lay,
                                                     double* __restrict__ partials,
                                                     const Block& blk)
 {
@@ -351,13 +377,13 @@ __device__ __forceinline__ void gradient_r_box_body(const uint8_t* __restrict__ 
             gr.z = 0.0f + gz * sc;
         }
         if (accumulate) {
-            float3 o = ld3(nd, v.p);
+            float3 o = ld_lay(nd, v.p, lay);
             o.x = o.x + gr.x;
             o.y = o.y + gr.y;
             o.z = o.z + gr.z;
-            st3(nd, v.p, o);
+            st_lay(nd, v.p, lay, o);
         } else {
-            st3(nd, v.p, gr);
+            st_lay(nd, v.p, lay, gr);
         }
         cost_sum += double(cost);
     }
@@ -389,10 +415,10 @@ inline bool grad_large(const FieldGeo& g) { return g.n >= kGLargeVoxels; }
 template <bool LARGE>
 __global__ __launch_bounds__(GradTile<LARGE>::kThreads) void gradient_r_box_kernel(
     const uint8_t* __restrict__ Js, const uint8_t* __restrict__ It, FieldGeo g, int accumulate,
-    float* __restrict__ nd, double* __restrict__ partials)
+    float* __restrict__ nd, Lay lay, double* __restrict__ partials)
 {
     using Tile = GradTile<LARGE>;
-    gradient_r_box_body<Tile::kSide, Tile::kSide, Tile::kThreads>(Js, It, g, accumulate, nd, partials,
+    gradient_r_box_body<Tile::kSide, Tile::kSide, Tile::kThreads>(Js, It, g, accumulate, nd, lay, partials,
                                                                   logical_block());
 }
 
@@ -464,9 +490,10 @@ __global__ __launch_bounds__(1024) void max_reduce_kernel(const float* __restric
 // ---------------------------------------------------------------------------
 constexpr float kInvD2 = -0.5f / 3.0f;
 
-// Volumes of at most this many voxels take four sweeps a launch
-// (poisson4_kernel), larger ones two (poisson2_kernel).
-constexpr size_t kPoisson4Voxels = size_t(1) << 20;
+// Volumes of at most this many voxels take poisson4_kernel (21 us for twelve
+// sweeps of 40x48x40), larger ones poisson_march_kernel (39 against 68 us at
+// 80x96x80).
+constexpr size_t kPoisson4Voxels = size_t(1) << 18;
 
 template <bool FIRST, bool MAXLEN>
 __global__ __launch_bounds__(256) void poisson_kernel(const float* __restrict__ nd,
@@ -821,8 +848,8 @@ __global__ __launch_bounds__(kQX * kQY) void poisson2_kernel(const float* __rest
 // reference's dropped neighbour.
 // What bounds it is latency -- one round of loads, four barriers -- where
 // poisson2_kernel chains a barrier pair and a load per plane.  Twelve sweeps:
-// 44 -> 17 us at 32x32x32 and below, 45 -> 21 at 40x48x40, 75 -> 68 at
-// 80x96x80, where the halo's work (eight times the core's) takes over.
+// 44 -> 17 us at 32x32x32 and below, 45 -> 21 at 40x48x40; at 80x96x80 the
+// halo's work (eight times the core's) takes over: 68, poisson_march_kernel 39.
 // ---------------------------------------------------------------------------
 constexpr int kCT = 8, kCH = 4, kCL = kCT + 2 * kCH;  // tile, halo (= sweeps), grown tile
 constexpr int kCThreads = kCL * kCL;
@@ -838,7 +865,8 @@ uint32_t poisson4_blocks(const FieldGeo& g)
 
 template <bool FIRST>
 __device__ __forceinline__ void poisson4_body(const float* __restrict__ nd, const float* __restrict__ a,
-                                              const FieldGeo& g, float* __restrict__ b, uint32_t blk)
+                                              const FieldGeo& g, const Lay& lay, float* __restrict__ b,
+                                              uint32_t blk)
 {
     __shared__ float plane[2][kCL][kCL + 2][kCL];  // rows -1 .. 16 of every plane
     const int tid = int(threadIdx.x), lx = tid & (kCL - 1), ly = tid / kCL;
@@ -848,11 +876,12 @@ __device__ __forceinline__ void poisson4_body(const float* __restrict__ nd, cons
     const int w = g.w, wh = int(g.wh), n = int(g.n);
     const int q0 = (z0 - kCH) * wh + (y0 - kCH) * w + (x0 - kCH);  // the grown tile's first voxel
     const int q = q0 + ly * w + lx;
-    const __amdgpu_buffer_rsrc_t rn = make_rsrc(nd, g.n * 12u);
-    const __amdgpu_buffer_rsrc_t ra = make_rsrc(FIRST ? nd : a, g.n * 12u);
+    const uint32_t bytes = ((g.n - 1u) * lay.ps + 1u) * 4u;
+    const __amdgpu_buffer_rsrc_t rn = make_rsrc(nd + size_t(comp) * lay.cs, bytes);
+    const __amdgpu_buffer_rsrc_t ra = make_rsrc((FIRST ? nd : a) + size_t(comp) * lay.cs, bytes);
+    const int pitch = int(lay.ps) * 4;
     auto load = [&](__amdgpu_buffer_rsrc_t rs, int k) {
-        return __uint_as_float(
-            __builtin_amdgcn_raw_buffer_load_b32(rs, (q + k * wh) * 12 + int(comp) * 4, 0, 0));
+        return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rs, (q + k * wh) * pitch, 0, 0));
     };
     float r[kCL], v[kCL];
 #pragma unroll
@@ -899,26 +928,206 @@ __device__ __forceinline__ void poisson4_body(const float* __restrict__ nd, cons
     if (x0 + lx - kCH >= w || y0 + ly - kCH >= g.h) return;
 #pragma unroll
     for (int k = kCH; k < kCH + kCT; ++k)
-        if (z0 + k - kCH < g.d) b[3 * size_t(q + k * wh) + comp] = v[k];
+        if (z0 + k - kCH < g.d) b[size_t(q + k * wh) * lay.ps + size_t(comp) * lay.cs] = v[k];
 }
 
 template <bool FIRST>
 __global__ __launch_bounds__(kCThreads) void poisson4_kernel(const float* __restrict__ nd,
                                                              const float* __restrict__ a, FieldGeo g,
-                                                             float* __restrict__ b)
+                                                             Lay lay, float* __restrict__ b)
 {
-    poisson4_body<FIRST>(nd, a, g, b, xcd_remap(blockIdx.x, gridDim.x));
+    poisson4_body<FIRST>(nd, a, g, lay, b, xcd_remap(blockIdx.x, gridDim.x));
+}
+
+// ---------------------------------------------------------------------------
+// K Jacobi sweeps per launch for large volumes, marching z.  As in
+// poisson4_kernel a workgroup takes one component, in flat-index offsets.
+// Its waves stack in y: lane l of wave v holds the kMR rows v * kMR .. of
+// column l, 64 x (kMWaves * kMR) columns in all, K of them halo on each side.
+// At step m plane m of the input arrives and stage t = 1 .. K computes plane
+// m - t from stage t - 1's planes m - t - 1, m - t, m - t + 1.  All planes
+// live in registers: p-+wh are the thread's own, p-+1 the neighbouring
+// lanes' (DPP wave shift), p-+w the thread's other rows; only a wave's first
+// and last row go through LDS, written in one step and read in the next, so
+// a step has one barrier for its K sweeps.  Rings of planes are indexed by
+// the unrolled step, so no value is moved.
+// FP32 issue bounds it (about 160 vector instructions a step for 16 updates a
+// thread).  Twelve sweeps, against six poisson2_kernel launches: 350 -> 204 us
+// at 182x218x182, 245 -> 120 at 160x192x160, 75 -> 39 at 80x96x80.
+// ---------------------------------------------------------------------------
+constexpr int kMWaves = 8, kMR = 4, kMThreads = 64 * kMWaves, kMRows = kMWaves * kMR;
+constexpr int kMK = 4;                   // sweeps per launch
+constexpr uint32_t kMarchBlocks = 512;   // workgroups resident at a time: two a CU
+constexpr int kMUnroll = 6;  // ring of six planes of input and new_d, three of each later stage
+
+struct March {
+    uint32_t gx, gy, gz;  // tiles
+    int zc;               // planes per workgroup
+    uint32_t blocks;
+};
+
+template <int K>
+March march_of(const FieldGeo& g)
+{
+    March m;
+    m.gx = uint32_t((g.w + 63 - 2 * K) / (64 - 2 * K));
+    m.gy = uint32_t((g.h + kMRows - 1 - 2 * K) / (kMRows - 2 * K));
+    // two workgroups run on a CU at a time: the number of z runs with the
+    // fewest steps over all rounds of them
+    const uint32_t cols = 3u * m.gx * m.gy;
+    long best = 0;
+    for (int zc = g.d; zc >= 2; --zc) {
+        const uint32_t gz = uint32_t((g.d + zc - 1) / zc);
+        const long rounds = long((uint64_t(cols) * gz + kMarchBlocks - 1) / kMarchBlocks);
+        const long steps = rounds * (zc + 2 * K + 2);
+        if (best && steps >= best) continue;
+        best = steps;
+        m.gz = gz;
+        m.zc = zc;
+        if (rounds > 64) break;
+    }
+    if (!best) {
+        m.gz = 1;
+        m.zc = g.d;
+    }
+    m.blocks = cols * m.gz;
+    return m;
+}
+
+template <int K, bool FIRST>
+__global__ __launch_bounds__(kMThreads, 4) void poisson_march_kernel(const float* __restrict__ nd,
+                                                                  const float* __restrict__ a,
+                                                                  FieldGeo g, March mg, Lay lay,
+                                                                  float* __restrict__ b)
+{
+    __shared__ float edge[2][K][kMWaves][2][64];
+    const int lane = int(threadIdx.x) & 63;
+    const int wv = __builtin_amdgcn_readfirstlane(int(threadIdx.x) >> 6);
+    const uint32_t L = xcd_remap(blockIdx.x, mg.blocks);
+    const uint32_t comp = L % 3u, tile = L / 3u;
+    const int x0 = int(tile % mg.gx) * (64 - 2 * K) - K;
+    const int y0 = int((tile / mg.gx) % mg.gy) * (kMRows - 2 * K) - K;
+    const int z0 = int(tile / (mg.gx * mg.gy)) * mg.zc, z1 = min(z0 + mg.zc, g.d);
+    const int w = g.w, wh = int(g.wh), n = int(g.n);
+    const uint32_t bytes = ((g.n - 1u) * lay.ps + 1u) * 4u;
+    const __amdgpu_buffer_rsrc_t rn = make_rsrc(nd + size_t(comp) * lay.cs, bytes);
+    const __amdgpu_buffer_rsrc_t ra = make_rsrc((FIRST ? nd : a) + size_t(comp) * lay.cs, bytes);
+    const __amdgpu_buffer_rsrc_t rb = make_rsrc(b + size_t(comp) * lay.cs, bytes);
+    const int pitch = int(lay.ps) * 4, row = w * pitch, slab = wh * pitch;
+    const int q0 = (y0 + wv * kMR) * w + x0 + lane;  // row 0 of this thread in plane 0
+    auto load = [&](__amdgpu_buffer_rsrc_t rs, int at, float (&dst)[kMR]) {
+#pragma unroll
+        for (int j = 0; j < kMR; ++j)
+            dst[j] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rs, at + j * row, 0, 0));
+    };
+    const int lo = y0 * w + x0 + (z0 - K) * wh;
+    const int hi = (y0 + kMRows - 1) * w + x0 + 63 + (z1 - 1 + K) * wh;
+    const bool ends = lo < 0 || hi >= n;
+    float in[kMUnroll][kMR], r[kMUnroll][kMR], st[K][3][kMR];
+#pragma unroll
+    for (int t = 1; t < K; ++t)
+#pragma unroll
+        for (int k = 0; k < 3; ++k)
+#pragma unroll
+            for (int j = 0; j < kMR; ++j) st[t][k][j] = 0.0f;
+#pragma unroll
+    for (int k = 0; k < kMUnroll; ++k)
+#pragma unroll
+        for (int j = 0; j < kMR; ++j) in[k][j] = r[k][j] = 0.0f;
+    const int first = z0 - K, last = z1 - 1 + K;
+    // plane m of the input is in[(m - first) % 6], of new_d r[(m - first) % 6]
+    int qm = q0 + first * wh;             // this thread's row 0 in plane m
+    int at = (q0 + (first + 2) * wh) * pitch;  // and its byte offset in plane m + 2
+    load(ra, at - 2 * slab, in[0]);
+    if (!FIRST) load(rn, at - 2 * slab, r[0]);
+    load(ra, at - slab, in[1]);
+    const bool xy_out = lane >= K && lane < 64 - K && x0 + lane < w;
+    for (int base = first; base <= last; base += kMUnroll) {
+#pragma unroll
+        for (int u = 0; u < kMUnroll; ++u) {
+            const int m = base + u;
+            if (m > last) break;
+            // two planes ahead
+            load(ra, at, in[(u + 2) % kMUnroll]);
+            if (!FIRST) load(rn, at - slab, r[(u + 1) % kMUnroll]);
+            if (FIRST) {
+#pragma unroll
+                for (int j = 0; j < kMR; ++j) {
+                    r[u][j] = in[u][j];
+                    in[u][j] = in[u][j] * kInvD2;
+                }
+            }
+            __syncthreads();
+            const int par = u & 1;
+#pragma unroll
+            for (int t = 1; t <= K; ++t) {
+                // stage t, plane m - t; needed from plane z0 - (K - t) on
+                if (m - t < z0 - (K - t)) continue;
+                const int c1 = (u - t + 12) % kMUnroll;  // ring slot of plane m - t
+                auto src = [&](int d) -> float(&)[kMR] {  // stage t - 1, plane m - t + d
+                    if (t == 1) return in[(u - 1 + d + 12) % kMUnroll];
+                    return st[t - 1][(u - t + d + 12) % 3];
+                };
+                float(&c)[kMR] = src(0);
+                float(&zm)[kMR] = src(-1);
+                float(&zp)[kMR] = src(1);
+                const float up = edge[par ^ 1][t - 1][wv > 0 ? wv - 1 : 0][1][lane];
+                const float dn = edge[par ^ 1][t - 1][wv < kMWaves - 1 ? wv + 1 : wv][0][lane];
+                float o[kMR];
+#pragma unroll
+                for (int j = 0; j < kMR; ++j) {
+                    float x = r[c1][j] - wave_prev(c[j]);
+                    x = x - wave_next(c[j]);
+                    x = x - (j > 0 ? c[j - 1] : up);
+                    x = x - (j < kMR - 1 ? c[j + 1] : dn);
+                    x = x - zm[j];
+                    x = x - zp[j];
+                    o[j] = x * kInvD2;
+                }
+                if (t < K) {
+                    if (ends) {
+                        const int q = qm - t * wh;
+#pragma unroll
+                        for (int j = 0; j < kMR; ++j)
+                            o[j] = uint32_t(q + j * w) < uint32_t(n) ? o[j] : 0.0f;
+                    }
+#pragma unroll
+                    for (int j = 0; j < kMR; ++j) st[t][(u - t + 12) % 3][j] = o[j];
+                } else if (m - K >= z0) {
+                    const int to = at - (K + 2) * slab;
+#pragma unroll
+                    for (int j = 0; j < kMR; ++j) {
+                        const int rj = wv * kMR + j;
+                        if (rj >= K && rj < kMRows - K && y0 + rj < g.h && xy_out)
+                            __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(o[j]), rb, to + j * row, 0, 0);
+                    }
+                }
+            }
+            // this step's new planes: first and last row of the wave
+#pragma unroll
+            for (int t = 0; t < K; ++t) {
+                float(&v)[kMR] = t == 0 ? in[u] : st[t][(u - t + 12) % 3];
+                edge[par][t][wv][0][lane] = v[0];
+                edge[par][t][wv][1][lane] = v[kMR - 1];
+            }
+            at += slab;
+            qm += wh;
+            // (keeps the two running offsets in two registers: the compiler
+            // otherwise carries one per unrolled use and spills)
+            asm volatile("" : "+v"(at), "+v"(qm));
+        }
+    }
 }
 
 // cdm_max_displacement_length of a whole field: per-block maxima.
-constexpr uint32_t kMaxLenBlocks = 128;
+constexpr uint32_t kMaxLenBlocks = 1024;
 
 __global__ __launch_bounds__(256) void max_length_kernel(const float* __restrict__ d, uint32_t n,
-                                                         float* __restrict__ maxparts)
+                                                         Lay lay, float* __restrict__ maxparts)
 {
     float m = 0.0f;
     for (uint32_t p = blockIdx.x * 256u + threadIdx.x; p < n; p += gridDim.x * 256u) {
-        const float3 r = ld3(d, p);
+        const float3 r = ld_lay(d, p, lay);
         float s2 = r.x * r.x + r.y * r.y;
         s2 = s2 + r.z * r.z;
         m = fmaxf(m, float(sqrt(double(s2))));
@@ -931,15 +1140,16 @@ __global__ __launch_bounds__(256) void max_length_kernel(const float* __restrict
 }
 
 // ---------------------------------------------------------------------------
-// new_d *= k, then accumulate_displacement(cur, new_d) in place:
-// new(x) = m(x + new(x)) - x with m(y) = cur(y) + y by trilinear
+// new_d *= k, then accumulate_displacement(cur, new_d) into out (which may be
+// new_d itself where that is packed): new(x) = m(x + new(x)) - x with m(y) = cur(y) + y by trilinear
 // interpolation; cur(x) where new(x) == 0 or the sample is outside.
 // ---------------------------------------------------------------------------
 // The accumulated displacement at voxel p = (x, y, z).
 __device__ inline float3 accumulated(const float* __restrict__ cur, const float* __restrict__ nd,
-                                     float k, const FieldGeo& g, uint32_t p, int x, int y, int z)
+                                     const Lay& lay, float k, const FieldGeo& g, uint32_t p, int x, int y,
+                                     int z)
 {
-    float3 d = ld3(nd, p);
+    float3 d = ld_lay(nd, p, lay);
     d.x = d.x * k;
     d.y = d.y * k;
     d.z = d.z * k;
@@ -970,13 +1180,12 @@ __device__ inline float3 accumulated(const float* __restrict__ cur, const float*
     return ld3(cur, p);
 }
 
-__global__ __launch_bounds__(256) void accumulate_kernel(const float* __restrict__ cur,
-                                                         float* __restrict__ nd, float k,
-                                                         FieldGeo g)
+__global__ __launch_bounds__(256) void accumulate_kernel(const float* __restrict__ cur, const float* nd,
+                                                         Lay lay, float k, FieldGeo g, float* out)
 {
     const Vox v = this_voxel(g);
     if (!v.ok) return;
-    st3(nd, v.p, accumulated(cur, nd, k, g, v.p, v.x, v.y, v.z));
+    st3(out, v.p, accumulated(cur, nd, lay, k, g, v.p, v.x, v.y, v.z));
 }
 
 // One packed float3 voxel through a raw buffer resource: a load past the
@@ -993,10 +1202,11 @@ __device__ inline float3 ld3_rsrc(__amdgpu_buffer_rsrc_t r, uint32_t p)
 // cur(p); corners past the field's end read 0 and are unused) and the
 // result is selected.  Where the sample is taken every operation is
 // accumulated()'s, in its order.  Needs 12 n < 2^32.
-__device__ inline float3 accumulated_bf(__amdgpu_buffer_rsrc_t rcur, __amdgpu_buffer_rsrc_t rnd,
-                                        float k, const FieldGeo& g, uint32_t p, int x, int y, int z)
+__device__ inline float3 accumulated_bf(__amdgpu_buffer_rsrc_t rcur, const float* __restrict__ nd,
+                                        const Lay& lay, float k, const FieldGeo& g, uint32_t p, int x, int y,
+                                        int z)
 {
-    float3 d = ld3_rsrc(rnd, p);
+    float3 d = ld_lay(nd, p, lay);
     d.x = d.x * k;
     d.y = d.y * k;
     d.z = d.z * k;
@@ -1054,8 +1264,9 @@ __device__ inline float3 accumulated_bf(__amdgpu_buffer_rsrc_t rcur, __amdgpu_bu
 // before the step, as the reference's loop does), keep aliasing neither.
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ void accumulate_smooth_body(
-    const float* __restrict__ cur, const float* __restrict__ nd, float k, float w_6, float w_1,
-    const FieldGeo& g, int zq, float* __restrict__ out, float* __restrict__ keep, const Block& blk)
+    const float* __restrict__ cur, const float* __restrict__ nd, const Lay& lay, float k, float w_6,
+    float w_1, const FieldGeo& g, int zq, float* __restrict__ out, float* __restrict__ keep,
+    const Block& blk)
 {
     __shared__ float3 A[4][kS1Y][kS1X];
     const int tx = int(threadIdx.x), ty = int(threadIdx.y), tid = ty * kQX + tx;
@@ -1064,7 +1275,6 @@ __device__ __forceinline__ void accumulate_smooth_body(
     const long long n = g.n, w = g.w, wh = g.wh;
     const long long base = (long long)y0 * w + x0;
     const __amdgpu_buffer_rsrc_t rcur = make_rsrc(cur, g.n * 12u);
-    const __amdgpu_buffer_rsrc_t rnd = make_rsrc(nd, g.n * 12u);
     int ri = 0, rj = 0;
     const bool has_ring = tid < kRing;
     if (has_ring) ring_offset(tid, ri, rj);
@@ -1076,7 +1286,7 @@ __device__ __forceinline__ void accumulate_smooth_body(
         const uint32_t p = ok ? uint32_t(q) : 0u;
         const uint32_t z = p / g.wh, r = p - z * g.wh;
         const uint32_t y = r / uint32_t(g.w), x = r - y * uint32_t(g.w);
-        const float3 v = accumulated_bf(rcur, rnd, k, g, p, int(x), int(y), int(z));
+        const float3 v = accumulated_bf(rcur, nd, lay, k, g, p, int(x), int(y), int(z));
         return ok ? v : zero;
     };
     auto fill = [&](int m) {
@@ -1118,10 +1328,10 @@ __device__ __forceinline__ void accumulate_smooth_body(
 }
 
 __global__ __launch_bounds__(kQX * kQY) void accumulate_smooth_kernel(
-    const float* __restrict__ cur, const float* __restrict__ nd, float k, float w_6, float w_1,
+    const float* __restrict__ cur, const float* __restrict__ nd, Lay lay, float k, float w_6, float w_1,
     FieldGeo g, int zq, float* __restrict__ out)
 {
-    accumulate_smooth_body(cur, nd, k, w_6, w_1, g, zq, out, nullptr, logical_block());
+    accumulate_smooth_body(cur, nd, lay, k, w_6, w_1, g, zq, out, nullptr, logical_block());
 }
 
 // ---------------------------------------------------------------------------
@@ -1196,7 +1406,7 @@ __global__ __launch_bounds__(GradTile<LARGE>::kThreads) void gradient_seg_kernel
     int s;
     const Block b = seg_block(st, s);
     gradient_r_box_body<Tile::kSide, Tile::kSide, Tile::kThreads>(st.Js[s], st.It[s], st.g[s], 0, st.nd[s],
-                                                                  st.partials[s], b);
+                                                                  Lay{3u, 1u}, st.partials[s], b);
 }
 
 // one workgroup per field
@@ -1226,7 +1436,7 @@ __global__ __launch_bounds__(kQX * kQY) void accumulate_smooth_seg_kernel(const 
 {
     int s;
     const Block b = seg_block(st, s);
-    accumulate_smooth_body(st.cur[s], st.nd[s], st.k[s], st.w_6[s], st.w_1[s], st.g[s], st.zq[s],
+    accumulate_smooth_body(st.cur[s], st.nd[s], Lay{3u, 1u}, st.k[s], st.w_6[s], st.w_1[s], st.g[s], st.zq[s],
                            st.dst[s], st.keep[s], b);
 }
 
@@ -1323,23 +1533,23 @@ void launch_compose(tiplhip_ctx* ctx, const uint8_t* Is, const float* d, const F
 }
 
 void launch_gradient(tiplhip_ctx* ctx, const uint8_t* Js, const uint8_t* It, const FieldGeo& g,
-                     char type, int accumulate, float* nd, double* partials, float* cost_out,
+                     char type, int accumulate, float* nd, Lay lay, double* partials, float* cost_out,
                      float* host_cost = nullptr)
 {
     uint32_t parts;
     if (type == 'd') {
         hipLaunchKernelGGL(gradient_kernel<'d'>, tile_grid(g), dim3(kTX, kTY), 0, ctx->stream, Js,
-                           It, g, accumulate, nd, partials);
+                           It, g, accumulate, nd, lay, partials);
         const dim3 tg = tile_grid(g);
         parts = tg.x * tg.y * tg.z;
     } else {
         const dim3 bg = box_grid(g);
         if (grad_large(g))
             hipLaunchKernelGGL(gradient_r_box_kernel<true>, bg, dim3(GradTile<true>::kThreads), 0,
-                               ctx->stream, Js, It, g, accumulate, nd, partials);
+                               ctx->stream, Js, It, g, accumulate, nd, lay, partials);
         else
             hipLaunchKernelGGL(gradient_r_box_kernel<false>, bg, dim3(GradTile<false>::kThreads), 0,
-                               ctx->stream, Js, It, g, accumulate, nd, partials);
+                               ctx->stream, Js, It, g, accumulate, nd, lay, partials);
         parts = bg.x * bg.y * bg.z;
     }
     TIPLHIP_CHECK(hipGetLastError());
@@ -1348,13 +1558,13 @@ void launch_gradient(tiplhip_ctx* ctx, const uint8_t* Js, const uint8_t* It, con
     TIPLHIP_CHECK(hipGetLastError());
 }
 
-// `sweeps` Jacobi sweeps: four per launch while the volume is small
-// (poisson4_kernel), two per launch (poisson2_kernel) otherwise, and a single
-// z-marching sweep for an odd remainder; returns the buffer holding the
-// result.  With maxlen, per-block maxima of the displacement length (from the
+// `sweeps` Jacobi sweeps, four per launch (poisson4_kernel for small volumes,
+// poisson_march_kernel for large ones); of a packed field also the remainder,
+// and all of a volume whose byte offsets pass 2^31, by two (poisson2_kernel)
+// and one (the z-marching sweep).  Returns the buffer holding the result.  With maxlen, per-block maxima of the displacement length (from the
 // last launch, or a pass of their own after a four-sweep one) are reduced by
 // max_reduce_kernel.
-float* launch_poisson(tiplhip_ctx* ctx, const float* nd, float* a, float* b, const FieldGeo& g,
+float* launch_poisson(tiplhip_ctx* ctx, const float* nd, float* a, float* b, const FieldGeo& g, Lay lay,
                       int sweeps, unsigned int* maxlen, float* maxparts)
 {
     float* src = a;
@@ -1366,20 +1576,43 @@ float* launch_poisson(tiplhip_ctx* ctx, const float* nd, float* a, float* b, con
         if (sweeps - done >= kCH && poisson4_fits(g)) {
             const dim3 grid(poisson4_blocks(g)), block(kCThreads);
             if (first)
-                hipLaunchKernelGGL(poisson4_kernel<true>, grid, block, 0, ctx->stream, nd, src, g, dst);
+                hipLaunchKernelGGL(poisson4_kernel<true>, grid, block, 0, ctx->stream, nd, src, g, lay,
+                                   dst);
             else
-                hipLaunchKernelGGL(poisson4_kernel<false>, grid, block, 0, ctx->stream, nd, src, g, dst);
+                hipLaunchKernelGGL(poisson4_kernel<false>, grid, block, 0, ctx->stream, nd, src, g, lay,
+                                   dst);
             TIPLHIP_CHECK(hipGetLastError());
             done += kCH;
             if (done == sweeps && maxlen) {
                 last_blocks = std::min(kMaxLenBlocks, block_count(g));
                 hipLaunchKernelGGL(max_length_kernel, dim3(last_blocks), dim3(256), 0, ctx->stream, dst,
-                                   g.n, maxparts);
+                                   g.n, lay, maxparts);
                 TIPLHIP_CHECK(hipGetLastError());
             }
             std::swap(src, dst);
             continue;
         }
+        if (sweeps - done >= kMK && planar_fits(g)) {
+            const March mg = march_of<kMK>(g);
+            const dim3 grid(mg.blocks), block(kMThreads);
+            if (first)
+                hipLaunchKernelGGL((poisson_march_kernel<kMK, true>), grid, block, 0, ctx->stream, nd, src,
+                                   g, mg, lay, dst);
+            else
+                hipLaunchKernelGGL((poisson_march_kernel<kMK, false>), grid, block, 0, ctx->stream, nd, src,
+                                   g, mg, lay, dst);
+            TIPLHIP_CHECK(hipGetLastError());
+            done += kMK;
+            if (done == sweeps && maxlen) {
+                last_blocks = std::min(kMaxLenBlocks, block_count(g));
+                hipLaunchKernelGGL(max_length_kernel, dim3(last_blocks), dim3(256), 0, ctx->stream, dst,
+                                   g.n, lay, maxparts);
+                TIPLHIP_CHECK(hipGetLastError());
+            }
+            std::swap(src, dst);
+            continue;
+        }
+        TIPLHIP_REQUIRE(lay.ps == 3u, "one- and two-sweep launches take packed fields");
         const bool pair = sweeps - done >= 2;
         const bool last = done + (pair ? 2 : 1) == sweeps && maxlen;
         if (pair) {
@@ -1427,21 +1660,23 @@ float* launch_poisson(tiplhip_ctx* ctx, const float* nd, float* a, float* b, con
     return src;
 }
 
-void launch_accumulate(tiplhip_ctx* ctx, const float* cur, float* nd, float k, const FieldGeo& g)
+void launch_accumulate(tiplhip_ctx* ctx, const float* cur, const float* nd, Lay lay, float k,
+                       const FieldGeo& g, float* out)
 {
-    hipLaunchKernelGGL(accumulate_kernel, tile_grid(g), dim3(kTX, kTY), 0, ctx->stream, cur, nd, k, g);
+    hipLaunchKernelGGL(accumulate_kernel, tile_grid(g), dim3(kTX, kTY), 0, ctx->stream, cur, nd, lay, k, g,
+                       out);
     TIPLHIP_CHECK(hipGetLastError());
 }
 
 // accumulate then cdm_smooth with `smoothing` (non-zero) in one pass into out.
-void launch_accumulate_smooth(tiplhip_ctx* ctx, const float* cur, const float* nd, float k,
+void launch_accumulate_smooth(tiplhip_ctx* ctx, const float* cur, const float* nd, Lay lay, float k,
                               float smoothing, const FieldGeo& g, float* out)
 {
     const float w_6 = smoothing / float(2.0f * 3.0f);
     const float w_1 = 1.0f - smoothing;
     const int zq = poisson2_zq(g);
     hipLaunchKernelGGL(accumulate_smooth_kernel, poisson2_grid(g, zq), dim3(kQX, kQY), 0, ctx->stream,
-                       cur, nd, k, w_6, w_1, g, zq, out);
+                       cur, nd, lay, k, w_6, w_1, g, zq, out);
     TIPLHIP_CHECK(hipGetLastError());
 }
 
@@ -2013,6 +2248,7 @@ bool cdm_level(CdmRun& run, const std::vector<const uint8_t*>& It,
     const uint32_t nblocks = block_count(g);
     DevMem partials(ctx, sizeof(double) * nblocks), maxparts(ctx, sizeof(float) * nblocks);
     DevMem scal(ctx, sizeof(float) * 16 + sizeof(unsigned int));
+    const Lay lay = grad_layout(g);
     float* d_cost = scal.as<float>();
     unsigned int* d_maxlen = reinterpret_cast<unsigned int*>(scal.as<float>() + 16);
     // the cost reductions store into ctx->h_cdm: if a step throws while one
@@ -2048,10 +2284,10 @@ bool cdm_level(CdmRun& run, const std::vector<const uint8_t*>& It,
             launch_compose(ctx, Is[size_t(i)], cur, g, Js.as<uint8_t>());
             const char type = run.param.gradient_type[std::min(i, 7)] == 'd' ? 'd' : 'r';
             launch_gradient(ctx, Js.as<uint8_t>(), It[size_t(i)], g, type, i > 0 ? 1 : 0,
-                            nd.as<float>(), partials.as<double>(), d_cost + i, h_cost + i);
+                            nd.as<float>(), lay, partials.as<double>(), d_cost + i, h_cost + i);
         }
         const bool need_theta = theta == 0.0f;
-        float* solved = launch_poisson(ctx, nd.as<float>(), pa, pb, g, 12,
+        float* solved = launch_poisson(ctx, nd.as<float>(), pa, pb, g, lay, 12,
                                        need_theta ? d_maxlen : nullptr, maxparts.as<float>());
         wait_for_slots(static_cast<const volatile uint32_t*>(slots), size_t(run.nmod), kCostPending,
                        std::chrono::microseconds(kCostSpinUs),
@@ -2084,7 +2320,7 @@ bool cdm_level(CdmRun& run, const std::vector<const uint8_t*>& It,
         // accumulated field is then unused), as in the reference
         if (cur_smoothing != 0.0f) {
             float* spare = solved == pa ? pb : pa;
-            launch_accumulate_smooth(ctx, cur, solved, k, cur_smoothing, g, spare);
+            launch_accumulate_smooth(ctx, cur, solved, lay, k, cur_smoothing, g, spare);
             pa = cur;
             pb = solved;
             cur = spare;
@@ -2132,6 +2368,7 @@ void cdm_fixed(CdmRun& run, const std::vector<const uint8_t*>& It,
     const uint32_t nblocks = block_count(g);
     DevMem partials(ctx, sizeof(double) * nblocks), maxparts(ctx, sizeof(float) * nblocks);
     DevMem scal(ctx, sizeof(float) * 16 + sizeof(unsigned int));
+    const Lay lay = grad_layout(g);
     float* d_cost = scal.as<float>();
     unsigned int* d_maxlen = reinterpret_cast<unsigned int*>(scal.as<float>() + 16);
     float theta = 0.0f;
@@ -2145,10 +2382,10 @@ void cdm_fixed(CdmRun& run, const std::vector<const uint8_t*>& It,
             launch_compose(ctx, Is[size_t(i)], field, g, Js.as<uint8_t>());
             const char type = run.param.gradient_type[std::min(i, 7)] == 'd' ? 'd' : 'r';
             launch_gradient(ctx, Js.as<uint8_t>(), It[size_t(i)], g, type, i > 0 ? 1 : 0,
-                            nd.as<float>(), partials.as<double>(), d_cost + i);
+                            nd.as<float>(), lay, partials.as<double>(), d_cost + i);
         }
         const bool need_theta = theta == 0.0f;
-        float* solved = launch_poisson(ctx, nd.as<float>(), pa.as<float>(), pb.as<float>(), g, 12,
+        float* solved = launch_poisson(ctx, nd.as<float>(), pa.as<float>(), pb.as<float>(), g, lay, 12,
                                        need_theta ? d_maxlen : nullptr, maxparts.as<float>());
         if (need_theta) {
             unsigned int bits = 0;
@@ -2156,13 +2393,13 @@ void cdm_fixed(CdmRun& run, const std::vector<const uint8_t*>& It,
             std::memcpy(&theta, &bits, sizeof(theta));
         }
         if (theta == 0.0f) break;
-        launch_accumulate(ctx, field, solved, run.param.speed / theta, g);
+        float* spare = solved == pa.as<float>() ? pb.as<float>() : pa.as<float>();
+        launch_accumulate(ctx, field, solved, lay, run.param.speed / theta, g, spare);
         if (run.param.field_bandwidth > 0) {
-            float* spare = solved == pa.as<float>() ? pb.as<float>() : pa.as<float>();
-            launch_gaussian_to(ctx, solved, field, spare, dim, 3, unsigned(run.param.field_bandwidth));
+            launch_gaussian_to(ctx, spare, field, solved, dim, 3, unsigned(run.param.field_bandwidth));
         } else if (run.param.smoothing != 0.0f) {
             // cdm_smooth with weight 0 leaves the field untouched, as in the reference
-            launch_smooth(ctx, solved, field, run.param.smoothing, g);
+            launch_smooth(ctx, spare, field, run.param.smoothing, g);
         }
     }
     TIPLHIP_CHECK(hipStreamSynchronize(ctx->stream));
@@ -2322,7 +2559,7 @@ int tiplhip_cdm_gradient(tiplhip_ctx* ctx, const uint8_t* Js, const uint8_t* It,
         TIPLHIP_CHECK(hipMemcpyAsync(dJ.p, Js, g.n, hipMemcpyHostToDevice, ctx->stream));
         TIPLHIP_CHECK(hipMemcpyAsync(dI.p, It, g.n, hipMemcpyHostToDevice, ctx->stream));
         launch_gradient(ctx, dJ.as<uint8_t>(), dI.as<uint8_t>(), g, type, 0, dN.as<float>(),
-                        part.as<double>(), dc.as<float>());
+                        packed_layout(), part.as<double>(), dc.as<float>());
         TIPLHIP_CHECK(hipMemcpyAsync(new_d, dN.p, sizeof(float) * 3 * g.n, hipMemcpyDeviceToHost, ctx->stream));
         float c = 0.0f;
         TIPLHIP_CHECK(hipMemcpyAsync(&c, dc.p, sizeof(float), hipMemcpyDeviceToHost, ctx->stream));
@@ -2344,7 +2581,7 @@ int tiplhip_cdm_poisson(tiplhip_ctx* ctx, float* new_d, const int dim[3], int sw
         const size_t fb = sizeof(float) * 3 * g.n;
         DevMem dN(ctx, fb), a(ctx, fb), b(ctx, fb), ml(ctx, sizeof(unsigned int)), mp(ctx, sizeof(float) * block_count(g));
         TIPLHIP_CHECK(hipMemcpyAsync(dN.p, new_d, fb, hipMemcpyHostToDevice, ctx->stream));
-        float* out = launch_poisson(ctx, dN.as<float>(), a.as<float>(), b.as<float>(), g, sweeps,
+        float* out = launch_poisson(ctx, dN.as<float>(), a.as<float>(), b.as<float>(), g, packed_layout(), sweeps,
                                     ml.as<unsigned int>(), mp.as<float>());
         TIPLHIP_CHECK(hipMemcpyAsync(new_d, out, fb, hipMemcpyDeviceToHost, ctx->stream));
         unsigned int bits = 0;
@@ -2367,7 +2604,7 @@ int tiplhip_accumulate_displacement(tiplhip_ctx* ctx, const float* cur, float* n
         DevMem dC(ctx, fb), dN(ctx, fb);
         TIPLHIP_CHECK(hipMemcpyAsync(dC.p, cur, fb, hipMemcpyHostToDevice, ctx->stream));
         TIPLHIP_CHECK(hipMemcpyAsync(dN.p, new_d, fb, hipMemcpyHostToDevice, ctx->stream));
-        launch_accumulate(ctx, dC.as<float>(), dN.as<float>(), scale, g);
+        launch_accumulate(ctx, dC.as<float>(), dN.as<float>(), packed_layout(), scale, g, dN.as<float>());
         TIPLHIP_CHECK(hipMemcpyAsync(new_d, dN.p, fb, hipMemcpyDeviceToHost, ctx->stream));
         TIPLHIP_CHECK(hipStreamSynchronize(ctx->stream));
     });
