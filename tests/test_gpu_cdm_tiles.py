@@ -76,12 +76,15 @@ def test_poisson_marched_tiles(ctx, oracle, shape):
         assert ml == oracle.max_length(want)
 
 
-@pytest.mark.parametrize("shape", [(21, 30, 27), (61, 67, 71)])
-def test_level_iterations_by_size(ctx, oracle, shape):
-    """The loop's planar gradient fields, on each side of the size where the
-    Poisson kernel changes: the oracle's step functions in the loop's order."""
+@pytest.mark.parametrize("speed", [0.3, 4.0])
+@pytest.mark.parametrize("shape", [(21, 30, 27), (61, 67, 71), (130, 2, 1100), (1, 33, 9), (9, 1, 33), (40, 9, 1)])
+def test_level_iterations_by_size(ctx, oracle, shape, speed):
+    """The loop's planar gradient fields and its fused field update, on each
+    side of the sizes where their kernels change, with steps inside a voxel
+    and across several: the oracle's step functions in the loop's order."""
     from test_gpu_cdm import _pair, oracle_level_iterations
     It, Is = _pair(shape, 31)
-    want = oracle_level_iterations(oracle, It, Is, 4)
-    got = ctx.cdm_level_iterations(ctx.volume(It), ctx.volume(Is), 4, want_field=True)
+    want = oracle_level_iterations(oracle, It, Is, 4, speed=speed)
+    p = ctx.cdm_param(speed=speed)
+    got = ctx.cdm_level_iterations(ctx.volume(It), ctx.volume(Is), 4, p, want_field=True)
     assert _bits_equal(got, want)

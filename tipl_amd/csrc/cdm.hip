@@ -50,7 +50,7 @@ namespace {
 struct Lay {
     uint32_t ps, cs;
 };
-inline Lay packed_layout() { return Lay{3u, 1u}; }
+__host__ __device__ inline Lay packed_layout() { return Lay{3u, 1u}; }
 inline bool planar_fits(const FieldGeo& g) { return size_t(g.n) * 12 < (size_t(1) << 31); }
 inline Lay grad_layout(const FieldGeo& g) { return planar_fits(g) ? Lay{1u, g.n} : packed_layout(); }
 
@@ -70,20 +70,22 @@ __device__ inline void st_lay(float* f, uint32_t p, const Lay& l, float3 v)
 // ---------------------------------------------------------------------------
 // compose_displacement: Js(x) = Is(x + d(x)); exact copy where d(x) == 0.
 // ---------------------------------------------------------------------------
+// Js at voxel p = (x, y, z) under the displacement dv.
+__device__ __forceinline__ uint8_t composed(const uint8_t* __restrict__ Is, const FieldGeo& g, int x, int y,
+                                            int z, uint32_t p, const float3& dv)
+{
+    if (dv.x == 0.0f && dv.y == 0.0f && dv.z == 0.0f) return Is[p];
+    const __amdgpu_buffer_rsrc_t r = make_rsrc(Is, g.n);
+    VolGeo vg{g.w, g.h, g.d, g.wh, g.wm1, g.hm1, g.dm1};
+    return uint8_t(sample_u8(r, vg, float(x) + dv.x, float(y) + dv.y, float(z) + dv.z));
+}
+
 __device__ __forceinline__ void compose_body(const uint8_t* __restrict__ Is,
                                              const float* __restrict__ d, const FieldGeo& g,
                                              uint8_t* __restrict__ Js, const Block& blk)
 {
     const Vox v = voxel_of(g, blk);
-    if (!v.ok) return;
-    const float3 dv = ld3(d, v.p);
-    if (dv.x == 0.0f && dv.y == 0.0f && dv.z == 0.0f) {
-        Js[v.p] = Is[v.p];
-        return;
-    }
-    const __amdgpu_buffer_rsrc_t r = make_rsrc(Is, g.n);
-    VolGeo vg{g.w, g.h, g.d, g.wh, g.wm1, g.hm1, g.dm1};
-    Js[v.p] = uint8_t(sample_u8(r, vg, float(v.x) + dv.x, float(v.y) + dv.y, float(v.z) + dv.z));
+    if (v.ok) Js[v.p] = composed(Is, g, v.x, v.y, v.z, v.p, ld3(d, v.p));
 }
 
 __global__ __launch_bounds__(256) void compose_kernel(const uint8_t* __restrict__ Is,
@@ -1196,142 +1198,265 @@ __device__ inline float3 ld3_rsrc(__amdgpu_buffer_rsrc_t r, uint32_t p)
     return make_float3(__uint_as_float(v[0]), __uint_as_float(v[1]), __uint_as_float(v[2]));
 }
 
-// accumulated() without branches, so that several evaluations per thread
-// keep their loads in flight together: the eight corners are always loaded
-// (at the voxel itself when the sample is not taken, so corner 0 is then
-// cur(p); corners past the field's end read 0 and are unused) and the
-// result is selected.  Where the sample is taken every operation is
-// accumulated()'s, in its order.  Needs 12 n < 2^32.
-__device__ inline float3 accumulated_bf(__amdgpu_buffer_rsrc_t rcur, const float* __restrict__ nd,
-                                        const Lay& lay, float k, const FieldGeo& g, uint32_t p, int x, int y,
-                                        int z)
-{
-    float3 d = ld_lay(nd, p, lay);
-    d.x = d.x * k;
-    d.y = d.y * k;
-    d.z = d.z * k;
-    const bool moved = d.x != 0.0f || d.y != 0.0f || d.z != 0.0f;
-    const float sx = d.x + float(x), sy = d.y + float(y), sz = d.z + float(z);
-    const bool in = (fminf(fminf(sx, sy), sz) >= 0.0f) & (sx < g.wm1) & (sy < g.hm1) & (sz < g.dm1);
-    const bool use = moved && in;
-    const uint32_t ix = use ? cvt_u32_sat(sx) : 0u, iy = use ? cvt_u32_sat(sy) : 0u,
-                   iz = use ? cvt_u32_sat(sz) : 0u;
-    const uint32_t i0 = use ? iz * g.wh + iy * uint32_t(g.w) + ix : p;
-    float3 m[8];
-#pragma unroll
-    for (int c = 0; c < 8; ++c) m[c] = ld3_rsrc(rcur, corner(g, i0, c));
-    const float p0 = sx - float(ix), p1 = sy - float(iy), p2 = sz - float(iz);
-    const float n0 = 1.0f - p0, n1 = 1.0f - p1, n2 = 1.0f - p2;
-    const float n0n1 = n0 * n1, p0n1 = p0 * n1, n0p1 = n0 * p1, p0p1 = p0 * p1;
-    const float w[8] = {n0n1 * n2, p0n1 * n2, n0p1 * n2, p0p1 * n2,
-                        n0n1 * p2, p0n1 * p2, n0p1 * p2, p0p1 * p2};
-    float3 acc;
-#pragma unroll
-    for (int c = 0; c < 8; ++c) {
-        const float mx = m[c].x + float(int(ix) + (c & 1));
-        const float my = m[c].y + float(int(iy) + ((c >> 1) & 1));
-        const float mz = m[c].z + float(int(iz) + ((c >> 2) & 1));
-        if (c == 0) {
-            acc.x = mx * w[0];
-            acc.y = my * w[0];
-            acc.z = mz * w[0];
-        } else {
-            acc.x = acc.x + mx * w[c];
-            acc.y = acc.y + my * w[c];
-            acc.z = acc.z + mz * w[c];
-        }
-    }
-    return use ? make_float3(acc.x - float(x), acc.y - float(y), acc.z - float(z)) : m[0];
-}
-
 // ---------------------------------------------------------------------------
-// accumulate_displacement then cdm_smooth in one pass, marching z:
-// out = smooth(acc), acc = the accumulated field of accumulate_kernel.
-// Tiles are laid out in flat-index space as in poisson2_kernel, so smooth's
-// neighbours p-+1 and p-+w are offsets (i-+1, j), (i, j-+1) of the tile grown
-// by 1 (row and plane wrap included) and p-+wh the same offset in planes
-// m-+1.  A position outside [0, n) holds +0.0, which adds nothing to the
-// neighbour sum (that sum starts at +0.0 and is never -0.0), as the
-// reference drops it.  Per plane the block computes acc once on the tile and
-// its 148-position ring (two branch-free evaluations per thread, their loads
-// in flight together) and keeps the planes in an LDS ring.  HBM traffic per
-// voxel: new_d read, cur gathered, out written (36 B, against 36 + 24 B for
-// the two passes).  Measured at 182x218x182, whole iterations: 1558
-// iterations/s against 1546 with the two passes, 1490 with branching
-// evaluations and 1538 with two planes a step (four evaluations, 125
-// VGPRs, half the occupancy).  out must not alias cur or nd.  With keep,
-// cur is also copied into keep (the best field taking the running one
-// before the step, as the reference's loop does), keep aliasing neither.
+// accumulate_displacement, cdm_smooth and the next iteration's
+// compose_displacement in one pass: out = smooth(acc), acc = the accumulated
+// field of accumulate_kernel, and Js(x) = Is(x + out(x)) where Js is given.
+// A block owns TX x TY x TZ outputs, evaluates acc on them and on the six
+// faces around them, keeps it in LDS, and smooths behind one barrier.  Offsets are flat-index offsets:
+// a cell past the end of its row or plane is the next row's or plane's first
+// voxel, as smooth's neighbours p-+1, p-+w, p-+wh are.  A position outside
+// [0, n) holds +0.0, which adds nothing to the neighbour sum (that sum starts
+// at +0.0 and is never -0.0), as the reference drops it.  HBM traffic per
+// voxel: new_d read, cur gathered, out written (36 B), Is gathered and Js
+// written (2 B).  out must not alias cur or nd.  With keep, cur is also
+// copied into keep (the best field taking the running one before the step, as
+// the reference's loop does), keep aliasing neither.
+// The eight 12-byte corner gathers bind the address unit (a quad of lanes a
+// cycle or two), so large volumes stage cur on the tile grown by 2 in LDS and
+// gather there; a sample that leaves it (a displacement of a voxel or more, a
+// wrapped neighbour) is evaluated again from memory.  Then vector issue binds.
+// Against the z-marching kernel without compose and compose_kernel after it:
+// 12.4 -> 5.1 us at 32x32x32, 24 -> 20 at 80x96x80, 177 -> 152 at
+// 182x218x182 (164 unstaged).
 // ---------------------------------------------------------------------------
+template <int TX, int TY, int TZ, int NT, bool STAGED>
 __device__ __forceinline__ void accumulate_smooth_body(
     const float* __restrict__ cur, const float* __restrict__ nd, const Lay& lay, float k, float w_6,
-    float w_1, const FieldGeo& g, int zq, float* __restrict__ out, float* __restrict__ keep,
-    const Block& blk)
+    float w_1, const FieldGeo& g, float* __restrict__ out, float* __restrict__ keep,
+    const uint8_t* __restrict__ Is, uint8_t* __restrict__ Js, const Block& blk)
 {
-    __shared__ float3 A[4][kS1Y][kS1X];
-    const int tx = int(threadIdx.x), ty = int(threadIdx.y), tid = ty * kQX + tx;
-    const int x0 = blk.x * kQX, y0 = blk.y * kQY;
-    const int z0 = blk.z * zq, z1 = min(z0 + zq, g.d);
-    const long long n = g.n, w = g.w, wh = g.wh;
-    const long long base = (long long)y0 * w + x0;
+    constexpr int kCore = TX * TY * TZ;
+    constexpr int kFx = TY * TZ, kFy = TX * TZ, kFz = TX * TY;  // one face along each axis
+    constexpr int kCells = kCore + 2 * (kFx + kFy + kFz);
+    constexpr int kSX = TX + 4, kSY = TY + 4, kSZ = TZ + 4, kSN = kSX * kSY * kSZ;
+    constexpr int kWaves = NT / 64, kBatch = 10;
+    static_assert(kCore % NT == 0 && kCells % NT == 0, "whole passes");
+    static_assert(!STAGED || ((kSY * kSZ) % (kWaves * kBatch) == 0 && 3 * kSX <= 64),
+                  "whole passes over the rows, each a wave wide at most");
+    // cur on the grown tile, one array per component; then acc on the cells
+    constexpr int kAccN = (TX + 2) * (TY + 2) * (TZ + 2);
+    static_assert(kAccN <= kSN, "acc fits the staged field");
+    __shared__ float field[3 * (STAGED ? kSN : kAccN)];
+    float3(*A)[TY + 2][TX + 2] = reinterpret_cast<float3(*)[TY + 2][TX + 2]>(field);
+    static_assert((NT & (NT - 1)) == 0, "the mask below");
+    const int tid = int(threadIdx.x) & (NT - 1);  // (its range decides most of cell())
+    const int x0 = blk.x * TX, y0 = blk.y * TY, z0 = blk.z * TZ;
     const __amdgpu_buffer_rsrc_t rcur = make_rsrc(cur, g.n * 12u);
-    int ri = 0, rj = 0;
-    const bool has_ring = tid < kRing;
-    if (has_ring) ring_offset(tid, ri, rj);
-    const long long ro = (long long)rj * w + ri;
-    const long long io = (long long)ty * w + tx;
-    const float3 zero = make_float3(0.0f, 0.0f, 0.0f);
-    auto acc_at = [&](long long q) -> float3 {
-        const bool ok = q >= 0 && q < n;
-        const uint32_t p = ok ? uint32_t(q) : 0u;
-        const uint32_t z = p / g.wh, r = p - z * g.wh;
-        const uint32_t y = r / uint32_t(g.w), x = r - y * uint32_t(g.w);
-        const float3 v = accumulated_bf(rcur, nd, lay, k, g, p, int(x), int(y), int(z));
-        return ok ? v : zero;
+    const int lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+
+    // the running field on the outputs grown by 2, a row a wave at a time:
+    // lane e takes dword e of the row's 3 (TX + 4)
+    if constexpr (STAGED) {
+        const int e = lane, cx = e / 3, gx = x0 - 2 + cx;
+        const uint32_t col = (e < 3 * kSX) & (uint32_t(gx) < uint32_t(g.w)) ? 0u : ~0u;
+        float* dst = &field[0] + (e % 3) * kSN + cx;
+        for (int r0 = wv; r0 < kSY * kSZ; r0 += kWaves * kBatch) {
+            float v[kBatch];
+#pragma unroll
+            for (int q = 0; q < kBatch; ++q) {
+                const int r = r0 + q * kWaves;
+                const int gy = y0 - 2 + r % kSY, gz = z0 - 2 + r / kSY;
+                const uint32_t at = (uint32_t(gz) * g.wh + uint32_t(gy) * uint32_t(g.w) + uint32_t(x0 - 2)) * 12u;
+                // rows and columns outside the volume read past the buffer: 0
+                const uint32_t row = (uint32_t(gy) < uint32_t(g.h)) & (uint32_t(gz) < uint32_t(g.d)) ? 0u : ~0u;
+                v[q] = __uint_as_float(
+                    __builtin_amdgcn_raw_buffer_load_b32(rcur, int((at + uint32_t(e) * 4u) | row | col), 0, 0));
+            }
+            if (e < 3 * kSX) {
+#pragma unroll
+                for (int q = 0; q < kBatch; ++q) dst[(r0 + q * kWaves) * kSX] = v[q];
+            }
+        }
+    }
+    auto cell = [&](int c, int& i, int& j, int& l) {
+        if (c < kCore) {
+            i = c % TX;
+            j = (c / TX) % TY;
+            l = c / (TX * TY);
+            return;
+        }
+        c -= kCore;
+        if (c < 2 * kFz) {
+            l = c < kFz ? -1 : TZ;
+            c = c < kFz ? c : c - kFz;
+            i = c % TX;
+            j = c / TX;
+            return;
+        }
+        c -= 2 * kFz;
+        if (c < 2 * kFy) {
+            j = c < kFy ? -1 : TY;
+            c = c < kFy ? c : c - kFy;
+            i = c % TX;
+            l = c / TX;
+            return;
+        }
+        c -= 2 * kFy;
+        i = c < kFx ? -1 : TX;
+        c = c < kFx ? c : c - kFx;
+        j = c % TY;
+        l = c / TY;
     };
-    auto fill = [&](int m) {
-        const long long pm = (long long)m * wh + base;
-        const float3 a_in = acc_at(pm + io);
-        const float3 a_r = has_ring ? acc_at(pm + ro) : zero;
-        float3(*da)[kS1X] = A[(m + 4) & 3];
-        da[ty + 1][tx + 1] = a_in;
-        if (has_ring) da[rj + 1][ri + 1] = a_r;
+    // cell c's voxel (x, y, z), its index p, and whether it is one
+    auto locate_cell = [&](int c, int& x, int& y, int& z, uint32_t& p) {
+        int i, j, l;
+        cell(c, i, j, l);
+        x = x0 + i;
+        y = y0 + j;
+        z = z0 + l;
+        // no output needs a cell more than one past the volume
+        bool ok = x <= g.w && y <= g.h && z <= g.d;
+        y = x < 0 ? y - 1 : x >= g.w ? y + 1 : y;
+        x = x < 0 ? x + g.w : x >= g.w ? x - g.w : x;
+        z = y < 0 ? z - 1 : y >= g.h ? z + 1 : z;
+        y = y < 0 ? y + g.h : y >= g.h ? y - g.h : y;
+        // (the last test: a cell one past both its row and a one-row plane)
+        p = uint32_t(z) * g.wh + uint32_t(y) * uint32_t(g.w) + uint32_t(x);
+        ok = ok && z >= 0 && z < g.d && p < g.n;
+        p = ok ? p : 0u;
+        return ok;
     };
-    auto smooth = [&](int m) {
-        if (m >= z1 || x0 + tx >= g.w || y0 + ty >= g.h) return;
-        float3(*am)[kS1X] = A[(m + 3) & 3];
-        float3(*ac)[kS1X] = A[(m + 4) & 3];
-        float3(*ap)[kS1X] = A[(m + 5) & 3];
-        const int ci = tx + 1, cj = ty + 1;
-        const float3 t[6] = {ac[cj][ci + 1], ac[cj][ci - 1], ac[cj + 1][ci],
-                             ac[cj - 1][ci], ap[cj][ci],     am[cj][ci]};
-        float3 v = zero;
+    // every new_d value first: one latency for all evaluations of a thread
+    constexpr int kEvals = kCells / NT;
+    float3 d[kEvals];
+#pragma unroll
+    for (int u = 0; u < kEvals; ++u) {
+        int x, y, z;
+        uint32_t p;
+        locate_cell(tid + u * NT, x, y, z, p);
+        d[u] = ld_lay(nd, p, lay);
+    }
+    if constexpr (STAGED) __syncthreads();
+    // accumulate_kernel's value, operation for operation: the eight corners
+    // from the staged tile where it holds them (a displacement below a voxel
+    // never leaves it), else from memory
+    float3 acc[kEvals];
+#pragma unroll
+    for (int u = 0; u < kEvals; ++u) {
+        int x, y, z;
+        uint32_t p;
+        const bool ok = locate_cell(tid + u * NT, x, y, z, p);
+        const float dx = d[u].x * k, dy = d[u].y * k, dz = d[u].z * k;
+        const bool moved = dx != 0.0f || dy != 0.0f || dz != 0.0f;
+        const float sx = dx + float(x), sy = dy + float(y), sz = dz + float(z);
+        const bool in = (fminf(fminf(sx, sy), sz) >= 0.0f) & (sx < g.wm1) & (sy < g.hm1) & (sz < g.dm1);
+        const bool use = moved && in;
+        const int ix = use ? int(cvt_u32_sat(sx)) : x, iy = use ? int(cvt_u32_sat(sy)) : y,
+                  iz = use ? int(cvt_u32_sat(sz)) : z;
+        const float p0 = sx - float(ix), p1 = sy - float(iy), p2 = sz - float(iz);
+        const float n0 = 1.0f - p0, n1 = 1.0f - p1, n2 = 1.0f - p2;
+        const float n0n1 = n0 * n1, p0n1 = p0 * n1, n0p1 = n0 * p1, p0p1 = p0 * p1;
+        const float w[8] = {n0n1 * n2, p0n1 * n2, n0p1 * n2, p0p1 * n2,
+                            n0n1 * p2, p0n1 * p2, n0p1 * p2, p0p1 * p2};
+        const float gx[2] = {float(ix), float(ix + 1)}, gy[2] = {float(iy), float(iy + 1)},
+                    gz[2] = {float(iz), float(iz + 1)};
+        auto blend = [&](auto corner_at) {
+            float3 t = make_float3(0.0f, 0.0f, 0.0f), m0 = t;
+#pragma unroll
+            for (int c = 0; c < 8; ++c) {
+                const float3 m = corner_at(c);
+                const float mx = m.x + gx[c & 1];
+                const float my = m.y + gy[(c >> 1) & 1];
+                const float mz = m.z + gz[(c >> 2) & 1];
+                if (c == 0) {
+                    m0 = m;
+                    t.x = mx * w[0];
+                    t.y = my * w[0];
+                    t.z = mz * w[0];
+                } else {
+                    t.x = t.x + mx * w[c];
+                    t.y = t.y + my * w[c];
+                    t.z = t.z + mz * w[c];
+                }
+            }
+            t = make_float3(t.x - float(x), t.y - float(y), t.z - float(z));
+            return make_float3(!ok ? 0.0f : use ? t.x : m0.x, !ok ? 0.0f : use ? t.y : m0.y,
+                               !ok ? 0.0f : use ? t.z : m0.z);
+        };
+        const uint32_t i0 = ok ? uint32_t(iz) * g.wh + uint32_t(iy) * uint32_t(g.w) + uint32_t(ix) : 0u;
+        auto from_memory = [&](int c) { return ld3_rsrc(rcur, corner(g, i0, c)); };
+        if constexpr (!STAGED) {
+            acc[u] = blend(from_memory);
+            continue;
+        }
+        const int tx = ix - (x0 - 2), ty = iy - (y0 - 2), tz = iz - (z0 - 2);
+        const bool staged = (uint32_t(tx) < uint32_t(kSX - 1)) & (uint32_t(ty) < uint32_t(kSY - 1)) &
+                            (uint32_t(tz) < uint32_t(kSZ - 1));
+        const float* q = &field[staged ? (tz * kSY + ty) * kSX + tx : 0];
+        acc[u] = blend([&](int c) {
+            const int o = (c & 1) + ((c & 2) ? kSX : 0) + ((c & 4) ? kSX * kSY : 0);
+            return make_float3(q[o], q[o + kSN], q[o + 2 * kSN]);
+        });
+        if (__ballot(!staged)) {
+            if (!staged) acc[u] = blend(from_memory);
+        }
+        // one evaluation's corners in registers at a time
+        asm volatile("" ::: "memory");
+    }
+    if constexpr (STAGED) __syncthreads();  // the staged field has been read
+#pragma unroll
+    for (int u = 0; u < kEvals; ++u) {
+        int i, j, l;
+        cell(tid + u * NT, i, j, l);
+        A[l + 1][j + 1][i + 1] = acc[u];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < kCore / NT; ++u) {
+        int i, j, l;
+        cell(tid + u * NT, i, j, l);
+        const int x = x0 + i, y = y0 + j, z = z0 + l;
+        if (x >= g.w || y >= g.h || z >= g.d) continue;
+        const float3 t[6] = {A[l + 1][j + 1][i + 2], A[l + 1][j + 1][i], A[l + 1][j + 2][i + 1],
+                             A[l + 1][j][i + 1],     A[l + 2][j + 1][i + 1], A[l][j + 1][i + 1]};
+        float3 v = make_float3(0.0f, 0.0f, 0.0f);
 #pragma unroll
         for (int e = 0; e < 6; ++e) {
             v.x = v.x + t[e].x;
             v.y = v.y + t[e].y;
             v.z = v.z + t[e].z;
         }
-        const float3 c = ac[cj][ci];
-        const uint32_t p = uint32_t((long long)m * wh + base + io);
-        st3(out, p, make_float3(c.x * w_1 + v.x * w_6, c.y * w_1 + v.y * w_6, c.z * w_1 + v.z * w_6));
+        const float3 c = A[l + 1][j + 1][i + 1];
+        const uint32_t p = uint32_t(z) * g.wh + uint32_t(y) * uint32_t(g.w) + uint32_t(x);
+        const float3 o = make_float3(c.x * w_1 + v.x * w_6, c.y * w_1 + v.y * w_6, c.z * w_1 + v.z * w_6);
+        st3(out, p, o);
         if (keep) st3(keep, p, ld3(cur, p));
-    };
-    fill(z0 - 1);
-    fill(z0);
-    for (int m = z0; m < z1; ++m) {
-        fill(m + 1);
-        __syncthreads();
-        smooth(m);
-        __syncthreads();
+        if (Js) Js[p] = composed(Is, g, x, y, z, p, o);
     }
 }
 
-__global__ __launch_bounds__(kQX * kQY) void accumulate_smooth_kernel(
-    const float* __restrict__ cur, const float* __restrict__ nd, Lay lay, float k, float w_6, float w_1,
-    FieldGeo g, int zq, float* __restrict__ out)
+// Outputs per block of accumulate_smooth_kernel: large volumes take the tile
+// with fewer faces (1.5 evaluations per output, not 2) and its staged field,
+// small ones the tile with more workgroups, whose gathers are a shorter chain
+// than staging first (5.1 against 8.0 us at 32x32x32).
+template <bool LARGE>
+struct AccTile {
+    static constexpr int kX = LARGE ? 16 : 8, kY = LARGE ? 16 : 8, kZ = LARGE ? 8 : 4;
+    static constexpr int kThreads = LARGE ? 512 : 256;
+};
+constexpr size_t kALargeVoxels = size_t(1) << 18;
+inline bool acc_large(const FieldGeo& g) { return g.n >= kALargeVoxels; }
+
+template <class Tile>
+dim3 acc_grid_t(const FieldGeo& g)
 {
-    accumulate_smooth_body(cur, nd, lay, k, w_6, w_1, g, zq, out, nullptr, logical_block());
+    return dim3(uint32_t((g.w + Tile::kX - 1) / Tile::kX), uint32_t((g.h + Tile::kY - 1) / Tile::kY),
+                uint32_t((g.d + Tile::kZ - 1) / Tile::kZ));
+}
+dim3 acc_grid(const FieldGeo& g)
+{
+    return acc_large(g) ? acc_grid_t<AccTile<true>>(g) : acc_grid_t<AccTile<false>>(g);
+}
+
+template <bool LARGE>
+__global__ __launch_bounds__(AccTile<LARGE>::kThreads, 4) void accumulate_smooth_kernel(
+    const float* __restrict__ cur, const float* __restrict__ nd, Lay lay, float k, float w_6, float w_1,
+    FieldGeo g, float* __restrict__ out, const uint8_t* __restrict__ Is, uint8_t* __restrict__ Js)
+{
+    using T = AccTile<LARGE>;
+    accumulate_smooth_body<T::kX, T::kY, T::kZ, T::kThreads, LARGE>(cur, nd, lay, k, w_6, w_1, g, out, nullptr, Is,
+                                                             Js, logical_block());
 }
 
 // ---------------------------------------------------------------------------
@@ -1406,7 +1531,7 @@ __global__ __launch_bounds__(GradTile<LARGE>::kThreads) void gradient_seg_kernel
     int s;
     const Block b = seg_block(st, s);
     gradient_r_box_body<Tile::kSide, Tile::kSide, Tile::kThreads>(st.Js[s], st.It[s], st.g[s], 0, st.nd[s],
-                                                                  Lay{3u, 1u}, st.partials[s], b);
+                                                                  packed_layout(), st.partials[s], b);
 }
 
 // one workgroup per field
@@ -1432,12 +1557,15 @@ __global__ __launch_bounds__(1024) void max_reduce_seg_kernel(const CdmStep st)
     max_reduce_body(st.maxparts[s], st.count[s], st.maxlen[s], st.host_maxlen[s]);
 }
 
-__global__ __launch_bounds__(kQX * kQY) void accumulate_smooth_seg_kernel(const CdmStep st)
+template <bool LARGE>
+__global__ __launch_bounds__(AccTile<LARGE>::kThreads, 4) void accumulate_smooth_seg_kernel(const CdmStep st)
 {
+    using T = AccTile<LARGE>;
     int s;
     const Block b = seg_block(st, s);
-    accumulate_smooth_body(st.cur[s], st.nd[s], Lay{3u, 1u}, st.k[s], st.w_6[s], st.w_1[s], st.g[s], st.zq[s],
-                           st.dst[s], st.keep[s], b);
+    accumulate_smooth_body<T::kX, T::kY, T::kZ, T::kThreads, LARGE>(st.cur[s], st.nd[s], packed_layout(), st.k[s],
+                                                             st.w_6[s], st.w_1[s], st.g[s], st.dst[s],
+                                                             st.keep[s], st.Is[s], st.Js[s], b);
 }
 
 // cdm_smooth: dd = d*(1-s) + (s/6)*(neighbours +1, -1, +w, -w, +wh, -wh by
@@ -1668,15 +1796,19 @@ void launch_accumulate(tiplhip_ctx* ctx, const float* cur, const float* nd, Lay 
     TIPLHIP_CHECK(hipGetLastError());
 }
 
-// accumulate then cdm_smooth with `smoothing` (non-zero) in one pass into out.
+// accumulate then cdm_smooth with `smoothing` (non-zero) in one pass into
+// out, and compose_displacement of Is by out into Js where Js is set.
 void launch_accumulate_smooth(tiplhip_ctx* ctx, const float* cur, const float* nd, Lay lay, float k,
-                              float smoothing, const FieldGeo& g, float* out)
+                              float smoothing, const FieldGeo& g, float* out, const uint8_t* Is, uint8_t* Js)
 {
     const float w_6 = smoothing / float(2.0f * 3.0f);
     const float w_1 = 1.0f - smoothing;
-    const int zq = poisson2_zq(g);
-    hipLaunchKernelGGL(accumulate_smooth_kernel, poisson2_grid(g, zq), dim3(kQX, kQY), 0, ctx->stream,
-                       cur, nd, lay, k, w_6, w_1, g, zq, out);
+    if (acc_large(g))
+        hipLaunchKernelGGL(accumulate_smooth_kernel<true>, acc_grid(g), dim3(AccTile<true>::kThreads), 0,
+                           ctx->stream, cur, nd, lay, k, w_6, w_1, g, out, Is, Js);
+    else
+        hipLaunchKernelGGL(accumulate_smooth_kernel<false>, acc_grid(g), dim3(AccTile<false>::kThreads), 0,
+                           ctx->stream, cur, nd, lay, k, w_6, w_1, g, out, Is, Js);
     TIPLHIP_CHECK(hipGetLastError());
 }
 
@@ -1723,7 +1855,7 @@ bool is_terminated(const CdmRun& r) { return r.terminated && *r.terminated; }
 // gate's lock.
 struct CdmJob : GateSlot {
     FieldGeo g{};
-    dim3 tile, box, p2;       // grids: compose, gradient, Jacobi and accumulate+smooth
+    dim3 tile, box, p2, acc;  // grids: compose, gradient, Jacobi, accumulate+smooth
     int zq_p2 = 0;
     const uint8_t* It = nullptr;
     const uint8_t* Is = nullptr;
@@ -1793,28 +1925,55 @@ void launch_cdm_steps(hipStream_t stream, CdmJob* const* J, int n)
         if (j.restore)
             TIPLHIP_CHECK(hipMemcpyAsync(j.cur, j.best, fb, hipMemcpyDeviceToDevice, stream));
     }
-    {
+    // the field update of the jobs that have one, compose_displacement
+    // included; one launch per tile shape among them
+    for (const bool large : {false, true}) {
         CdmStep st;
         CdmJob* sm[kMaxSegs];
         int m = 0;
         for (int s = 0; s < n; ++s)
-            if (J[s]->smooth) sm[m++] = J[s];
+            if (J[s]->smooth && acc_large(J[s]->g) == large) sm[m++] = J[s];
+        if (!m) continue;
+        st.nseg = uint32_t(m);
+        set_grids(st, sm, m, &CdmJob::acc);
+        for (int s = 0; s < m; ++s) {
+            const CdmJob& j = *sm[s];
+            st.g[s] = j.g;
+            st.cur[s] = j.s_src;
+            st.nd[s] = const_cast<float*>(j.s_nd);
+            st.dst[s] = j.s_out;
+            st.keep[s] = j.s_keep;
+            st.Is[s] = j.Is;
+            st.Js[s] = j.Js;
+            st.k[s] = j.k;
+            st.w_6[s] = j.w_6;
+            st.w_1[s] = j.w_1;
+        }
+        if (large)
+            hipLaunchKernelGGL(accumulate_smooth_seg_kernel<true>, dim3(st.total),
+                               dim3(AccTile<true>::kThreads), 0, stream, st);
+        else
+            hipLaunchKernelGGL(accumulate_smooth_seg_kernel<false>, dim3(st.total),
+                               dim3(AccTile<false>::kThreads), 0, stream, st);
+        TIPLHIP_CHECK(hipGetLastError());
+    }
+    // compose_displacement of the jobs whose field was not just updated
+    {
+        CdmStep st;
+        CdmJob* cj[kMaxSegs];
+        int m = 0;
+        for (int s = 0; s < n; ++s)
+            if (!J[s]->smooth) cj[m++] = J[s];
         if (m) {
             st.nseg = uint32_t(m);
-            set_grids(st, sm, m, &CdmJob::p2);
+            set_grids(st, cj, m, &CdmJob::tile);
             for (int s = 0; s < m; ++s) {
-                const CdmJob& j = *sm[s];
-                st.g[s] = j.g;
-                st.zq[s] = j.zq_p2;
-                st.cur[s] = j.s_src;
-                st.nd[s] = const_cast<float*>(j.s_nd);
-                st.dst[s] = j.s_out;
-                st.keep[s] = j.s_keep;
-                st.k[s] = j.k;
-                st.w_6[s] = j.w_6;
-                st.w_1[s] = j.w_1;
+                st.g[s] = cj[s]->g;
+                st.Is[s] = cj[s]->Is;
+                st.Js[s] = cj[s]->Js;
+                st.cur[s] = cj[s]->cur;
             }
-            hipLaunchKernelGGL(accumulate_smooth_seg_kernel, dim3(st.total), dim3(kQX, kQY), 0, stream, st);
+            hipLaunchKernelGGL(compose_seg_kernel, dim3(st.total), dim3(kTX, kTY), 0, stream, st);
             TIPLHIP_CHECK(hipGetLastError());
         }
     }
@@ -1838,9 +1997,6 @@ void launch_cdm_steps(hipStream_t stream, CdmJob* const* J, int n)
         st.n[s] = double(j.g.n);
         theta = theta || j.need_theta;
     }
-    set_grids(st, J, n, &CdmJob::tile);
-    hipLaunchKernelGGL(compose_seg_kernel, dim3(st.total), dim3(kTX, kTY), 0, stream, st);
-    TIPLHIP_CHECK(hipGetLastError());
     // one gradient launch per tile shape among the fields
     for (const bool large : {false, true}) {
         CdmStep gs;
@@ -2101,6 +2257,7 @@ bool cdm_iterate_batched(CdmRun& run, const uint8_t* It, const uint8_t* Is, cons
     job.box = box_grid(g);
     job.zq_p2 = poisson2_zq(g);
     job.p2 = poisson2_grid(g, job.zq_p2);
+    job.acc = acc_grid(g);
     job.It = It;
     job.Is = Is;
     job.Js = Js.as<uint8_t>();
@@ -2262,6 +2419,7 @@ bool cdm_level(CdmRun& run, const std::vector<const uint8_t*>& It,
     std::vector<float> cost;
     float best_cost = 3.402823466e+38f;
     float cur_smoothing = 0.8f;
+    bool composed = false;  // Js holds compose_displacement of cur
     std::vector<float> mod_cost(size_t(run.nmod));
     TIPLHIP_REQUIRE(run.nmod >= 1 && run.nmod <= 16, "1 to 16 modalities");
     ctx->h_cdm.reserve(sizeof(float) * 16);
@@ -2281,11 +2439,13 @@ bool cdm_level(CdmRun& run, const std::vector<const uint8_t*>& It,
         std::fill(slots, slots + run.nmod, kCostPending);
         float* h_cost = static_cast<float*>(ctx->h_cdm.dev);
         for (int i = 0; i < run.nmod; ++i) {
-            launch_compose(ctx, Is[size_t(i)], cur, g, Js.as<uint8_t>());
+            // (of a single modality the field update has composed Js)
+            if (!composed) launch_compose(ctx, Is[size_t(i)], cur, g, Js.as<uint8_t>());
             const char type = run.param.gradient_type[std::min(i, 7)] == 'd' ? 'd' : 'r';
             launch_gradient(ctx, Js.as<uint8_t>(), It[size_t(i)], g, type, i > 0 ? 1 : 0,
                             nd.as<float>(), lay, partials.as<double>(), d_cost + i, h_cost + i);
         }
+        composed = false;
         const bool need_theta = theta == 0.0f;
         float* solved = launch_poisson(ctx, nd.as<float>(), pa, pb, g, lay, 12,
                                        need_theta ? d_maxlen : nullptr, maxparts.as<float>());
@@ -2320,7 +2480,9 @@ bool cdm_level(CdmRun& run, const std::vector<const uint8_t*>& It,
         // accumulated field is then unused), as in the reference
         if (cur_smoothing != 0.0f) {
             float* spare = solved == pa ? pb : pa;
-            launch_accumulate_smooth(ctx, cur, solved, lay, k, cur_smoothing, g, spare);
+            composed = run.nmod == 1;
+            launch_accumulate_smooth(ctx, cur, solved, lay, k, cur_smoothing, g, spare, Is[0],
+                                     composed ? Js.as<uint8_t>() : nullptr);
             pa = cur;
             pb = solved;
             cur = spare;
