@@ -431,31 +431,38 @@ dim3 box_grid(const FieldGeo& g)
                 uint32_t((g.d + side - 1) / side));
 }
 
-// Sums the block partials in a fixed order and stores float(sum / n).
-__device__ __forceinline__ void cost_reduce_body(const double* __restrict__ partials,
-                                                 uint32_t count, double n, float* __restrict__ out,
-                                                 float* __restrict__ host_out)
+// Sums the block partials in a fixed order, the same for every workgroup size
+// that calls it, and stores float(sum / n): each of 256 threads sums its
+// strided share, then waves and their totals in order.
+struct CostReduce {
+    const double* partials = nullptr;
+    uint32_t count = 0;
+    double n = 0.0;
+    float* out = nullptr;
+    float* host_out = nullptr;
+};
+constexpr uint32_t kReduceThreads = 256;
+
+__device__ __forceinline__ void cost_reduce_body(const CostReduce& r, double* part)
 {
     double acc = 0.0;
-    for (uint32_t i = threadIdx.x; i < count; i += blockDim.x) acc += partials[i];
-    __shared__ double part[16];
+    if (threadIdx.x < kReduceThreads)
+        for (uint32_t i = threadIdx.x; i < r.count; i += kReduceThreads) acc += r.partials[i];
     acc = wave_sum_f64(acc);
-    if ((threadIdx.x & 63u) == 0) part[threadIdx.x >> 6] = acc;
+    if ((threadIdx.x & 63u) == 0 && threadIdx.x < kReduceThreads) part[threadIdx.x >> 6] = acc;
     __syncthreads();
     if (threadIdx.x == 0) {
         double s = 0.0;
-        for (uint32_t w = 0; w < (blockDim.x >> 6); ++w) s += part[w];
-        out[0] = float(s / n);
-        if (host_out) host_out[0] = float(s / n);
+        for (uint32_t w = 0; w < kReduceThreads / 64; ++w) s += part[w];
+        r.out[0] = float(s / r.n);
+        if (r.host_out) r.host_out[0] = float(s / r.n);
     }
 }
 
-__global__ __launch_bounds__(1024) void cost_reduce_kernel(const double* __restrict__ partials,
-                                                           uint32_t count, double n,
-                                                           float* __restrict__ out,
-                                                           float* __restrict__ host_out)
+__global__ __launch_bounds__(kReduceThreads) void cost_reduce_kernel(const CostReduce r)
 {
-    cost_reduce_body(partials, count, n, out, host_out);
+    __shared__ double part[kReduceThreads / 64];
+    cost_reduce_body(r, part);
 }
 
 // Max of the per-block maxima (non-negative floats), as float bits.
@@ -936,9 +943,21 @@ __device__ __forceinline__ void poisson4_body(const float* __restrict__ nd, cons
 template <bool FIRST>
 __global__ __launch_bounds__(kCThreads) void poisson4_kernel(const float* __restrict__ nd,
                                                              const float* __restrict__ a, FieldGeo g,
-                                                             Lay lay, float* __restrict__ b)
+                                                             Lay lay, float* __restrict__ b,
+                                                             const CostReduce cost)
 {
-    poisson4_body<FIRST>(nd, a, g, lay, b, xcd_remap(blockIdx.x, gridDim.x));
+    uint32_t blk = blockIdx.x, blocks = gridDim.x;
+    if (FIRST && cost.partials) {
+        // one more workgroup, the first, sums the gradient's cost
+        if (blk == 0) {
+            __shared__ double part[kReduceThreads / 64];
+            cost_reduce_body(cost, part);
+            return;
+        }
+        --blk;
+        --blocks;
+    }
+    poisson4_body<FIRST>(nd, a, g, lay, b, xcd_remap(blk, blocks));
 }
 
 // ---------------------------------------------------------------------------
@@ -1000,12 +1019,22 @@ template <int K, bool FIRST>
 __global__ __launch_bounds__(kMThreads, 4) void poisson_march_kernel(const float* __restrict__ nd,
                                                                   const float* __restrict__ a,
                                                                   FieldGeo g, March mg, Lay lay,
-                                                                  float* __restrict__ b)
+                                                                  float* __restrict__ b,
+                                                                  const CostReduce cost)
 {
-    __shared__ float edge[2][K][kMWaves][2][64];
+    __shared__ __align__(16) float edge[2][K][kMWaves][2][64];
+    uint32_t blk = blockIdx.x;
+    if (FIRST && cost.partials) {
+        // one more workgroup, the first, sums the gradient's cost
+        if (blk == 0) {
+            cost_reduce_body(cost, reinterpret_cast<double*>(edge));
+            return;
+        }
+        --blk;
+    }
     const int lane = int(threadIdx.x) & 63;
     const int wv = __builtin_amdgcn_readfirstlane(int(threadIdx.x) >> 6);
-    const uint32_t L = xcd_remap(blockIdx.x, mg.blocks);
+    const uint32_t L = xcd_remap(blk, mg.blocks);
     const uint32_t comp = L % 3u, tile = L / 3u;
     const int x0 = int(tile % mg.gx) * (64 - 2 * K) - K;
     const int y0 = int((tile / mg.gx) % mg.gy) * (kMRows - 2 * K) - K;
@@ -1535,10 +1564,11 @@ __global__ __launch_bounds__(GradTile<LARGE>::kThreads) void gradient_seg_kernel
 }
 
 // one workgroup per field
-__global__ __launch_bounds__(1024) void cost_reduce_seg_kernel(const CdmStep st)
+__global__ __launch_bounds__(kReduceThreads) void cost_reduce_seg_kernel(const CdmStep st)
 {
+    __shared__ double part[kReduceThreads / 64];
     const int s = int(blockIdx.x);
-    cost_reduce_body(st.partials[s], st.count[s], st.n[s], st.cost[s], st.host_cost[s]);
+    cost_reduce_body(CostReduce{st.partials[s], st.count[s], st.n[s], st.cost[s], st.host_cost[s]}, part);
 }
 
 template <bool FIRST, bool MAXLEN>
@@ -1660,7 +1690,15 @@ void launch_compose(tiplhip_ctx* ctx, const uint8_t* Is, const float* d, const F
     TIPLHIP_CHECK(hipGetLastError());
 }
 
-void launch_gradient(tiplhip_ctx* ctx, const uint8_t* Js, const uint8_t* It, const FieldGeo& g,
+// Queues the sum of a gradient's cost partials.
+void launch_cost_reduce(tiplhip_ctx* ctx, const CostReduce& r)
+{
+    hipLaunchKernelGGL(cost_reduce_kernel, dim3(1), dim3(kReduceThreads), 0, ctx->stream, r);
+    TIPLHIP_CHECK(hipGetLastError());
+}
+
+// Queues the gradient; the sum of its cost partials is left to the caller.
+CostReduce launch_gradient(tiplhip_ctx* ctx, const uint8_t* Js, const uint8_t* It, const FieldGeo& g,
                      char type, int accumulate, float* nd, Lay lay, double* partials, float* cost_out,
                      float* host_cost = nullptr)
 {
@@ -1681,9 +1719,7 @@ void launch_gradient(tiplhip_ctx* ctx, const uint8_t* Js, const uint8_t* It, con
         parts = bg.x * bg.y * bg.z;
     }
     TIPLHIP_CHECK(hipGetLastError());
-    hipLaunchKernelGGL(cost_reduce_kernel, dim3(1), dim3(1024), 0, ctx->stream, partials, parts,
-                       double(g.n), cost_out, host_cost);
-    TIPLHIP_CHECK(hipGetLastError());
+    return CostReduce{partials, parts, double(g.n), cost_out, host_cost};
 }
 
 // `sweeps` Jacobi sweeps, four per launch (poisson4_kernel for small volumes,
@@ -1693,8 +1729,12 @@ void launch_gradient(tiplhip_ctx* ctx, const uint8_t* Js, const uint8_t* It, con
 // last launch, or a pass of their own after a four-sweep one) are reduced by
 // max_reduce_kernel.
 float* launch_poisson(tiplhip_ctx* ctx, const float* nd, float* a, float* b, const FieldGeo& g, Lay lay,
-                      int sweeps, unsigned int* maxlen, float* maxparts)
+                      int sweeps, unsigned int* maxlen, float* maxparts,
+                      const CostReduce& cost = CostReduce{})
 {
+    // a gradient's cost partials, when given, are summed by one more workgroup
+    // of the first launch
+    const uint32_t extra = cost.partials ? 1u : 0u;
     float* src = a;
     float* dst = b;
     uint32_t last_blocks = 0;
@@ -1702,13 +1742,14 @@ float* launch_poisson(tiplhip_ctx* ctx, const float* nd, float* a, float* b, con
     while (done < sweeps) {
         const bool first = done == 0;
         if (sweeps - done >= kCH && poisson4_fits(g)) {
-            const dim3 grid(poisson4_blocks(g)), block(kCThreads);
+            const dim3 block(kCThreads);
+            const uint32_t blocks = poisson4_blocks(g);
             if (first)
-                hipLaunchKernelGGL(poisson4_kernel<true>, grid, block, 0, ctx->stream, nd, src, g, lay,
-                                   dst);
+                hipLaunchKernelGGL(poisson4_kernel<true>, dim3(blocks + extra), block, 0, ctx->stream, nd,
+                                   src, g, lay, dst, cost);
             else
-                hipLaunchKernelGGL(poisson4_kernel<false>, grid, block, 0, ctx->stream, nd, src, g, lay,
-                                   dst);
+                hipLaunchKernelGGL(poisson4_kernel<false>, dim3(blocks), block, 0, ctx->stream, nd, src, g,
+                                   lay, dst, CostReduce{});
             TIPLHIP_CHECK(hipGetLastError());
             done += kCH;
             if (done == sweeps && maxlen) {
@@ -1722,13 +1763,13 @@ float* launch_poisson(tiplhip_ctx* ctx, const float* nd, float* a, float* b, con
         }
         if (sweeps - done >= kMK && planar_fits(g)) {
             const March mg = march_of<kMK>(g);
-            const dim3 grid(mg.blocks), block(kMThreads);
+            const dim3 block(kMThreads);
             if (first)
-                hipLaunchKernelGGL((poisson_march_kernel<kMK, true>), grid, block, 0, ctx->stream, nd, src,
-                                   g, mg, lay, dst);
+                hipLaunchKernelGGL((poisson_march_kernel<kMK, true>), dim3(mg.blocks + extra), block, 0,
+                                   ctx->stream, nd, src, g, mg, lay, dst, cost);
             else
-                hipLaunchKernelGGL((poisson_march_kernel<kMK, false>), grid, block, 0, ctx->stream, nd, src,
-                                   g, mg, lay, dst);
+                hipLaunchKernelGGL((poisson_march_kernel<kMK, false>), dim3(mg.blocks), block, 0,
+                                   ctx->stream, nd, src, g, mg, lay, dst, CostReduce{});
             TIPLHIP_CHECK(hipGetLastError());
             done += kMK;
             if (done == sweeps && maxlen) {
@@ -1740,6 +1781,7 @@ float* launch_poisson(tiplhip_ctx* ctx, const float* nd, float* a, float* b, con
             std::swap(src, dst);
             continue;
         }
+        if (first && extra) launch_cost_reduce(ctx, cost);
         TIPLHIP_REQUIRE(lay.ps == 3u, "one- and two-sweep launches take packed fields");
         const bool pair = sweeps - done >= 2;
         const bool last = done + (pair ? 2 : 1) == sweeps && maxlen;
@@ -2023,7 +2065,7 @@ void launch_cdm_steps(hipStream_t stream, CdmJob* const* J, int n)
         TIPLHIP_CHECK(hipGetLastError());
     }
     for (int s = 0; s < n; ++s) st.count[s] = J[s]->box.x * J[s]->box.y * J[s]->box.z;
-    hipLaunchKernelGGL(cost_reduce_seg_kernel, dim3(st.nseg), dim3(1024), 0, stream, st);
+    hipLaunchKernelGGL(cost_reduce_seg_kernel, dim3(st.nseg), dim3(kReduceThreads), 0, stream, st);
     TIPLHIP_CHECK(hipGetLastError());
     set_grids(st, J, n, &CdmJob::p2);
     for (int s = 0; s < n; ++s) {
@@ -2395,13 +2437,16 @@ bool cdm_level(CdmRun& run, const std::vector<const uint8_t*>& It,
         !run.no_early_exit && n <= run.ctx->cdm_batch->max_voxels())
         return cdm_iterate_batched(run, It[0], Is[0], g, best_d);
 
-    // three fields rotate: the running field and the two Jacobi buffers;
-    // accumulate+smooth writes the new running field into the Jacobi buffer
-    // that does not hold the solved new_d
+    // four fields rotate: the running field, the best field so far -- which may
+    // be the running one: then `spare_field` holds the fourth -- and the two
+    // Jacobi buffers.  accumulate+smooth writes the new running field into the
+    // Jacobi buffer that does not hold the solved new_d.
     DevMem f0(ctx, fb), f1(ctx, fb), f2(ctx, fb), nd(ctx, fb), Js(ctx, n);
-    float* cur = f0.as<float>();
-    float* pa = f1.as<float>();
-    float* pb = f2.as<float>();
+    float* cur = best_d;
+    float* best = best_d;
+    float* pa = f0.as<float>();
+    float* pb = f1.as<float>();
+    float* spare_field = f2.as<float>();
     const uint32_t nblocks = block_count(g);
     DevMem partials(ctx, sizeof(double) * nblocks), maxparts(ctx, sizeof(float) * nblocks);
     DevMem scal(ctx, sizeof(float) * 16 + sizeof(unsigned int));
@@ -2413,7 +2458,6 @@ bool cdm_level(CdmRun& run, const std::vector<const uint8_t*>& It,
     // can be reused
     auto drain = [ctx] { (void)hipStreamSynchronize(ctx->stream); };
     DrainOnUnwind<decltype(drain)> unwind(drain);
-    copy_d2d(ctx, cur, best_d, fb);
 
     float theta = 0.0f;
     std::vector<float> cost;
@@ -2438,17 +2482,20 @@ bool cdm_level(CdmRun& run, const std::vector<const uint8_t*>& It,
         uint32_t* slots = ctx->h_cdm.as<uint32_t>();
         std::fill(slots, slots + run.nmod, kCostPending);
         float* h_cost = static_cast<float*>(ctx->h_cdm.dev);
+        CostReduce reduce;
         for (int i = 0; i < run.nmod; ++i) {
             // (of a single modality the field update has composed Js)
             if (!composed) launch_compose(ctx, Is[size_t(i)], cur, g, Js.as<uint8_t>());
             const char type = run.param.gradient_type[std::min(i, 7)] == 'd' ? 'd' : 'r';
-            launch_gradient(ctx, Js.as<uint8_t>(), It[size_t(i)], g, type, i > 0 ? 1 : 0,
-                            nd.as<float>(), lay, partials.as<double>(), d_cost + i, h_cost + i);
+            reduce = launch_gradient(ctx, Js.as<uint8_t>(), It[size_t(i)], g, type, i > 0 ? 1 : 0,
+                                     nd.as<float>(), lay, partials.as<double>(), d_cost + i, h_cost + i);
+            // the last modality's sum rides on the first Poisson launch
+            if (i + 1 < run.nmod) launch_cost_reduce(ctx, reduce);
         }
         composed = false;
         const bool need_theta = theta == 0.0f;
         float* solved = launch_poisson(ctx, nd.as<float>(), pa, pb, g, lay, 12,
-                                       need_theta ? d_maxlen : nullptr, maxparts.as<float>());
+                                       need_theta ? d_maxlen : nullptr, maxparts.as<float>(), reduce);
         wait_for_slots(static_cast<const volatile uint32_t*>(slots), size_t(run.nmod), kCostPending,
                        std::chrono::microseconds(kCostSpinUs),
                        [ctx] { TIPLHIP_CHECK(hipStreamSynchronize(ctx->stream)); });
@@ -2461,11 +2508,17 @@ bool cdm_level(CdmRun& run, const std::vector<const uint8_t*>& It,
         cost.push_back(sum_cost / float(run.nmod));
         if (cost.back() < best_cost) {
             best_cost = cost.back();
-            if (index) copy_d2d(ctx, best_d, cur, fb);
+            if (best != cur) {
+                spare_field = best;
+                best = cur;
+            }
         }
         if (!cdm_improved(cost) && !run.no_early_exit) {
             if (cur_smoothing <= run.param.smoothing) break;
-            copy_d2d(ctx, cur, best_d, fb);
+            if (best != cur) {
+                spare_field = cur;
+                cur = best;
+            }
             cur_smoothing *= 0.5f;
             cost.clear();
         }
@@ -2483,13 +2536,14 @@ bool cdm_level(CdmRun& run, const std::vector<const uint8_t*>& It,
             composed = run.nmod == 1;
             launch_accumulate_smooth(ctx, cur, solved, lay, k, cur_smoothing, g, spare, Is[0],
                                      composed ? Js.as<uint8_t>() : nullptr);
-            pa = cur;
+            pa = cur == best ? spare_field : cur;
             pb = solved;
             cur = spare;
         }
     }
     // timing mode reports the running field after the fixed iteration count
-    if (run.no_early_exit) copy_d2d(ctx, best_d, cur, fb);
+    const float* result = run.no_early_exit ? cur : best;
+    if (result != best_d) copy_d2d(ctx, best_d, result, fb);
     TIPLHIP_CHECK(hipStreamSynchronize(ctx->stream));
     return true;
 }
@@ -2543,6 +2597,7 @@ void cdm_fixed(CdmRun& run, const std::vector<const uint8_t*>& It,
         for (int i = 0; i < run.nmod; ++i) {
             launch_compose(ctx, Is[size_t(i)], field, g, Js.as<uint8_t>());
             const char type = run.param.gradient_type[std::min(i, 7)] == 'd' ? 'd' : 'r';
+            // (the fixed schedule does not look at the cost)
             launch_gradient(ctx, Js.as<uint8_t>(), It[size_t(i)], g, type, i > 0 ? 1 : 0,
                             nd.as<float>(), lay, partials.as<double>(), d_cost + i);
         }
@@ -2720,8 +2775,9 @@ int tiplhip_cdm_gradient(tiplhip_ctx* ctx, const uint8_t* Js, const uint8_t* It,
         DevMem part(ctx, sizeof(double) * block_count(g)), dc(ctx, sizeof(float));
         TIPLHIP_CHECK(hipMemcpyAsync(dJ.p, Js, g.n, hipMemcpyHostToDevice, ctx->stream));
         TIPLHIP_CHECK(hipMemcpyAsync(dI.p, It, g.n, hipMemcpyHostToDevice, ctx->stream));
-        launch_gradient(ctx, dJ.as<uint8_t>(), dI.as<uint8_t>(), g, type, 0, dN.as<float>(),
-                        packed_layout(), part.as<double>(), dc.as<float>());
+        launch_cost_reduce(ctx, launch_gradient(ctx, dJ.as<uint8_t>(), dI.as<uint8_t>(), g, type, 0,
+                                                dN.as<float>(), packed_layout(), part.as<double>(),
+                                                dc.as<float>()));
         TIPLHIP_CHECK(hipMemcpyAsync(new_d, dN.p, sizeof(float) * 3 * g.n, hipMemcpyDeviceToHost, ctx->stream));
         float c = 0.0f;
         TIPLHIP_CHECK(hipMemcpyAsync(&c, dc.p, sizeof(float), hipMemcpyDeviceToHost, ctx->stream));
