@@ -63,11 +63,12 @@ def test_poisson_four_sweep_tiles(ctx, oracle, shape):
 
 
 @pytest.mark.parametrize("shape", [(64, 64, 64), (64, 64, 65), (3, 300, 301), (300, 3, 301), (301, 300, 3),
-                                   (70, 57, 113), (90, 48, 112)])
+                                   (70, 57, 113), (90, 48, 112), (1, 1, 2700000)])
 def test_poisson_marched_tiles(ctx, oracle, shape):
     """The largest volume on 8 x 8 x 8 tiles and larger ones that march z:
     thinner than the halo along each axis, and with rows and planes ending on
-    and inside the 56 x 24 core of a column.  13 sweeps end in a single one."""
+    and inside the 56 x 24 core of a column.  13 sweeps end in a single one.
+    The last: rows so long that the marched kernel's offsets would overflow."""
     nd = np.random.default_rng(5).standard_normal(shape + (3,)).astype(np.float32)
     for sweeps in (12, 13):
         out, ml = ctx.poisson(nd, sweeps)

@@ -20,10 +20,10 @@
 // read back per iteration; everything else stays on the device.
 #include "cdm_control.hpp"
 #include "device.hpp"
-#include "div_count.hpp"
 #include "field.hpp"
 #include "host_wait.hpp"
 #include "internal.hpp"
+#include "regression.hpp"
 #include "step_gate.hpp"
 
 #include <algorithm>
@@ -46,12 +46,16 @@ namespace {
 // array per component), so that kernels which take one component each read
 // whole lines: twelve sweeps 269 -> 204 us at 182x218x182, 120 against 216 at
 // 160x192x160.  Packed like the displacement fields where a caller's buffer
-// is, and where 12 n reaches 2^31.
+// is, and where byte offsets, those of a grown tile's planes and rows outside
+// the volume included, would pass 2^31.
 struct Lay {
     uint32_t ps, cs;
 };
 __host__ __device__ inline Lay packed_layout() { return Lay{3u, 1u}; }
-inline bool planar_fits(const FieldGeo& g) { return size_t(g.n) * 12 < (size_t(1) << 31); }
+inline bool planar_fits(const FieldGeo& g)
+{
+    return (size_t(g.n) + 8 * size_t(g.wh) + 64 * size_t(g.w)) * 12 < (size_t(1) << 31);
+}
 inline Lay grad_layout(const FieldGeo& g) { return planar_fits(g) ? Lay{1u, g.n} : packed_layout(); }
 
 __device__ inline float3 ld_lay(const float* f, uint32_t p, const Lay& l)
@@ -215,38 +219,6 @@ __global__ __launch_bounds__(256) void gradient_kernel(const uint8_t* __restrict
 constexpr uint32_t kCostPending = 0x7FC0C057u;
 constexpr int kCostSpinUs = 2000;
 
-struct Sums5 {
-    uint32_t j, i, jj, ii, ji;
-};
-
-// The regression of one voxel: the factor of its image gradient (0 where the
-// voxel takes no part) and its cost term.  linear_regression's FP64 order.
-__device__ inline float regress(uint32_t js, uint32_t it, const Sums5& s, int count, float& cost)
-{
-    if (js == 0u || it == 0u) return 0.0f;
-    double dn = 125.0, inv = 1.0 / 125.0;
-    if (count != 125) {
-        dn = double(count);
-        inv = 1.0 / dn;
-    }
-    const double mean_x = div_count(s.j, dn, inv);
-    const double mean_y = div_count(s.i, dn, inv);
-    const double x_var = div_count(s.jj, dn, inv) - mean_x * mean_x;
-    const double y_var = div_count(s.ii, dn, inv) - mean_y * mean_y;
-    if (x_var == 0.0 || y_var == 0.0) return 0.0f;
-    const double cov = div_count(s.ji, dn, inv) - mean_x * mean_y;
-    const float a = float(cov / x_var);
-    if (!(a > 0.0f)) return 0.0f;
-    const float b = float(mean_y - double(a) * mean_x);
-    const float r2 = float(cov * cov / x_var / y_var);
-    float sc = float(js) * a;
-    sc = sc + b;
-    sc = sc - float(it);
-    sc = r2 * sc;
-    cost = -r2;
-    return sc;
-}
-
 constexpr int kGX = 16;     // outputs per tile row
 constexpr int kGWords = 6;  // dwords that hold a row's 20 bytes at any alignment
 
@@ -366,7 +338,7 @@ __device__ __forceinline__ void gradient_r_box_body(const uint8_t* __restrict__ 
         const int ny = min(v.y + 2, g.h - 1) - max(v.y - 2, 0) + 1;
         const int nz = min(v.z + 2, g.d - 1) - max(v.z - 2, 0) + 1;
         float cost = 0.0f;
-        const float sc = regress(byte_at(0, r, 0), byte_at(1, r, 0),
+        const float sc = regress<125>(byte_at(0, r, 0), byte_at(1, r, 0),
                                  Sums5{s.x & 0xffffu, s.x >> 16, s.y, s.z, s.w}, nx * ny * nz, cost);
         float3 gr = make_float3(0.0f, 0.0f, 0.0f);
         if (cost != 0.0f || sc != 0.0f) {

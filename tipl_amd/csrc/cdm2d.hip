@@ -19,9 +19,10 @@
 //   cdm / cdm_cuda              reg/cdm.hpp:373-532
 //
 // A slice is 10^4..10^6 pixels, a fraction of the chip, so the loop is bound
-// by launches: each step is one kernel with one thread per pixel on 64 x 4
-// tiles, except the Jacobi solve, which runs four (or two) sweeps per launch
-// over flat-index tiles held in LDS.  The loop control (cost history,
+// by launches and by the chain inside each: an iteration is three of them --
+// gradient, all twelve Jacobi sweeps with the cost sum, and the field update
+// with the next composition -- each a load, a few barriers and a store.
+// (218x182, per iteration: 26 us with eight launches, 13.5 now.)  The loop control (cost history,
 // cdm_improved, smoothing schedule) runs on the host from the modality costs,
 // which the cost reduction stores into coherent host memory while the Jacobi
 // sweeps are already queued, as in the 3-D loop.  Fields are packed float2
@@ -32,6 +33,7 @@
 #include "field.hpp"
 #include "host_wait.hpp"
 #include "internal.hpp"
+#include "regression.hpp"
 
 #include <algorithm>
 #include <chrono>
@@ -213,26 +215,6 @@ __global__ __launch_bounds__(kThreads2) void up2_kernel(const float* __restrict_
 
 // ---- the loop body ----------------------------------------------------------
 
-// compose_displacement: Js(x) = Is(x + d(x)); an exact copy where d(x) == 0,
-// 0 where the sample is outside.
-__global__ __launch_bounds__(kThreads2) void compose2_kernel(const uint8_t* __restrict__ Is,
-                                                             Geo2 g, const float* __restrict__ d,
-                                                             uint8_t* __restrict__ Js)
-{
-    const Pix q = this_pixel(g);
-    if (!q.ok) return;
-    const float2 v = ld2(d, q.p);
-    if (v.x == 0.0f && v.y == 0.0f) {
-        Js[q.p] = Is[q.p];
-        return;
-    }
-    float px = float(q.x), py = float(q.y);
-    px += v.x;
-    py += v.y;
-    Bil b;
-    Js[q.p] = locate2(g, px, py, b) ? bil_u8(Is, g, b) : uint8_t(0);
-}
-
 // gradient_at (2-D): central differences, 0 on the first and last column/row.
 __device__ inline float2 gradient_at2(const uint8_t* I, const Geo2& g, const Pix& q)
 {
@@ -256,70 +238,25 @@ __device__ inline double block_sum_f64(double v, double* sh)
     return sh[0];
 }
 
-// cdm_get_gradient: new_d(x) for 'r' (windowed regression of It on Js) or
-// 'd' (SSD); `accumulate` adds it to nd (the modality sum new_d += dd, with
-// dd zero where a pixel contributes nothing).  Each block's FP64 cost sum
-// goes to part[block].
-__global__ __launch_bounds__(kThreads2) void gradient2_kernel(const uint8_t* __restrict__ Js,
-                                                              const uint8_t* __restrict__ It,
-                                                              Geo2 g, char type, int accumulate,
-                                                              float* __restrict__ nd,
-                                                              double* __restrict__ part)
+// cdm_get_gradient 'd' (SSD): new_d(x); `accumulate` adds it to nd (the
+// modality sum new_d += dd, with dd zero where a pixel contributes nothing).
+// Each block's FP64 cost sum goes to part[block].
+__global__ __launch_bounds__(kThreads2) void gradient2_d_kernel(const uint8_t* __restrict__ Js,
+                                                                const uint8_t* __restrict__ It,
+                                                                Geo2 g, int accumulate,
+                                                                float* __restrict__ nd,
+                                                                double* __restrict__ part)
 {
     __shared__ double sh[kThreads2];
     const Pix q = this_pixel(g);
     float cost = 0.0f;
     if (q.ok) {
-        float2 val = make_float2(0.0f, 0.0f);
-        if (type == 'd') {
-            const float2 gr = gradient_at2(Js, g, q);
-            const int dif = int(Js[q.p]) - int(It[q.p]);
-            val.x = 0.0f + gr.x * float(dif);
-            val.y = 0.0f + gr.y * float(dif);
-            cost = float(dif * dif);
-        } else if (Js[q.p] != 0 && It[q.p] != 0) {
-            const int x0 = max(q.x - 2, 0), x1 = min(q.x + 2, g.w - 1);
-            const int y0 = max(q.y - 2, 0), y1 = min(q.y + 2, g.h - 1);
-            // at most 25 * 255^2 per sum: exact in int32
-            int sx = 0, sxx = 0, sy = 0, syy = 0, sxy = 0;
-            for (int yy = y0; yy <= y1; ++yy) {
-                const uint32_t row = uint32_t(yy) * uint32_t(g.w);
-                for (int xx = x0; xx <= x1; ++xx) {
-                    const int a = Js[row + uint32_t(xx)], b = It[row + uint32_t(xx)];
-                    sx += a;
-                    sxx += a * a;
-                    sy += b;
-                    syy += b * b;
-                    sxy += a * b;
-                }
-            }
-            const double dn = double((x1 - x0 + 1) * (y1 - y0 + 1));
-            const double mean_x = double(sx) / dn;
-            const double mean_y = double(sy) / dn;
-            const double x_var = double(sxx) / dn - mean_x * mean_x;
-            const double y_var = double(syy) / dn - mean_y * mean_y;
-            float a, b, r2;
-            if (x_var == 0.0 || y_var == 0.0) {
-                a = 0.0f;
-                b = float(mean_y);
-                r2 = 0.0f;
-            } else {
-                const double cov = double(sxy) / dn - mean_x * mean_y;
-                a = float(cov / x_var);
-                b = float(mean_y - double(a) * mean_x);
-                r2 = float(cov * cov / x_var / y_var);
-            }
-            if (a > 0.0f) {
-                const float2 gr = gradient_at2(Js, g, q);
-                float s = float(Js[q.p]) * a;
-                s = s + b;
-                s = s - float(It[q.p]);
-                s = r2 * s;
-                val.x = 0.0f + gr.x * s;
-                val.y = 0.0f + gr.y * s;
-                cost = -r2;
-            }
-        }
+        const float2 gr = gradient_at2(Js, g, q);
+        const int dif = int(Js[q.p]) - int(It[q.p]);
+        float2 val;
+        val.x = 0.0f + gr.x * float(dif);
+        val.y = 0.0f + gr.y * float(dif);
+        cost = float(dif * dif);
         if (accumulate) {
             const float2 o = ld2(nd, q.p);
             val.x = o.x + val.x;
@@ -331,21 +268,211 @@ __global__ __launch_bounds__(kThreads2) void gradient2_kernel(const uint8_t* __r
     if (threadIdx.x == 0 && threadIdx.y == 0) part[blockIdx.y * gridDim.x + blockIdx.x] = s;
 }
 
-// float(mean(cost_map)): the block sums added in block order, then / n;
-// also stored into host-visible memory when host_out is set.
-__global__ __launch_bounds__(kThreads2) void cost2_final_kernel(const double* __restrict__ part,
-                                                                uint32_t nparts, uint32_t n,
-                                                                float* __restrict__ out,
-                                                                float* __restrict__ host_out)
+// cdm_get_gradient 'r' (windowed regression of It on Js).  A block owns
+// 16 x 16 outputs: it stages both images' bytes with a 2-pixel halo (zero
+// outside) in LDS, forms the 5-tap sums along x, then y, one pass over LDS
+// each, and regresses.  Sum Js and sum It share a word (at most 25 * 255 each).
+// Latency bounds it: 6.4 -> 4.0 us at 109x91, 5.9 -> 3.9 below, against every pixel
+// reading its 50 window bytes from memory.
+constexpr int kG2 = 16, kG2Halo = kG2 + 4;
+
+dim3 tiles2(const Geo2& g)
 {
-    __shared__ double sh[kThreads2];
-    const uint32_t t = threadIdx.y * kBX + threadIdx.x;
+    return dim3(uint32_t((g.w + kG2 - 1) / kG2), uint32_t((g.h + kG2 - 1) / kG2));
+}
+
+__global__ __launch_bounds__(kThreads2) void gradient2_r_kernel(const uint8_t* __restrict__ Js,
+                                                                const uint8_t* __restrict__ It,
+                                                                Geo2 g, int accumulate,
+                                                                float* __restrict__ nd,
+                                                                double* __restrict__ part)
+{
+    static_assert(kG2 * kG2 == int(kThreads2), "one output per thread");
+    __shared__ uint8_t js[kG2Halo][kG2Halo], is[kG2Halo][kG2Halo];
+    __shared__ uint4 xs[kG2Halo][kG2];  // {j | i << 16, jj, ii, ji} along x
+    __shared__ double wave_part[kThreads2 / 64];
+    const int t = int(threadIdx.y) * kBX + int(threadIdx.x);
+    const int x0 = int(blockIdx.x) * kG2, y0 = int(blockIdx.y) * kG2;
+    for (int c = t; c < kG2Halo * kG2Halo; c += int(kThreads2)) {
+        const int cx = c % kG2Halo, cy = c / kG2Halo;
+        const int x = x0 - 2 + cx, y = y0 - 2 + cy;
+        const bool in = x >= 0 && x < g.w && y >= 0 && y < g.h;
+        const uint32_t p = in ? uint32_t(y) * uint32_t(g.w) + uint32_t(x) : 0u;
+        js[cy][cx] = in ? Js[p] : uint8_t(0);
+        is[cy][cx] = in ? It[p] : uint8_t(0);
+    }
+    __syncthreads();
+    for (int c = t; c < kG2Halo * kG2; c += int(kThreads2)) {
+        const int cx = c % kG2, cy = c / kG2;
+        uint4 s = make_uint4(0u, 0u, 0u, 0u);
+#pragma unroll
+        for (int k = 0; k < 5; ++k) {
+            const uint32_t a = js[cy][cx + k], b = is[cy][cx + k];
+            s.x += a | (b << 16);
+            s.y += a * a;
+            s.z += b * b;
+            s.w += a * b;
+        }
+        xs[cy][cx] = s;
+    }
+    __syncthreads();
+    const int cx = t % kG2, cy = t / kG2;
+    Pix q;
+    q.x = x0 + cx;
+    q.y = y0 + cy;
+    q.p = uint32_t(q.y) * uint32_t(g.w) + uint32_t(q.x);
+    float cost = 0.0f;
+    if (q.x < g.w && q.y < g.h) {
+        uint4 s = xs[cy][cx];
+#pragma unroll
+        for (int k = 1; k < 5; ++k) {
+            const uint4 u = xs[cy + k][cx];
+            s.x += u.x;
+            s.y += u.y;
+            s.z += u.z;
+            s.w += u.w;
+        }
+        const int nx = min(q.x + 2, g.w - 1) - max(q.x - 2, 0) + 1;
+        const int ny = min(q.y + 2, g.h - 1) - max(q.y - 2, 0) + 1;
+        const float sc = regress<25>(js[cy + 2][cx + 2], is[cy + 2][cx + 2],
+                                     Sums5{s.x & 0xffffu, s.x >> 16, s.y, s.z, s.w}, nx * ny, cost);
+        float2 val = make_float2(0.0f, 0.0f);
+        if (cost != 0.0f || sc != 0.0f) {
+            // gradient_at2 from the staged bytes
+            const float gx = (q.x + 1 < g.w && q.x) ? float(int(js[cy + 2][cx + 3]) - int(js[cy + 2][cx + 1])) : 0.0f;
+            const float gy = (q.y + 1 < g.h && q.y) ? float(int(js[cy + 3][cx + 2]) - int(js[cy + 1][cx + 2])) : 0.0f;
+            val.x = 0.0f + gx * sc;
+            val.y = 0.0f + gy * sc;
+        }
+        if (accumulate) {
+            const float2 o = ld2(nd, q.p);
+            val.x = o.x + val.x;
+            val.y = o.y + val.y;
+        }
+        st2(nd, q.p, val);
+    }
+    const double w = wave_sum_f64(double(cost));
+    if ((t & 63) == 0) wave_part[t >> 6] = w;
+    __syncthreads();
+    if (t == 0)
+        part[blockIdx.y * gridDim.x + blockIdx.x] =
+            (wave_part[0] + wave_part[1]) + (wave_part[2] + wave_part[3]);
+}
+
+// float(mean(cost_map)) from the gradient's block sums: each of 256 threads
+// adds its strided share, then waves and their totals in order.  Also stored
+// into host-visible memory when host_out is set.
+struct CostReduce2 {
+    const double* part = nullptr;
+    uint32_t count = 0, n = 0;
+    float* out = nullptr;
+    float* host_out = nullptr;
+};
+
+__device__ inline void cost_reduce2(const CostReduce2& r, uint32_t t, double* sh)
+{
     double s = 0.0;
-    for (uint32_t i = t; i < nparts; i += kThreads2) s += part[i];
-    const double tot = block_sum_f64(s, sh);
+    if (t < kThreads2)
+        for (uint32_t i = t; i < r.count; i += kThreads2) s += r.part[i];
+    s = wave_sum_f64(s);
+    if ((t & 63u) == 0 && t < kThreads2) sh[t >> 6] = s;
+    __syncthreads();
     if (t == 0) {
-        *out = float(tot / double(n));
-        if (host_out) *host_out = float(tot / double(n));
+        const double tot = (sh[0] + sh[1]) + (sh[2] + sh[3]);
+        *r.out = float(tot / double(r.n));
+        if (r.host_out) *r.host_out = float(tot / double(r.n));
+    }
+}
+
+__global__ __launch_bounds__(kThreads2) void cost2_final_kernel(const CostReduce2 r)
+{
+    __shared__ double sh[kThreads2 / 64];
+    cost_reduce2(r, threadIdx.x, sh);
+}
+
+// Up to twelve Jacobi sweeps of cdm_solve_poisson in one launch.  The two
+// components are independent, so a workgroup takes one component of a 40 x 40
+// tile, grown by 12 on every side to 64 x 64: lane l of wave v holds rows
+// 4 v .. 4 v + 3 of column l in registers.  p -+ 1 are the neighbouring lanes
+// (DPP wave shift), p -+ w the thread's other rows, or, at a wave's first and
+// last row, a value the neighbouring wave left in LDS: one barrier a sweep.
+// Offsets are flat-index offsets (row wrap included); positions outside
+// [0, n) read 0 through the buffer's range check and are kept 0, which
+// changes nothing where the reference drops the neighbour (x - (+0) == x).  A
+// sweep spoils one layer of the grown tile, so up to twelve leave the core
+// exact.  Latency bounds it: twelve sweeps of 109x91 in one launch of 6.4 us
+// (three of 8.1 us with four sweeps a launch over flat segments in LDS).
+// One more workgroup, the first, sums the gradient's cost when asked to.
+constexpr int kP2Halo = 12, kP2Rows = 4, kP2Waves = 16, kP2Side = kP2Rows * kP2Waves;
+constexpr int kP2Core = kP2Side - 2 * kP2Halo;
+static_assert(kP2Side == 64, "a tile row is one wave");
+
+__global__ __launch_bounds__(64 * kP2Waves) void poisson2d_tile_kernel(const float* __restrict__ nd,
+                                                                       const float* __restrict__ src,
+                                                                       Geo2 g, int first, int sweeps,
+                                                                       float* __restrict__ dst,
+                                                                       const CostReduce2 cost)
+{
+    __shared__ float edge[2][kP2Waves + 2][2][64];  // a wave's first and last row
+    constexpr float inv_d2 = -0.5f / 2.0f;
+    uint32_t blk = blockIdx.x;
+    if (cost.part) {
+        if (blk == 0) {
+            __shared__ double sh[kThreads2 / 64];
+            cost_reduce2(cost, threadIdx.x, sh);
+            return;
+        }
+        --blk;
+    }
+    const int lane = int(threadIdx.x) & 63;
+    const int wv = __builtin_amdgcn_readfirstlane(int(threadIdx.x) >> 6);
+    const uint32_t gx = uint32_t((g.w + kP2Core - 1) / kP2Core);
+    const uint32_t comp = blk & 1u, tile = blk >> 1;
+    const int x0 = int(tile % gx) * kP2Core - kP2Halo, y0 = int(tile / gx) * kP2Core - kP2Halo;
+    const int w = g.w, n = int(g.n);
+    const int q0 = (y0 + wv * kP2Rows) * w + x0 + lane;
+    const __amdgpu_buffer_rsrc_t rn = make_rsrc(nd, g.n * 8u);
+    const __amdgpu_buffer_rsrc_t rs = make_rsrc(first ? nd : src, g.n * 8u);
+    float r[kP2Rows], v[kP2Rows];
+#pragma unroll
+    for (int j = 0; j < kP2Rows; ++j)
+        r[j] = __uint_as_float(
+            __builtin_amdgcn_raw_buffer_load_b32(rn, (q0 + j * w) * 8 + int(comp) * 4, 0, 0));
+#pragma unroll
+    for (int j = 0; j < kP2Rows; ++j)
+        v[j] = __uint_as_float(
+            __builtin_amdgcn_raw_buffer_load_b32(rs, (q0 + j * w) * 8 + int(comp) * 4, 0, 0));
+    if (first) {
+#pragma unroll
+        for (int j = 0; j < kP2Rows; ++j) v[j] = v[j] * inv_d2;
+    }
+    bool in[kP2Rows];
+#pragma unroll
+    for (int j = 0; j < kP2Rows; ++j) in[j] = uint32_t(q0 + j * w) < uint32_t(n);
+    for (int s = 0; s < sweeps; ++s) {
+        edge[s & 1][wv + 1][0][lane] = v[0];
+        edge[s & 1][wv + 1][1][lane] = v[kP2Rows - 1];
+        __syncthreads();
+        const float up = edge[s & 1][wv][1][lane], down = edge[s & 1][wv + 2][0][lane];
+        float o[kP2Rows];
+#pragma unroll
+        for (int j = 0; j < kP2Rows; ++j) {
+            float x = r[j] - wave_prev(v[j]);
+            x = x - wave_next(v[j]);
+            x = x - (j > 0 ? v[j - 1] : up);
+            x = x - (j < kP2Rows - 1 ? v[j + 1] : down);
+            x = x * inv_d2;
+            o[j] = in[j] ? x : 0.0f;
+        }
+#pragma unroll
+        for (int j = 0; j < kP2Rows; ++j) v[j] = o[j];
+    }
+    if (lane < kP2Halo || lane >= kP2Side - kP2Halo || x0 + lane >= w) return;
+#pragma unroll
+    for (int j = 0; j < kP2Rows; ++j) {
+        const int row = wv * kP2Rows + j;
+        if (row >= kP2Halo && row < kP2Side - kP2Halo && y0 + row < g.h)
+            dst[2 * size_t(q0 + j * w) + comp] = v[j];
     }
 }
 
@@ -397,78 +524,6 @@ __global__ __launch_bounds__(kThreads2) void poisson2d_kernel(const float* __res
     st2(dst, p, v);
 }
 
-// K Jacobi sweeps in one launch over a flat-index segment [a, a + L) of the
-// field.  The stencil reaches p +- 1 and p +- w, so sweep s (1..K) is
-// evaluated on [a - (K-s)w, a + L + (K-s)w) from sweep s-1's values one w
-// wider on each side; the input solve (sweep 0) covers [a - Kw, a + L + Kw).
-// Two LDS buffers of L + 2Kw values alternate.  Positions outside the array
-// hold +0.0: subtracting +0.0 leaves a value unchanged bit for bit
-// (x - (+0) == x, -0 included), so every neighbour is subtracted, in the
-// reference's order, and the dropped ones change nothing.  `first`: the
-// input solve is nd * -1/4 (the initial solve).  Dynamic LDS:
-// 2 (L + 2Kw) float2.
-template <int K>
-__global__ __launch_bounds__(kThreads2) void poisson2d_xk_kernel(const float* __restrict__ nd,
-                                                                 const float* __restrict__ src,
-                                                                 uint32_t n, uint32_t w, uint32_t L,
-                                                                 int first, float* __restrict__ dst)
-{
-    extern __shared__ float2 sm2[];
-    constexpr float inv_d2 = -0.5f / 2.0f;
-    const int64_t a = int64_t(blockIdx.x) * int64_t(L);
-    const int64_t W = int64_t(w), span = int64_t(L) + 2 * K * W;
-    float2* buf[2] = {sm2, sm2 + span};
-    const uint32_t t = threadIdx.y * kBX + threadIdx.x;
-    {
-        const int64_t lo = a - K * W;
-        for (int64_t i = t; i < span; i += kThreads2) {
-            const int64_t q = lo + i;
-            float2 v = make_float2(0.0f, 0.0f);
-            if (q >= 0 && q < int64_t(n)) {
-                if (first) {
-                    v = ld2(nd, uint32_t(q));
-                    v.x *= inv_d2;
-                    v.y *= inv_d2;
-                } else {
-                    v = ld2(src, uint32_t(q));
-                }
-            }
-            buf[0][i] = v;
-        }
-    }
-#pragma unroll
-    for (int s = 1; s <= K; ++s) {
-        __syncthreads();
-        const float2* in = buf[(s - 1) & 1];
-        float2* out = buf[s & 1];
-        const int64_t lo = a - (K - s) * W, len = int64_t(L) + 2 * (K - s) * W;
-        for (int64_t i = t; i < len; i += kThreads2) {
-            const int64_t q = lo + i;
-            if (s == K && q >= int64_t(n)) break;
-            float2 v = make_float2(0.0f, 0.0f);
-            if (q >= 0 && q < int64_t(n)) {
-                const int64_t k = i + W;  // in's index of q
-                v = ld2(nd, uint32_t(q));
-                const float2 a1 = in[k - 1], a2 = in[k + 1], a3 = in[k - W], a4 = in[k + W];
-                v.x -= a1.x;
-                v.y -= a1.y;
-                v.x -= a2.x;
-                v.y -= a2.y;
-                v.x -= a3.x;
-                v.y -= a3.y;
-                v.x -= a4.x;
-                v.y -= a4.y;
-                v.x *= inv_d2;
-                v.y *= inv_d2;
-            }
-            if (s == K)
-                st2(dst, uint32_t(q), v);
-            else
-                out[i] = v;
-        }
-    }
-}
-
 // cdm_max_displacement_length: the largest float(sqrt(x*x + y*y)) as float
 // bits in *out (lengths are >= 0, so their bit patterns order as uints).
 __global__ __launch_bounds__(kThreads2) void maxlen2_kernel(const float* __restrict__ d, Geo2 g,
@@ -486,49 +541,6 @@ __global__ __launch_bounds__(kThreads2) void maxlen2_kernel(const float* __restr
     }
     len = wave_max_f32(len);
     if ((threadIdx.x & 63u) == 0) atomicMax(out, __float_as_uint(len));
-}
-
-// new_d *= k, then accumulate_displacement(cur, new_d): with the mapping
-// m(x) = cur(x) + x, new(x) = m(x + new(x)) - x by bilinear interpolation;
-// where the scaled new(x) is 0 or the sample is outside, new(x) = cur(x).
-// Out of place: the smoothing after it reads the neighbours of new.
-__global__ __launch_bounds__(kThreads2) void acc2_kernel(const float* __restrict__ cur,
-                                                         const float* __restrict__ nd, float k,
-                                                         Geo2 g, float* __restrict__ out)
-{
-    const Pix q = this_pixel(g);
-    if (!q.ok) return;
-    float2 d = ld2(nd, q.p);
-    d.x *= k;
-    d.y *= k;
-    if (d.x != 0.0f || d.y != 0.0f) {
-        const float px = d.x + float(q.x), py = d.y + float(q.y);
-        Bil b;
-        if (locate2(g, px, py, b)) {
-            float2 r;
-#pragma unroll
-            for (int kk = 0; kk < 4; ++kk) {
-                const uint32_t t = tap2(g, b.i0, kk);
-                float2 m = ld2(cur, t);
-                m.x = m.x + float(b.ix + (kk & 1));
-                m.y = m.y + float(b.iy + ((kk & 2) ? 1 : 0));
-                if (kk == 0) {
-                    r.x = m.x * b.w[0];
-                    r.y = m.y * b.w[0];
-                } else {
-                    m.x *= b.w[kk];
-                    m.y *= b.w[kk];
-                    r.x += m.x;
-                    r.y += m.y;
-                }
-            }
-            r.x = r.x - float(q.x);
-            r.y = r.y - float(q.y);
-            st2(out, q.p, r);
-            return;
-        }
-    }
-    st2(out, q.p, ld2(cur, q.p));
 }
 
 // cdm_smooth: out = a*(1-s) + (s/4)*(a[+1] + a[-1] + a[+w] + a[-w]) over
@@ -570,6 +582,119 @@ __global__ __launch_bounds__(kThreads2) void smooth2_kernel(const float* __restr
     st2(out, p, r);
 }
 
+// The accumulated displacement at pixel p = (x, y): with new_d scaled by k and
+// the mapping m(x) = cur(x) + x, new(x) = m(x + new(x)) - x by bilinear
+// interpolation; where the scaled new(x) is 0 or the sample is outside,
+// new(x) = cur(x).
+__device__ inline float2 accumulated2(const float* __restrict__ cur, const float* __restrict__ nd, float k,
+                                      const Geo2& g, uint32_t p, int x, int y)
+{
+    float2 d = ld2(nd, p);
+    d.x *= k;
+    d.y *= k;
+    Bil b;
+    if ((d.x != 0.0f || d.y != 0.0f) && locate2(g, d.x + float(x), d.y + float(y), b)) {
+        float2 r = make_float2(0.0f, 0.0f);
+#pragma unroll
+        for (int kk = 0; kk < 4; ++kk) {
+            float2 m = ld2(cur, tap2(g, b.i0, kk));
+            m.x = m.x + float(b.ix + (kk & 1));
+            m.y = m.y + float(b.iy + ((kk & 2) ? 1 : 0));
+            m.x *= b.w[kk];
+            m.y *= b.w[kk];
+            r.x = kk ? r.x + m.x : m.x;
+            r.y = kk ? r.y + m.y : m.y;
+        }
+        return make_float2(r.x - float(x), r.y - float(y));
+    }
+    return ld2(cur, p);
+}
+
+// compose_displacement: Is(x + d(x)) at pixel p; an exact copy where d(x) == 0,
+// 0 where the sample is outside.
+__device__ inline uint8_t composed2(const uint8_t* __restrict__ Is, const Geo2& g, int x, int y, uint32_t p,
+                                    float2 v)
+{
+    if (v.x == 0.0f && v.y == 0.0f) return Is[p];
+    float px = float(x), py = float(y);
+    px += v.x;
+    py += v.y;
+    Bil b;
+    return locate2(g, px, py, b) ? bil_u8(Is, g, b) : uint8_t(0);
+}
+
+// new_d *= k, then accumulate_displacement(cur, new_d), out of place.
+__global__ __launch_bounds__(kThreads2) void acc2_kernel(const float* __restrict__ cur,
+                                                         const float* __restrict__ nd, float k,
+                                                         Geo2 g, float* __restrict__ out)
+{
+    const Pix q = this_pixel(g);
+    if (q.ok) st2(out, q.p, accumulated2(cur, nd, k, g, q.p, q.x, q.y));
+}
+
+__global__ __launch_bounds__(kThreads2) void compose2_kernel(const uint8_t* __restrict__ Is,
+                                                             Geo2 g, const float* __restrict__ d,
+                                                             uint8_t* __restrict__ Js)
+{
+    const Pix q = this_pixel(g);
+    if (q.ok) Js[q.p] = composed2(Is, g, q.x, q.y, q.p, ld2(d, q.p));
+}
+
+// acc2 then smooth2 (with weights w_4, w_1), and compose2 of Is by the result
+// into Js where Js is given, in one pass: a block evaluates acc on its
+// 16 x 16 outputs and the four edges around them, keeps it in LDS and smooths
+// behind one barrier.  A cell past the end of its row is the next row's first
+// pixel, as smooth2's flat-index neighbours are; a position outside [0, n)
+// holds +0.0, which adds nothing to the neighbour sum (it starts at +0.0 and
+// is never -0.0).  One launch of 4.5 us for three of 2.3 to 2.9.
+constexpr int kU2 = 16;
+
+__global__ __launch_bounds__(kThreads2) void update2_kernel(const float* __restrict__ cur,
+                                                            const float* __restrict__ nd, float k,
+                                                            float w_4, float w_1, Geo2 g,
+                                                            float* __restrict__ out,
+                                                            const uint8_t* __restrict__ Is,
+                                                            uint8_t* __restrict__ Js)
+{
+    __shared__ float2 A[kU2 + 2][kU2 + 2];
+    const int t = int(threadIdx.y) * kBX + int(threadIdx.x);
+    const int x0 = int(blockIdx.x) * kU2, y0 = int(blockIdx.y) * kU2;
+    auto fill = [&](int i, int j) {
+        int x = x0 + i, y = y0 + j;
+        // no output needs a cell more than one past the image
+        bool ok = x <= g.w && y <= g.h;
+        y = x < 0 ? y - 1 : x >= g.w ? y + 1 : y;
+        x = x < 0 ? x + g.w : x >= g.w ? x - g.w : x;
+        ok = ok && y >= 0 && y < g.h;
+        const uint32_t p = ok ? uint32_t(y) * uint32_t(g.w) + uint32_t(x) : 0u;
+        A[j + 1][i + 1] = ok ? accumulated2(cur, nd, k, g, p, x, y) : make_float2(0.0f, 0.0f);
+    };
+    fill(t % kU2, t / kU2);
+    if (t < 4 * kU2) {
+        const int e = t % kU2, side = t / kU2;
+        fill(side == 0 ? -1 : side == 1 ? kU2 : e, side == 2 ? -1 : side == 3 ? kU2 : e);
+    }
+    __syncthreads();
+    const int i = t % kU2, j = t / kU2, x = x0 + i, y = y0 + j;
+    if (x >= g.w || y >= g.h) return;
+    const float2 nb[4] = {A[j + 1][i + 2], A[j + 1][i], A[j + 2][i + 1], A[j][i + 1]};
+    float2 v = make_float2(0.0f, 0.0f);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        v.x += nb[e].x;
+        v.y += nb[e].y;
+    }
+    v.x *= w_4;
+    v.y *= w_4;
+    const float2 c = A[j + 1][i + 1];
+    float2 r;
+    r.x = c.x * w_1 + v.x;
+    r.y = c.y * w_1 + v.y;
+    const uint32_t p = uint32_t(y) * uint32_t(g.w) + uint32_t(x);
+    st2(out, p, r);
+    if (Js) Js[p] = composed2(Is, g, x, y, p, r);
+}
+
 // ---- host ---------------------------------------------------------------------
 
 void check2(const int* dim)
@@ -586,48 +711,60 @@ void launch_compose2(tiplhip_ctx* ctx, const uint8_t* Is, const float* d, const 
     TIPLHIP_CHECK(hipGetLastError());
 }
 
-// The gradient of one modality into nd and its float cost into *cost
-// (device) and, when host_cost is set, into host-visible memory.
-void launch_gradient2(tiplhip_ctx* ctx, const uint8_t* Js, const uint8_t* It, const Geo2& g,
-                      char type, bool accumulate, float* nd, double* part, float* cost,
-                      float* host_cost = nullptr)
+// Block sums a gradient launch writes, at most.
+uint32_t cost_parts2(const Geo2& g)
 {
-    hipLaunchKernelGGL(gradient2_kernel, grid2(g), dim3(kBX, kBY), 0, ctx->stream, Js, It, g, type,
-                       accumulate ? 1 : 0, nd, part);
-    TIPLHIP_CHECK(hipGetLastError());
-    hipLaunchKernelGGL(cost2_final_kernel, dim3(1), dim3(kBX, kBY), 0, ctx->stream, part, blocks2(g),
-                       g.n, cost, host_cost);
+    const dim3 t = tiles2(g);
+    return std::max(blocks2(g), t.x * t.y);
+}
+
+void launch_cost2(tiplhip_ctx* ctx, const CostReduce2& r)
+{
+    hipLaunchKernelGGL(cost2_final_kernel, dim3(1), dim3(kThreads2), 0, ctx->stream, r);
     TIPLHIP_CHECK(hipGetLastError());
 }
 
-// Flat outputs per multi-sweep launch; a launch runs K = 4 sweeps while the
-// two LDS buffers (2 (L + 8w) float2) fit in 64 KB, K = 2 up to twice that
-// width, and one sweep per launch beyond.
-constexpr uint32_t kSweepTile = 1024;
-constexpr uint32_t kMaxX4Width = 384;
-constexpr uint32_t kMaxX2Width = 768;
+// The gradient of one modality into nd; the sum of its block costs into
+// *cost (device) and, when host_cost is set, into host-visible memory is left
+// to the caller.
+CostReduce2 launch_gradient2(tiplhip_ctx* ctx, const uint8_t* Js, const uint8_t* It, const Geo2& g,
+                             char type, bool accumulate, float* nd, double* part, float* cost,
+                             float* host_cost = nullptr)
+{
+    const dim3 grid = type == 'd' ? grid2(g) : tiles2(g);
+    if (type == 'd')
+        hipLaunchKernelGGL(gradient2_d_kernel, grid, dim3(kBX, kBY), 0, ctx->stream, Js, It, g,
+                           accumulate ? 1 : 0, nd, part);
+    else
+        hipLaunchKernelGGL(gradient2_r_kernel, grid, dim3(kBX, kBY), 0, ctx->stream, Js, It, g,
+                           accumulate ? 1 : 0, nd, part);
+    TIPLHIP_CHECK(hipGetLastError());
+    return CostReduce2{part, grid.x * grid.y, g.n, cost, host_cost};
+}
 
-// `sweeps` Jacobi sweeps ping-ponging a/b (several per launch where the
-// tile fits); returns the buffer holding the result.
-float* launch_poisson2(tiplhip_ctx* ctx, const float* nd, float* a, float* b, const Geo2& g, int sweeps)
+// `sweeps` Jacobi sweeps ping-ponging a/b, up to twelve per launch (one where
+// byte offsets would pass 2^31); returns the buffer holding the result.  A
+// gradient's cost, when given, is summed by the first launch.
+float* launch_poisson2(tiplhip_ctx* ctx, const float* nd, float* a, float* b, const Geo2& g, int sweeps,
+                       const CostReduce2& cost = CostReduce2{})
 {
     float* src = a;
     float* dst = a;
-    const uint32_t w = uint32_t(g.w);
-    const dim3 tiles((g.n + kSweepTile - 1) / kSweepTile);
+    // (the grown tiles' byte offsets, up to 76 rows outside the image, in 31 bits)
+    const bool tiled = (size_t(g.n) + 128 * size_t(g.w)) * 8 < (size_t(1) << 31);
+    if (!tiled && cost.part) launch_cost2(ctx, cost);
     int done = 0;
     for (int i = 0; done < sweeps; ++i) {
         dst = (i & 1) ? b : a;
-        if (w <= kMaxX4Width && sweeps - done >= 4) {
-            const size_t lds = sizeof(float2) * 2 * (size_t(kSweepTile) + 8 * size_t(w));
-            hipLaunchKernelGGL(poisson2d_xk_kernel<4>, tiles, dim3(kBX, kBY), lds, ctx->stream, nd, src,
-                               g.n, w, kSweepTile, done == 0 ? 1 : 0, dst);
-            done += 4;
-        } else if (w <= kMaxX2Width && sweeps - done >= 2) {
-            const size_t lds = sizeof(float2) * 2 * (size_t(kSweepTile) + 4 * size_t(w));
-            hipLaunchKernelGGL(poisson2d_xk_kernel<2>, tiles, dim3(kBX, kBY), lds, ctx->stream, nd, src,
-                               g.n, w, kSweepTile, done == 0 ? 1 : 0, dst);
-            done += 2;
+        if (tiled) {
+            const int run = std::min(sweeps - done, kP2Halo);
+            const CostReduce2 c = done == 0 ? cost : CostReduce2{};
+            const uint32_t blocks = 2u * uint32_t((g.w + kP2Core - 1) / kP2Core) *
+                                    uint32_t((g.h + kP2Core - 1) / kP2Core);
+            hipLaunchKernelGGL(poisson2d_tile_kernel, dim3(blocks + (c.part ? 1u : 0u)),
+                               dim3(64 * kP2Waves), 0, ctx->stream, nd, src, g, done == 0 ? 1 : 0, run,
+                               dst, c);
+            done += run;
         } else {
             hipLaunchKernelGGL(poisson2d_kernel, grid2(g), dim3(kBX, kBY), 0, ctx->stream, nd, src, g,
                                done == 0 ? 1 : 0, dst);
@@ -662,6 +799,18 @@ void launch_smooth2(tiplhip_ctx* ctx, const float* a, float smoothing, const Geo
     const float w_4 = smoothing / (2.0f * 2.0f);
     const float w_1 = 1.0f - smoothing;
     hipLaunchKernelGGL(smooth2_kernel, grid2(g), dim3(kBX, kBY), 0, ctx->stream, a, g, w_4, w_1, out);
+    TIPLHIP_CHECK(hipGetLastError());
+}
+
+// acc2, smooth2 with `smoothing` (non-zero) and, where Js is set, compose2.
+void launch_update2(tiplhip_ctx* ctx, const float* cur, const float* nd, float k, float smoothing,
+                    const Geo2& g, float* out, const uint8_t* Is, uint8_t* Js)
+{
+    static_assert(kU2 == kG2, "tiles2 counts the update's blocks too");
+    const float w_4 = smoothing / (2.0f * 2.0f);
+    const float w_1 = 1.0f - smoothing;
+    hipLaunchKernelGGL(update2_kernel, tiles2(g), dim3(kBX, kBY), 0, ctx->stream, cur, nd, k, w_4, w_1, g,
+                       out, Is, Js);
     TIPLHIP_CHECK(hipGetLastError());
 }
 
@@ -719,8 +868,13 @@ bool cdm2_level(Cdm2Run& run, const std::vector<const uint8_t*>& It,
     }
 
     const size_t fb = sizeof(float) * 2 * g.n;
-    DevMem cur(ctx, fb), nd(ctx, fb), acc(ctx, fb), pa(ctx, fb), pb(ctx, fb), Js(ctx, g.n);
-    DevMem part(ctx, sizeof(double) * blocks2(g)), costs(ctx, sizeof(float) * size_t(nmod)),
+    // the running field, the best field so far -- which may be the running
+    // one -- and a spare one rotate through these and `best`
+    DevMem f0(ctx, fb), f1(ctx, fb), nd(ctx, fb), pa(ctx, fb), pb(ctx, fb), Js(ctx, g.n);
+    float* cur = best;
+    float* best_f = best;
+    float* spare[2] = {f0.as<float>(), f1.as<float>()};  // the second free only while best_f == cur
+    DevMem part(ctx, sizeof(double) * cost_parts2(g)), costs(ctx, sizeof(float) * size_t(nmod)),
         word(ctx, sizeof(unsigned int));
     // the cost reductions also store into ctx->h_cdm: if a step throws while
     // one is queued, drain the stream before the slots (and the buffers
@@ -728,7 +882,7 @@ bool cdm2_level(Cdm2Run& run, const std::vector<const uint8_t*>& It,
     auto drain = [ctx] { (void)hipStreamSynchronize(ctx->stream); };
     DrainOnUnwind<decltype(drain)> unwind(drain);
     ctx->h_cdm.reserve(sizeof(float) * 16);
-    copy2(ctx, cur.p, best, fb);
+    bool composed = false;  // Js holds compose_displacement of cur
     float theta = 0.0f;
     std::vector<float> cost;
     float best_cost = std::numeric_limits<float>::max();
@@ -749,13 +903,18 @@ bool cdm2_level(Cdm2Run& run, const std::vector<const uint8_t*>& It,
         uint32_t* slots = ctx->h_cdm.as<uint32_t>();
         std::fill(slots, slots + nmod, kCostPending2);
         float* h_cost = static_cast<float*>(ctx->h_cdm.dev);
+        CostReduce2 reduce;
         for (int i = 0; i < nmod; ++i) {
-            launch_compose2(ctx, Is[size_t(i)], cur.as<float>(), g, Js.as<uint8_t>());
+            // (of a single modality the field update has composed Js)
+            if (!composed) launch_compose2(ctx, Is[size_t(i)], cur, g, Js.as<uint8_t>());
             const char type = run.param.gradient_type[i] == 'd' ? 'd' : 'r';
-            launch_gradient2(ctx, Js.as<uint8_t>(), It[size_t(i)], g, type, i > 0, nd.as<float>(),
-                             part.as<double>(), costs.as<float>() + i, h_cost + i);
+            reduce = launch_gradient2(ctx, Js.as<uint8_t>(), It[size_t(i)], g, type, i > 0, nd.as<float>(),
+                                      part.as<double>(), costs.as<float>() + i, h_cost + i);
+            // the last modality's sum rides on the Poisson launch
+            if (i + 1 < nmod) launch_cost2(ctx, reduce);
         }
-        float* solved = launch_poisson2(ctx, nd.as<float>(), pa.as<float>(), pb.as<float>(), g, 12);
+        composed = false;
+        float* solved = launch_poisson2(ctx, nd.as<float>(), pa.as<float>(), pb.as<float>(), g, 12, reduce);
         wait_for_slots(static_cast<const volatile uint32_t*>(slots), size_t(nmod), kCostPending2,
                        std::chrono::microseconds(kCostSpinUs2),
                        [ctx] { TIPLHIP_CHECK(hipStreamSynchronize(ctx->stream)); });
@@ -768,21 +927,34 @@ bool cdm2_level(Cdm2Run& run, const std::vector<const uint8_t*>& It,
         cost.push_back(sum_cost / float(nmod));
         if (cost.back() < best_cost) {
             best_cost = cost.back();
-            if (index) copy2(ctx, best, cur.p, fb);
+            if (best_f != cur) {
+                spare[1] = best_f;
+                best_f = cur;
+            }
         }
         if (!cdm_improved(cost)) {
             if (cur_smoothing <= run.param.smoothing) break;
-            copy2(ctx, cur.p, best, fb);
+            if (best_f != cur) {
+                spare[1] = cur;
+                cur = best_f;
+            }
             cur_smoothing *= 0.5f;
             cost.clear();
         }
         if (theta == 0.0f) theta = max_length2(ctx, solved, g, word.as<unsigned int>());
         if (theta == 0.0f) break;
         const float k = run.param.speed / theta;
-        launch_acc2(ctx, cur.as<float>(), solved, k, g, acc.as<float>());
         // cdm_smooth(new_d, cur_d, 0) leaves cur_d as it was
-        if (cur_smoothing != 0.0f) launch_smooth2(ctx, acc.as<float>(), cur_smoothing, g, cur.as<float>());
+        if (cur_smoothing != 0.0f) {
+            composed = nmod == 1;
+            launch_update2(ctx, cur, solved, k, cur_smoothing, g, spare[0], Is[0],
+                           composed ? Js.as<uint8_t>() : nullptr);
+            float* next = spare[0];
+            spare[0] = best_f == cur ? spare[1] : cur;
+            cur = next;
+        }
     }
+    if (best_f != best) copy2(ctx, best, best_f, fb);
     return true;
 }
 
@@ -878,11 +1050,11 @@ int tiplhip_cdm2d_gradient(tiplhip_ctx* ctx, const uint8_t* Js, const uint8_t* I
         DeviceGuard dg(ctx->device);
         const Geo2 g = geo2(dim[0], dim[1]);
         DevMem dJ(ctx, g.n), dI(ctx, g.n), dN(ctx, sizeof(float) * 2 * g.n);
-        DevMem part(ctx, sizeof(double) * blocks2(g)), dc(ctx, sizeof(float));
+        DevMem part(ctx, sizeof(double) * cost_parts2(g)), dc(ctx, sizeof(float));
         TIPLHIP_CHECK(hipMemcpyAsync(dJ.p, Js, g.n, hipMemcpyHostToDevice, ctx->stream));
         TIPLHIP_CHECK(hipMemcpyAsync(dI.p, It, g.n, hipMemcpyHostToDevice, ctx->stream));
-        launch_gradient2(ctx, dJ.as<uint8_t>(), dI.as<uint8_t>(), g, type, false, dN.as<float>(),
-                         part.as<double>(), dc.as<float>());
+        launch_cost2(ctx, launch_gradient2(ctx, dJ.as<uint8_t>(), dI.as<uint8_t>(), g, type, false,
+                                           dN.as<float>(), part.as<double>(), dc.as<float>()));
         TIPLHIP_CHECK(hipMemcpyAsync(new_d, dN.p, sizeof(float) * 2 * g.n, hipMemcpyDeviceToHost, ctx->stream));
         float c = 0.0f;
         TIPLHIP_CHECK(hipMemcpyAsync(&c, dc.p, sizeof(float), hipMemcpyDeviceToHost, ctx->stream));
