@@ -2676,8 +2676,7 @@ int tiplhip_cdm(tiplhip_ctx* ctx, const tiplhip_volume* const* It, const tiplhip
         DevMem best(ctx, fb);
         const int rc = cdm_device(ctx, It, Is, n, param, best.as<float>(), terminated, iterations);
         if (rc == TIPLHIP_ERR_FAILED) throw Error(TIPLHIP_ERR_FAILED, "cdm returned false (zero cost)");
-        TIPLHIP_CHECK(hipMemcpyAsync(field, best.p, fb, hipMemcpyDeviceToHost, ctx->stream));
-        TIPLHIP_CHECK(hipStreamSynchronize(ctx->stream));
+        copy_to_host(ctx, field, best.p, fb);
         // As in the reference, a terminated run still returns its best field.
         if (rc == TIPLHIP_ERR_TERMINATED) throw Error(TIPLHIP_ERR_TERMINATED, "terminated by the caller");
     });
@@ -2706,10 +2705,7 @@ int tiplhip_cdm_level_iterations(tiplhip_ctx* ctx, const tiplhip_volume* It,
         DevMem best(ctx, fb);
         zero(ctx, best.p, fb);
         (void)cdm_level(run, vt, vs, dim, best.as<float>(), 1.0f);
-        if (field) {
-            TIPLHIP_CHECK(hipMemcpyAsync(field, best.p, fb, hipMemcpyDeviceToHost, ctx->stream));
-            TIPLHIP_CHECK(hipStreamSynchronize(ctx->stream));
-        }
+        if (field) copy_to_host(ctx, field, best.p, fb);
     });
 }
 

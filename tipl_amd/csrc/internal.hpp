@@ -142,6 +142,8 @@ struct tiplhip_ctx {
     tiplhip::PinnedBuffer h_out;
     tiplhip::PinnedBuffer h_costs;   // coherent: cost kernels write the K costs here directly
     tiplhip::PinnedBuffer h_cdm;     // coherent: a CDM iteration's per-modality costs
+    tiplhip::PinnedBuffer h_stage;   // staging ring of large copies to the host
+    std::vector<hipEvent_t> stage_events;  // one per slot of it
     // d_hist once queued work ends: [0, hist_dirty) holds counts no entropy
     // pass consumed, [hist_dirty, hist_zero) is zero
     size_t hist_dirty = 0, hist_zero = 0;
@@ -222,6 +224,8 @@ int cdm_device(tiplhip_ctx* ctx, const tiplhip_volume* const* It, const tiplhip_
 // Copies `bytes` of device memory to host memory through ctx's pinned
 // staging buffer and waits for it (ctx's stream is synchronised).
 void read_back(tiplhip_ctx* ctx, const void* dev, void* host, size_t bytes);
+// Copies a result into the caller's memory and waits for it; ctx->mu held.
+void copy_to_host(tiplhip_ctx* ctx, void* host, const void* dev, size_t bytes);
 
 // A second context on ctx's device (own stream), created on first use and
 // destroyed with ctx: the reverse CDM of a registration runs on it.

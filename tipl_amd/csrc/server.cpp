@@ -54,7 +54,8 @@ struct Joiner {
 
 void to_host(tiplhip_ctx* ctx, void* dst, const void* src, size_t bytes)
 {
-    TIPLHIP_CHECK(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, ctx->stream));
+    std::lock_guard<std::recursive_mutex> lk(ctx->mu);
+    copy_to_host(ctx, dst, src, bytes);
 }
 
 // One registration on ctx; costs go through `eval`.
