@@ -236,16 +236,10 @@ __global__ __launch_bounds__(256) void ztab_kernel(const float* __restrict__ Ts,
 // crop for an integer-shift transform (numerical/resampling.hpp:1244-1262).
 // ---------------------------------------------------------------------------
 template <bool ZT>
-__global__ __launch_bounds__(256) void corr_sums_kernel(const Segment* __restrict__ segs,
-                                                        uint32_t nseg, uint32_t total_blocks,
-                                                        const float* __restrict__ Ts,
-                                                        const int4* __restrict__ crop,
-                                                        const float4* __restrict__ ztab,
-                                                        uint32_t zstride,
-                                                        unsigned long long* __restrict__ sums)
+__device__ __forceinline__ void corr_sums_body(const Segment& sg, uint32_t L, const float* Ts,
+                                               const int4* crop, const float4* __restrict__ ztab,
+                                               uint32_t zstride, unsigned long long* __restrict__ sums)
 {
-    const uint32_t L = xcd_remap(blockIdx.x, total_blocks);
-    const Segment& sg = segs[find_segment(segs, nseg, L, ByBlock{})];
     const BatchGeo g = sg.g;
     const uint32_t local = L - sg.block_begin;
     const uint32_t cand = sg.cand_begin + local % g.K;
@@ -337,21 +331,65 @@ __global__ __launch_bounds__(256) void corr_sums_kernel(const Segment* __restric
     }
 }
 
+template <bool ZT>
+__global__ __launch_bounds__(256) void corr_sums_kernel(const Segment* __restrict__ segs,
+                                                        uint32_t nseg, uint32_t total_blocks,
+                                                        const float* __restrict__ Ts,
+                                                        const int4* __restrict__ crop,
+                                                        const float4* __restrict__ ztab,
+                                                        uint32_t zstride,
+                                                        unsigned long long* __restrict__ sums)
+{
+    const uint32_t L = xcd_remap(blockIdx.x, total_blocks);
+    corr_sums_body<ZT>(segs[find_segment(segs, nseg, L, ByBlock{})], L, Ts, crop, ztab, zstride, sums);
+}
+
+// The inputs of a launch over one pair and few candidates, which travel as a
+// kernel argument: no upload, and no wait for one, before the launch.
+constexpr uint32_t kArgK = 56;
+struct ArgBatch {
+    Segment seg;
+    float T[12 * kArgK];
+};
+struct ArgCrops {
+    int4 crop[kArgK];
+};
+static_assert(sizeof(ArgBatch) + sizeof(ArgCrops) + 64 <= 4096, "kernel arguments end at 4 KB");
+
+__global__ __launch_bounds__(256) void corr_sums_arg_kernel(const ArgBatch in, const ArgCrops crops,
+                                                            uint32_t total_blocks,
+                                                            unsigned long long* __restrict__ sums)
+{
+    corr_sums_body<false>(in.seg, xcd_remap(blockIdx.x, total_blocks), in.T, crops.crop, nullptr, 0u, sums);
+}
+
+// What the finalizer needs of a candidate's `from` volume.
+struct FromSums {
+    long long sx, sxx;
+    double n;
+};
+
 // tipl::correlation from exact sums (numerical/statistics.hpp:555-586,
 // 407-443) in FP64, then `float c; 1.0f - c*c` (reg/linear.hpp:34-35).
-__global__ void corr_finalize_kernel(const Segment* __restrict__ segs, uint32_t nseg,
-                                     const unsigned long long* __restrict__ sums, int K,
+// segs null: one pair, whose sums are `one`.  Leaves the sums it has read
+// zero for the next launch, which then needs no clearing pass.
+__global__ void corr_finalize_kernel(const Segment* __restrict__ segs, uint32_t nseg, FromSums one,
+                                     unsigned long long* __restrict__ sums, int K,
                                      double* __restrict__ costs, double* __restrict__ host_costs,
                                      long long* __restrict__ sums_out)
 {
     int k = blockIdx.x * blockDim.x + threadIdx.x;
     if (k >= K) return;
-    const Segment& sg = segs[find_segment(segs, nseg, uint32_t(k), ByCandidate{})];
-    const long long sx = sg.sx, sxx = sg.sxx;
-    const double n = sg.n;
+    if (segs) {
+        const Segment& sg = segs[find_segment(segs, nseg, uint32_t(k), ByCandidate{})];
+        one = FromSums{sg.sx, sg.sxx, sg.n};
+    }
+    const long long sx = one.sx, sxx = one.sxx;
+    const double n = one.n;
     long long sy = (long long)sums[k * 4 + 0];
     long long syy = (long long)sums[k * 4 + 1];
     long long sxy = (long long)sums[k * 4 + 2];
+    for (int i = 0; i < 3; ++i) sums[k * 4 + i] = 0ull;
     double mean_x = double(sx) / n;
     double mean_y = double(sy) / n;
     double var_x = double(sxx) / n - mean_x * mean_x;
@@ -413,10 +451,9 @@ struct MiTraits<64> {
 };
 
 template <int BINS, bool ZT>
-__global__ __launch_bounds__(MiTraits<BINS>::kThreads) void mi_hist_kernel(
-    const Segment* __restrict__ segs, uint32_t nseg, uint32_t total_blocks,
-    const float* __restrict__ Ts, const float4* __restrict__ ztab, uint32_t zstride,
-    int* __restrict__ hist, uint32_t* __restrict__ to_hist)
+__device__ __forceinline__ void mi_hist_body(const Segment& sg, uint32_t L, const float* Ts,
+                                             const float4* __restrict__ ztab, uint32_t zstride,
+                                             int* __restrict__ hist, uint32_t* __restrict__ to_hist)
 {
     using Tr = MiTraits<BINS>;
     // cleared 16 bytes a store: the 256-bin kernel 0.8-1.4% faster at
@@ -427,8 +464,6 @@ __global__ __launch_bounds__(MiTraits<BINS>::kThreads) void mi_hist_kernel(
         reinterpret_cast<uint4*>(lds)[i] = make_uint4(0u, 0u, 0u, 0u);
     __syncthreads();
 
-    const uint32_t L = xcd_remap(blockIdx.x, total_blocks);
-    const Segment& sg = segs[find_segment(segs, nseg, L, ByBlock{})];
     const BatchGeo g = sg.g;
     const uint32_t local = L - sg.block_begin;
     const uint32_t cand = sg.cand_begin + local % g.K;
@@ -550,6 +585,23 @@ __global__ __launch_bounds__(MiTraits<BINS>::kThreads) void mi_hist_kernel(
     }
 }
 
+template <int BINS, bool ZT>
+__global__ __launch_bounds__(MiTraits<BINS>::kThreads) void mi_hist_kernel(
+    const Segment* __restrict__ segs, uint32_t nseg, uint32_t total_blocks,
+    const float* __restrict__ Ts, const float4* __restrict__ ztab, uint32_t zstride,
+    int* __restrict__ hist, uint32_t* __restrict__ to_hist)
+{
+    const uint32_t L = xcd_remap(blockIdx.x, total_blocks);
+    mi_hist_body<BINS, ZT>(segs[find_segment(segs, nseg, L, ByBlock{})], L, Ts, ztab, zstride, hist, to_hist);
+}
+
+template <int BINS>
+__global__ __launch_bounds__(MiTraits<BINS>::kThreads) void mi_hist_arg_kernel(
+    const ArgBatch in, uint32_t total_blocks, int* __restrict__ hist, uint32_t* __restrict__ to_hist)
+{
+    mi_hist_body<BINS, false>(in.seg, xcd_remap(blockIdx.x, total_blocks), in.T, nullptr, 0u, hist, to_hist);
+}
+
 // get_mutual_info_mean (reg/linear.hpp:87-104): the sum of
 // mu*log(mu/from_h[row]/to_h[col]) in FP64 over non-zero bins, divided by
 // float(BINS*BINS) and negated (reg/linear.hpp:201).  to_h comes from the
@@ -568,15 +620,16 @@ constexpr int entropy_slices() { return BINS * BINS / kEntropySlice; }
 
 template <int BINS>
 __global__ __launch_bounds__(kEntropyThreads) void mi_entropy_kernel(
-    const Segment* __restrict__ segs, uint32_t nseg, int* hist, uint32_t* to_hist,
-    double* __restrict__ part, double* __restrict__ costs, double* __restrict__ host_costs)
+    const Segment* __restrict__ segs, uint32_t nseg, const uint32_t* __restrict__ one_from_hist,
+    int* hist, uint32_t* to_hist, uint32_t* tickets, double* __restrict__ part,
+    double* __restrict__ costs, double* __restrict__ host_costs)
 {
     constexpr int G = entropy_slices<BINS>();
     constexpr int kVec = kEntropySlice / 4 / kEntropyThreads;
     constexpr int kWaves = kEntropyThreads / 64;
     const uint32_t cand = blockIdx.x / G, slice = blockIdx.x % G;
     const uint32_t* __restrict__ from_hist =
-        segs[find_segment(segs, nseg, cand, ByCandidate{})].from_hist;
+        segs ? segs[find_segment(segs, nseg, cand, ByCandidate{})].from_hist : one_from_hist;
     __shared__ uint32_t to_h[BINS];
     __shared__ double wpart[kWaves];
     // each wave's non-zero bins, packed in (slot, lane) order: at most 64 x 4 x kVec a wave
@@ -640,10 +693,35 @@ __global__ __launch_bounds__(kEntropyThreads) void mi_entropy_kernel(
             part[blockIdx.x] = t[0];
         }
     }
-    if constexpr (G == 1) {
+    bool clear = G == 1;
+    if constexpr (G > 1) {
+        // With tickets (the slice sums go to the host, and no combining launch
+        // follows) the candidate's last slice clears its row: every slice has
+        // read the row into LDS, behind the barriers above, before its ticket.
+        if (tickets) {
+            __shared__ uint32_t ticket;
+            if (threadIdx.x == 0) ticket = atomicAdd(&tickets[cand], 1u);
+            __syncthreads();
+            clear = ticket == uint32_t(G - 1);
+            if (clear && threadIdx.x == 0) tickets[cand] = 0u;
+        }
+    }
+    if (clear) {
         uint4* row4 = reinterpret_cast<uint4*>(to_hist + size_t(cand) * BINS);
         for (int i = int(threadIdx.x); i < BINS / 4; i += kEntropyThreads) row4[i] = make_uint4(0u, 0u, 0u, 0u);
     }
+}
+
+// The cost from a candidate's slice sums: a fixed tree, the same on the host.
+template <int BINS>
+__host__ __device__ inline double combine_slices(const double* part)
+{
+    constexpr int G = entropy_slices<BINS>();
+    double t[G];
+    for (int i = 0; i < G; ++i) t[i] = part[i];
+    for (int w = G / 2; w > 0; w /= 2)
+        for (int i = 0; i < w; ++i) t[i] = t[2 * i] + t[2 * i + 1];
+    return -(t[0] / double(float(BINS * BINS)));
 }
 
 // Also clears the block's candidates' to_hist rows (every slice has read
@@ -657,14 +735,7 @@ __global__ __launch_bounds__(256) void mi_entropy_final_kernel(const double* __r
     constexpr int G = entropy_slices<BINS>();
     const uint32_t first = blockIdx.x * 256u, cand = first + threadIdx.x;
     if (cand < K) {
-        double t[G];
-#pragma unroll
-        for (int i = 0; i < G; ++i) t[i] = part[size_t(cand) * G + i];
-#pragma unroll
-        for (int w = G / 2; w > 0; w /= 2)
-#pragma unroll
-            for (int i = 0; i < w; ++i) t[i] = t[2 * i] + t[2 * i + 1];
-        const double c = -(t[0] / double(float(BINS * BINS)));
+        const double c = combine_slices<BINS>(part + size_t(cand) * G);
         costs[cand] = c;
         if (host_costs) host_costs[cand] = c;
     }
@@ -800,6 +871,8 @@ struct Staged {
     uint32_t zstride = 0;   // the largest `from` depth: rows of the z-product table
     size_t bytes = 0;       // staged bytes (transforms, crop flags, segment table)
     bool grew = false;      // the device staging buffer was reallocated
+    const Segment* host_segs = nullptr;  // the staged inputs in host memory (until the next staging)
+    const float* host_T = nullptr;
 };
 
 // Launches of at least this many samples get a z-product table: its build
@@ -917,6 +990,8 @@ Staged stage_jobs(tiplhip_ctx* ctx, const std::vector<PairJob>& jobs, const floa
     if (crop) std::memcpy(h + tb, crop, cb);
     std::memcpy(h + tb + cb, segs.data(), sb);
     if (upload) TIPLHIP_CHECK(hipMemcpyAsync(ctx->d_T.p, h, st.bytes, hipMemcpyHostToDevice, ctx->stream));
+    st.host_T = hT;
+    st.host_segs = reinterpret_cast<const Segment*>(h + tb + cb);
     char* d = static_cast<char*>(ctx->d_T.p);
     st.T = reinterpret_cast<const float*>(d);
     st.crop = crop ? reinterpret_cast<const int4*>(d + tb) : nullptr;
@@ -943,11 +1018,36 @@ const float4* stage_ztab(tiplhip_ctx* ctx, const Staged& st)
     return ctx->d_ztab.as<float4>();
 }
 
+// The correlation kernel accumulates into zeroed sums, and the finalizer
+// leaves those it has read zero again: clearing passes run only over sums
+// never cleared since the buffer was allocated and after a launch whose sums
+// were not finalized (the autotuner).
+// Returns true when the buffer was reallocated.
+bool reserve_sums(tiplhip_ctx* ctx, size_t K)
+{
+    const size_t had = ctx->d_sums.bytes;
+    ctx->d_sums.reserve(sizeof(unsigned long long) * 4 * K);
+    if (ctx->d_sums.bytes == had) return false;
+    ctx->sums_dirty = ctx->sums_zero = 0;
+    return true;
+}
+
+// Queues the clearing passes that make the first K candidates' sums zero.
+void make_sums_clean(tiplhip_ctx* ctx, size_t K)
+{
+    unsigned long long* base = ctx->d_sums.as<unsigned long long>();
+    if (ctx->sums_dirty > 0) zero_u64(ctx, base, 4 * ctx->sums_dirty);
+    ctx->sums_dirty = 0;
+    if (ctx->sums_zero < K) zero_u64(ctx, base + 4 * ctx->sums_zero, 4 * (K - ctx->sums_zero));
+    ctx->sums_zero = std::max(ctx->sums_zero, K);
+}
+
 // Correlation sums Sy, Syy, Sxy of every staged candidate into ctx->d_sums (K x 4 u64).
 void launch_corr_sums(tiplhip_ctx* ctx, const Staged& st)
 {
-    ctx->d_sums.reserve(sizeof(unsigned long long) * 4 * size_t(st.K));
-    zero_u64(ctx, ctx->d_sums.p, 4 * size_t(st.K));
+    reserve_sums(ctx, st.K);
+    make_sums_clean(ctx, st.K);
+    ctx->sums_dirty = st.K;
     const float4* zt = stage_ztab(ctx, st);
     // per-lane uint32 sums of squares stay below 2^32 for < 65536 voxels a lane
     timing_begin(ctx);
@@ -968,9 +1068,10 @@ void launch_corr_finalize(tiplhip_ctx* ctx, const Staged& st, long long* sums_ou
 {
     ctx->d_costs.reserve(sizeof(double) * size_t(st.K));
     hipLaunchKernelGGL(corr_finalize_kernel, dim3((st.K + 63) / 64), dim3(64), 0, ctx->stream,
-                       st.segs, st.nseg, ctx->d_sums.as<unsigned long long>(), int(st.K),
+                       st.segs, st.nseg, FromSums{}, ctx->d_sums.as<unsigned long long>(), int(st.K),
                        ctx->d_costs.as<double>(), host_costs, sums_out);
     TIPLHIP_CHECK(hipGetLastError());
+    ctx->sums_dirty = 0;
 }
 
 // Joint histograms of every staged candidate into ctx->d_hist.
@@ -980,9 +1081,16 @@ uint32_t* to_hist_of(tiplhip_ctx* ctx, const Staged& st, int bins)
     return reinterpret_cast<uint32_t*>(ctx->d_hist.as<int>() + size_t(bins) * bins * size_t(st.K));
 }
 
+// ... then (arg_cost) a ticket per candidate.
 size_t hist_bytes(const Staged& st, int bins)
 {
-    return sizeof(int) * (size_t(bins) * bins + size_t(bins)) * size_t(st.K);
+    return sizeof(int) * (size_t(bins) * bins + size_t(bins)) * size_t(st.K) +
+           ((sizeof(uint32_t) * size_t(st.K) + 15) & ~size_t(15));
+}
+
+uint32_t* tickets_of(tiplhip_ctx* ctx, const Staged& st, int bins)
+{
+    return to_hist_of(ctx, st, bins) + size_t(bins) * size_t(st.K);
 }
 
 // The histogram kernel accumulates into a zeroed buffer.  The entropy
@@ -1045,8 +1153,8 @@ void launch_mi_entropy_t(tiplhip_ctx* ctx, const Staged& st, double* host_costs)
     double* costs = ctx->d_costs.as<double>();
     double* part = costs + st.K;
     hipLaunchKernelGGL(mi_entropy_kernel<BINS>, dim3(st.K * uint32_t(G)), dim3(kEntropyThreads), 0,
-                       ctx->stream, st.segs, st.nseg, ctx->d_hist.as<int>(), to_hist_of(ctx, st, BINS),
-                       part, costs, host_costs);
+                       ctx->stream, st.segs, st.nseg, nullptr, ctx->d_hist.as<int>(),
+                       to_hist_of(ctx, st, BINS), nullptr, part, costs, host_costs);
     TIPLHIP_CHECK(hipGetLastError());
     if constexpr (G > 1) {
         hipLaunchKernelGGL(mi_entropy_final_kernel<BINS>, dim3((st.K + 255) / 256), dim3(256), 0,
@@ -1081,6 +1189,62 @@ void launch_resample(tiplhip_ctx* ctx, const tiplhip_volume* src, const int* out
                        uint32_t(src->n), make_geo(src->dim), out_dim[0], out_dim[1], out_dim[2], ta,
                        crop, out);
     TIPLHIP_CHECK(hipGetLastError());
+}
+
+// The cost launches of one pair and at most kArgK candidates: the inputs are
+// kernel arguments, and a 256-bin launch's slice sums go to host_out, K x
+// slices of them, for the host to combine.  Two launches, where the staged
+// path has an upload and three (correlation: an upload, a clear and two).
+// Such a launch is latency: 33.5 -> 29.4 us a call for ten 48x48x48 candidates
+// at 256 bins, 50.2 -> 45.6 for twelve of 91x109x91.  (kArgK is what 4 KB of
+// arguments hold.)
+void arg_cost(tiplhip_ctx* ctx, const Staged& st, const int4* crop, int cost, int bins, double* host_out)
+{
+    ArgBatch in;
+    in.seg = st.host_segs[0];
+    std::memcpy(in.T, st.host_T, sizeof(float) * 12 * st.K);
+    if (cost == TIPLHIP_COST_CORR) {
+        ArgCrops crops;
+        std::memcpy(crops.crop, crop, sizeof(int4) * st.K);
+        make_sums_clean(ctx, st.K);
+        ctx->sums_dirty = st.K;
+        unsigned long long* sums = ctx->d_sums.as<unsigned long long>();
+        timing_begin(ctx);
+        hipLaunchKernelGGL(corr_sums_arg_kernel, dim3(st.total_blocks), dim3(256), 0, ctx->stream, in, crops,
+                           st.total_blocks, sums);
+        TIPLHIP_CHECK(hipGetLastError());
+        timing_end(ctx);
+        hipLaunchKernelGGL(corr_finalize_kernel, dim3((st.K + 63) / 64), dim3(64), 0, ctx->stream, nullptr,
+                           0u, FromSums{in.seg.sx, in.seg.sxx, in.seg.n}, sums, int(st.K),
+                           ctx->d_costs.as<double>(), host_out, nullptr);
+        TIPLHIP_CHECK(hipGetLastError());
+        ctx->sums_dirty = 0;
+        return;
+    }
+    const size_t hb = hist_bytes(st, bins);
+    make_hist_clean(ctx, hb);
+    ctx->hist_dirty = hb;
+    int* h = ctx->d_hist.as<int>();
+    uint32_t* th = to_hist_of(ctx, st, bins);
+    double* costs = ctx->d_costs.as<double>();
+    timing_begin(ctx);
+    if (bins == 256)
+        hipLaunchKernelGGL(mi_hist_arg_kernel<256>, dim3(st.total_blocks), dim3(1024), 0, ctx->stream, in,
+                           st.total_blocks, h, th);
+    else
+        hipLaunchKernelGGL(mi_hist_arg_kernel<64>, dim3(st.total_blocks), dim3(256), 0, ctx->stream, in,
+                           st.total_blocks, h, th);
+    TIPLHIP_CHECK(hipGetLastError());
+    timing_end(ctx);
+    if (bins == 256)
+        hipLaunchKernelGGL(mi_entropy_kernel<256>, dim3(st.K * uint32_t(entropy_slices<256>())),
+                           dim3(kEntropyThreads), 0, ctx->stream, nullptr, 0u, in.seg.from_hist, h, th,
+                           tickets_of(ctx, st, bins), host_out, costs, nullptr);
+    else
+        hipLaunchKernelGGL(mi_entropy_kernel<64>, dim3(st.K), dim3(kEntropyThreads), 0, ctx->stream, nullptr,
+                           0u, in.seg.from_hist, h, th, nullptr, nullptr, costs, host_out);
+    TIPLHIP_CHECK(hipGetLastError());
+    ctx->hist_dirty = 0;
 }
 
 // Costs of every candidate of every job in one launch (plus one finishing
@@ -1141,14 +1305,18 @@ void cost_jobs(tiplhip_ctx* ctx, std::vector<PairJob> jobs, const float* T, int 
         grow(ctx->d_costs, sizeof(double) * K * size_t(1 + (bins == 256 ? entropy_slices<256>()
                                                                         : entropy_slices<64>())));
     } else {
-        grow(ctx->d_sums, sizeof(unsigned long long) * 4 * K);
+        grew = reserve_sums(ctx, K) || grew;
         grow(ctx->d_costs, sizeof(double) * K);
     }
     if (st.samples >= kZTableSamples) grow(ctx->d_ztab, sizeof(float4) * K * st.zstride);
     // the finishing kernel writes the costs into coherent host memory: no
     // copy back, the host only waits for the stream
     const size_t had_hc = ctx->h_costs.bytes;
-    ctx->h_costs.reserve(sizeof(double) * K);
+    // (a small 256-bin launch stores its slice sums, combined by the host)
+    const bool small = !ctx->use_graphs && st.nseg == 1 && K <= kArgK && st.samples < kZTableSamples;
+    const size_t per_cand = small && mi && bins == 256 ? size_t(entropy_slices<256>()) : 1;
+    const size_t nslots = K * per_cand;
+    ctx->h_costs.reserve(sizeof(double) * nslots);
     grew = grew || ctx->h_costs.bytes != had_hc;
     double* hc = static_cast<double*>(ctx->h_costs.dev);
     auto enqueue = [&] {
@@ -1171,7 +1339,7 @@ void cost_jobs(tiplhip_ctx* ctx, std::vector<PairJob> jobs, const float* T, int 
     // stream synchronisation; after kCostSpinUs the wait falls back to one
     // (which also reports a failed launch).
     uint64_t* slots = static_cast<uint64_t*>(ctx->h_costs.p);
-    std::fill(slots, slots + K, kCostPending);
+    std::fill(slots, slots + nslots, kCostPending);
     // from here on a kernel may be queued that stores into the slots: if a
     // later step throws, drain the stream before the caller moves on
     auto drain = [ctx] { (void)hipStreamSynchronize(ctx->stream); };
@@ -1179,7 +1347,9 @@ void cost_jobs(tiplhip_ctx* ctx, std::vector<PairJob> jobs, const float* T, int 
     if (ctx->use_graphs && !ctx->kernel_timing) {
         // the same launch shape replays one graph; only the staged bytes
         // (transforms, crop flags, segment table) are new
-        if (mi) make_hist_clean(ctx, hist_bytes(st, bins));  // outside the graph
+        // (the clearing passes stay outside the graph)
+        if (mi) make_hist_clean(ctx, hist_bytes(st, bins));
+        else make_sums_clean(ctx, K);
         // (the buffers' addresses are part of the key: a graph is replayed
         // only on the buffers it was captured with, each reserved above for
         // this launch's sizes)
@@ -1218,13 +1388,20 @@ void cost_jobs(tiplhip_ctx* ctx, std::vector<PairJob> jobs, const float* T, int 
             it = ctx->graphs.emplace(key, ex).first;
         }
         TIPLHIP_CHECK(hipGraphLaunch(it->second, ctx->stream));
+    } else if (small) {
+        arg_cost(ctx, st, crop.data(), cost, bins, hc);
     } else {
         enqueue();
     }
-    wait_for_slots(static_cast<const volatile uint64_t*>(slots), K, kCostPending,
+    wait_for_slots(static_cast<const volatile uint64_t*>(slots), nslots, kCostPending,
                    std::chrono::microseconds(kCostSpinUs),
                    [ctx] { TIPLHIP_CHECK(hipStreamSynchronize(ctx->stream)); });
-    std::memcpy(costs, ctx->h_costs.p, sizeof(double) * K);
+    if (per_cand == 1) {
+        std::memcpy(costs, ctx->h_costs.p, sizeof(double) * K);
+    } else {
+        const double* part = ctx->h_costs.as<double>();
+        for (size_t k = 0; k < K; ++k) costs[k] = combine_slices<256>(part + k * per_cand);
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -1352,7 +1529,7 @@ void cost_noalloc(tiplhip_ctx* ctx, const tiplhip_volume* from, const tiplhip_vo
             TIPLHIP_CHECK(hipGetLastError());
             constexpr int G = entropy_slices<256>();
             hipLaunchKernelGGL(mi_entropy_kernel<256>, dim3(uint32_t(K) * uint32_t(G)), dim3(kEntropyThreads),
-                               0, st, d_seg, 1u, h, th, d_costs + K, d_costs, nullptr);
+                               0, st, d_seg, 1u, nullptr, h, th, nullptr, d_costs + K, d_costs, nullptr);
             TIPLHIP_CHECK(hipGetLastError());
             hipLaunchKernelGGL(mi_entropy_final_kernel<256>, dim3((uint32_t(K) + 255) / 256), dim3(256), 0,
                                st, d_costs + K, uint32_t(K), d_costs, nullptr, th);
@@ -1361,7 +1538,7 @@ void cost_noalloc(tiplhip_ctx* ctx, const tiplhip_volume* from, const tiplhip_vo
                                blocks, d_T, nullptr, 0u, h, th);
             TIPLHIP_CHECK(hipGetLastError());
             hipLaunchKernelGGL(mi_entropy_kernel<64>, dim3(uint32_t(K)), dim3(kEntropyThreads), 0, st, d_seg,
-                               1u, h, th, d_costs + K, d_costs, nullptr);
+                               1u, nullptr, h, th, nullptr, d_costs + K, d_costs, nullptr);
         }
         TIPLHIP_CHECK(hipGetLastError());
     } else {
@@ -1372,7 +1549,7 @@ void cost_noalloc(tiplhip_ctx* ctx, const tiplhip_volume* from, const tiplhip_vo
                            d_crop, nullptr, 0u, sums);
         TIPLHIP_CHECK(hipGetLastError());
         hipLaunchKernelGGL(corr_finalize_kernel, dim3((uint32_t(K) + 63) / 64), dim3(64), 0, st, d_seg, 1u,
-                           sums, K, d_costs, nullptr, nullptr);
+                           FromSums{}, sums, K, d_costs, nullptr, nullptr);
         TIPLHIP_CHECK(hipGetLastError());
     }
     TIPLHIP_CHECK(hipMemcpyAsync(costs, d_costs, sizeof(double) * size_t(K), hipMemcpyDeviceToHost, st));

@@ -147,6 +147,7 @@ struct tiplhip_ctx {
     // d_hist once queued work ends: [0, hist_dirty) holds counts no entropy
     // pass consumed, [hist_dirty, hist_zero) is zero
     size_t hist_dirty = 0, hist_zero = 0;
+    size_t sums_dirty = 0, sums_zero = 0;  // the same of d_sums, in candidates
     // autotuned launch shapes of single-pair cost launches
     std::map<tiplhip::TuneKey, tiplhip::LaunchShape> tuned;
     // timing
