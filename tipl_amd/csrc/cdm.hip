@@ -1184,11 +1184,12 @@ __device__ inline float3 accumulated(const float* __restrict__ cur, const float*
 }
 
 __global__ __launch_bounds__(256) void accumulate_kernel(const float* __restrict__ cur, const float* nd,
-                                                         Lay lay, float k, FieldGeo g, float* out)
+                                                         Lay lay, float k, FieldGeo g, float* out,
+                                                         Lay out_lay)
 {
     const Vox v = this_voxel(g);
     if (!v.ok) return;
-    st3(out, v.p, accumulated(cur, nd, lay, k, g, v.p, v.x, v.y, v.z));
+    st_lay(out, v.p, out_lay, accumulated(cur, nd, lay, k, g, v.p, v.x, v.y, v.z));
 }
 
 // One packed float3 voxel through a raw buffer resource: a load past the
@@ -1803,10 +1804,10 @@ float* launch_poisson(tiplhip_ctx* ctx, const float* nd, float* a, float* b, con
 }
 
 void launch_accumulate(tiplhip_ctx* ctx, const float* cur, const float* nd, Lay lay, float k,
-                       const FieldGeo& g, float* out)
+                       const FieldGeo& g, float* out, Lay out_lay)
 {
     hipLaunchKernelGGL(accumulate_kernel, tile_grid(g), dim3(kTX, kTY), 0, ctx->stream, cur, nd, lay, k, g,
-                       out);
+                       out, out_lay);
     TIPLHIP_CHECK(hipGetLastError());
 }
 
@@ -2583,9 +2584,12 @@ void cdm_fixed(CdmRun& run, const std::vector<const uint8_t*>& It,
         }
         if (theta == 0.0f) break;
         float* spare = solved == pa.as<float>() ? pb.as<float>() : pa.as<float>();
-        launch_accumulate(ctx, field, solved, lay, run.param.speed / theta, g, spare);
+        // (the gaussian reads a planar field where it marches four rounds a launch)
+        const bool planar = gaussian_takes_planar(dim, unsigned(run.param.field_bandwidth));
+        launch_accumulate(ctx, field, solved, lay, run.param.speed / theta, g, spare,
+                          planar ? Lay{1u, g.n} : packed_layout());
         if (run.param.field_bandwidth > 0) {
-            launch_gaussian_to(ctx, spare, field, solved, dim, 3, unsigned(run.param.field_bandwidth));
+            launch_gaussian_to(ctx, spare, field, solved, dim, 3, unsigned(run.param.field_bandwidth), planar);
         } else if (run.param.smoothing != 0.0f) {
             // cdm_smooth with weight 0 leaves the field untouched, as in the reference
             launch_smooth(ctx, spare, field, run.param.smoothing, g);
@@ -2790,7 +2794,8 @@ int tiplhip_accumulate_displacement(tiplhip_ctx* ctx, const float* cur, float* n
         DevMem dC(ctx, fb), dN(ctx, fb);
         TIPLHIP_CHECK(hipMemcpyAsync(dC.p, cur, fb, hipMemcpyHostToDevice, ctx->stream));
         TIPLHIP_CHECK(hipMemcpyAsync(dN.p, new_d, fb, hipMemcpyHostToDevice, ctx->stream));
-        launch_accumulate(ctx, dC.as<float>(), dN.as<float>(), packed_layout(), scale, g, dN.as<float>());
+        launch_accumulate(ctx, dC.as<float>(), dN.as<float>(), packed_layout(), scale, g, dN.as<float>(),
+                          packed_layout());
         TIPLHIP_CHECK(hipMemcpyAsync(new_d, dN.p, fb, hipMemcpyDeviceToHost, ctx->stream));
         TIPLHIP_CHECK(hipStreamSynchronize(ctx->stream));
     });

@@ -291,6 +291,18 @@ __device__ inline float wave_next(float v)
     return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x130, 0xf, 0xf, true));
 }
 
+// The same, a lane without one keeping its own value.
+__device__ inline float wave_prev_or(float v)
+{
+    return __int_as_float(
+        __builtin_amdgcn_update_dpp(__float_as_int(v), __float_as_int(v), 0x138, 0xf, 0xf, false));
+}
+__device__ inline float wave_next_or(float v)
+{
+    return __int_as_float(
+        __builtin_amdgcn_update_dpp(__float_as_int(v), __float_as_int(v), 0x130, 0xf, 0xf, false));
+}
+
 __device__ inline uint64_t wave_sum_u64(uint64_t v)
 {
     for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, kWave);

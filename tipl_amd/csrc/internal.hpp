@@ -250,6 +250,8 @@ float* launch_gaussian(tiplhip_ctx* ctx, float* a, float* tmp, const int* dim, i
                        unsigned bandwidth);
 // The same from src into dst (src is only read; tmp is clobbered).
 void launch_gaussian_to(tiplhip_ctx* ctx, const float* src, float* dst, float* tmp,
-                        const int* dim, int channels, unsigned bandwidth);
+                        const int* dim, int channels, unsigned bandwidth, bool planar = false);
+// Whether src may be planar (one array per channel) at this bandwidth.
+bool gaussian_takes_planar(const int* dim, unsigned bandwidth);
 
 }  // namespace tiplhip
