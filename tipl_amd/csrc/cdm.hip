@@ -2072,19 +2072,21 @@ void launch_cdm_steps(hipStream_t stream, CdmJob* const* J, int n)
 // The batch executor of one device: `lanes` streams, each with a StepGate
 // (at most kMaxSegs fields a batch, kGatherUs); a job keeps the lane it
 // joined (the one with the fewest members), whose stream orders its steps.
-// Levels above max_voxels run unbatched on their owner's stream.  Measured
-// on 32 uneven affine+CDM pairs served on 16 slots (pairs/s, two runs
-// each): unbatched 57.6-61.2; 1 lane (up to 8 fields a step, 5.5 on
-// average) 56.1-58.0 -- every registration held to the pace of the
-// largest field in its batch; 2 lanes 62.3-64.3; 3 lanes 64.6-65.6;
-// 4 lanes 65.6-68.8; 6 lanes 62.3; 8 lanes 61.6-61.9; 16 lanes (one field
-// a step) 58.9-61.3.  Leaving levels above 256K or 512K voxels unbatched
-// did not help (63.8-67.6).
+// Levels above max_voxels run unbatched on their owner's stream: a batch is
+// held to the pace of its largest field, and only a field of its own stream
+// takes the four-sweep Jacobi launches and the planar gradient field.
+// Measured on 32 uneven affine+CDM pairs served on 16 slots with 4 lanes
+// (pairs/s): every level batched 79.6-80.5, up to 2^18 voxels 83.7-87.3, up to
+// 4096 87.7-91.3, none 86.7-88.6; with four-sweep launches in the batched
+// steps 78.5-79.9.  The line is where a field alone would march.  Lanes, while every level was batched and took
+// two sweeps a launch alone as well: 1 lane 56.1-58.0, 2 62.3-64.3, 3
+// 64.6-65.6, 4 65.6-68.8, 6 62.3, 8 61.6-61.9, 16 58.9-61.3, unbatched
+// 57.6-61.2.
 class CdmBatcher {
 public:
     static constexpr int kGatherUs = 300;
     static constexpr int kDefaultLanes = 4;
-    static constexpr size_t kDefaultMaxVoxels = size_t(1) << 25;
+    static constexpr size_t kDefaultMaxVoxels = size_t(1) << 18;
 
     CdmBatcher(int device, int lanes, size_t max_voxels) : device_(device), max_voxels_(max_voxels)
     {
