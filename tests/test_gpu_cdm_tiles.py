@@ -48,11 +48,13 @@ def test_cdm_odd_levels_two_modalities(ctx, oracle):
     assert float(np.sqrt(((got - want) ** 2).sum(-1).mean())) <= 0.01
 
 
-@pytest.mark.parametrize("shape", [(1, 1, 1), (8, 8, 8), (9, 7, 17), (1, 3, 40), (40, 2, 1), (16, 24, 8),
-                                   (33, 20, 25)])
+@pytest.mark.parametrize("shape", [(1, 1, 1), (8, 8, 8), (9, 7, 17), (1, 3, 40), (40, 2, 1), (16, 16, 16),
+                                   (1, 1, 4096), (4096, 1, 1), (1, 1, 4097), (1030, 2, 2), (17, 16, 16),
+                                   (16, 24, 11), (33, 20, 25)])
 def test_poisson_four_sweep_tiles(ctx, oracle, shape):
-    """Volumes around the 8 x 8 x 8 tile of the four-sweep launch, thinner than
-    its halo, and with rows shorter than it: 4, 8 and 12 sweeps, and
+    """Volumes of up to 4096 voxels, which take every sweep in one launch, and
+    larger ones around the 8 x 8 x 8 tile of the four-sweep launch, thinner
+    than its halo, and with rows shorter than it: 4, 8 and 12 sweeps, and
     remainders after four-sweep launches."""
     nd = _field(shape, 21, 1.0, 0.0)
     for sweeps in (4, 12, 5, 6, 8, 11):
