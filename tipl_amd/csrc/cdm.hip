@@ -476,59 +476,8 @@ constexpr float kInvD2 = -0.5f / 3.0f;
 // 80x96x80).
 constexpr size_t kPoisson4Voxels = size_t(1) << 18;
 
-template <bool FIRST, bool MAXLEN>
-__global__ __launch_bounds__(256) void poisson_kernel(const float* __restrict__ nd,
-                                                      const float* __restrict__ a, FieldGeo g,
-                                                      float* __restrict__ b,
-                                                      float* __restrict__ maxparts)
-{
-    const Vox v = this_voxel(g);
-    float len = 0.0f;
-    if (v.ok) {
-        auto A = [&](uint32_t q) -> float3 {
-            if (FIRST) {
-                float3 t = ld3(nd, q);
-                return make_float3(t.x * kInvD2, t.y * kInvD2, t.z * kInvD2);
-            }
-            return ld3(a, q);
-        };
-        const uint32_t p = v.p, n = g.n, w = uint32_t(g.w), wh = g.wh;
-        float3 r = ld3(nd, p);
-        auto sub = [&](float3 t) {
-            r.x = r.x - t.x;
-            r.y = r.y - t.y;
-            r.z = r.z - t.z;
-        };
-        if (p >= 1u) sub(A(p - 1));
-        if (p < n - 1u) sub(A(p + 1));
-        if (p >= w) sub(A(p - w));
-        if (p < n - w) sub(A(p + w));
-        if (p >= wh) sub(A(p - wh));
-        if (p < n - wh) sub(A(p + wh));
-        r.x = r.x * kInvD2;
-        r.y = r.y * kInvD2;
-        r.z = r.z * kInvD2;
-        st3(b, p, r);
-        if (MAXLEN) {
-            float s2 = r.x * r.x + r.y * r.y;
-            s2 = s2 + r.z * r.z;
-            len = float(sqrt(double(s2)));
-        }
-    }
-    if (MAXLEN) {
-        __shared__ float part[4];
-        const uint32_t tid = threadIdx.y * blockDim.x + threadIdx.x;
-        float m = wave_max_f32(len);
-        if ((tid & 63u) == 0) part[tid >> 6] = m;
-        __syncthreads();
-        if (tid == 0) {
-            maxparts[logical_block().lin] = fmaxf(fmaxf(part[0], part[1]), fmaxf(part[2], part[3]));
-        }
-    }
-}
-
 // ---------------------------------------------------------------------------
-// The same Jacobi sweep, marching z.  A block owns a 64 x 8 column of voxels
+// One Jacobi sweep, marching z.  A block owns a 64 x 8 column of voxels
 // over kPZ planes; each thread keeps the previous iterate of its own column
 // at z-1, z, z+1 in registers (the +-wh neighbours), takes x-1 / x+1 from
 // the neighbouring lanes of its wave, y-1 / y+1 from the block's LDS copy of
