@@ -21,6 +21,7 @@
 #include "cdm_control.hpp"
 #include "device.hpp"
 #include "field.hpp"
+#include "field_limits.hpp"
 #include "host_wait.hpp"
 #include "internal.hpp"
 #include "regression.hpp"
@@ -52,10 +53,7 @@ struct Lay {
     uint32_t ps, cs;
 };
 __host__ __device__ inline Lay packed_layout() { return Lay{3u, 1u}; }
-inline bool planar_fits(const FieldGeo& g)
-{
-    return (size_t(g.n) + 8 * size_t(g.wh) + 64 * size_t(g.w)) * 12 < (size_t(1) << 31);
-}
+inline bool planar_fits(const FieldGeo& g) { return marched_field_fits(g.n, g.wh, size_t(g.w)); }
 inline Lay grad_layout(const FieldGeo& g) { return planar_fits(g) ? Lay{1u, g.n} : packed_layout(); }
 
 __device__ inline float3 ld_lay(const float* f, uint32_t p, const Lay& l)
@@ -1840,11 +1838,27 @@ void launch_accumulate(tiplhip_ctx* ctx, const float* cur, const float* nd, Lay 
     TIPLHIP_CHECK(hipGetLastError());
 }
 
-// accumulate then cdm_smooth with `smoothing` (non-zero) in one pass into
-// out, and compose_displacement of Is by out into Js where Js is set.
-void launch_accumulate_smooth(tiplhip_ctx* ctx, const float* cur, const float* nd, Lay lay, float k,
+void launch_smooth(tiplhip_ctx* ctx, const float* d, float* dd, float smoothing, const FieldGeo& g)
+{
+    const float w_6 = smoothing / float(2.0f * 3.0f);
+    const float w_1 = 1.0f - smoothing;
+    hipLaunchKernelGGL(smooth_kernel, tile_grid(g), dim3(kTX, kTY), 0, ctx->stream, d, dd, w_6, w_1, g);
+    TIPLHIP_CHECK(hipGetLastError());
+}
+
+// accumulate then cdm_smooth with `smoothing` (non-zero) into out, and where
+// the one-pass kernel runs compose_displacement of Is by out into Js, if Js is
+// set; returns whether it did.  That kernel addresses the packed field in 32
+// bits: a field of 2^32 bytes and more takes the two kernels it replaces, whose
+// addresses are 64 bits wide, and nd (packed there) is overwritten.
+bool launch_accumulate_smooth(tiplhip_ctx* ctx, const float* cur, float* nd, Lay lay, float k,
                               float smoothing, const FieldGeo& g, float* out, const uint8_t* Is, uint8_t* Js)
 {
+    if (!field_fits_32(g.n)) {
+        launch_accumulate(ctx, cur, nd, lay, k, g, nd, lay);
+        launch_smooth(ctx, nd, out, smoothing, g);
+        return false;
+    }
     const float w_6 = smoothing / float(2.0f * 3.0f);
     const float w_1 = 1.0f - smoothing;
     if (acc_large(g))
@@ -1854,14 +1868,7 @@ void launch_accumulate_smooth(tiplhip_ctx* ctx, const float* cur, const float* n
         hipLaunchKernelGGL(accumulate_smooth_kernel<false>, acc_grid(g), dim3(AccTile<false>::kThreads), 0,
                            ctx->stream, cur, nd, lay, k, w_6, w_1, g, out, Is, Js);
     TIPLHIP_CHECK(hipGetLastError());
-}
-
-void launch_smooth(tiplhip_ctx* ctx, const float* d, float* dd, float smoothing, const FieldGeo& g)
-{
-    const float w_6 = smoothing / float(2.0f * 3.0f);
-    const float w_1 = 1.0f - smoothing;
-    hipLaunchKernelGGL(smooth_kernel, tile_grid(g), dim3(kTX, kTY), 0, ctx->stream, d, dd, w_6, w_1, g);
-    TIPLHIP_CHECK(hipGetLastError());
+    return Js != nullptr;
 }
 
 void launch_upsample(tiplhip_ctx* ctx, const float* in, const FieldGeo& gi, const FieldGeo& go,
@@ -2438,7 +2445,7 @@ bool cdm_level(CdmRun& run, const std::vector<const uint8_t*>& It,
     }
     if (run.stopped) return true;
     if (run.ctx->cdm_batch && run.nmod == 1 && run.param.gradient_type[0] != 'd' &&
-        !run.no_early_exit && n <= run.ctx->cdm_batch->max_voxels())
+        !run.no_early_exit && n <= run.ctx->cdm_batch->max_voxels() && field_fits_32(n))
         return cdm_iterate_batched(run, It[0], Is[0], g, best_d);
 
     // four fields rotate: the running field, the best field so far -- which may
@@ -2537,9 +2544,8 @@ bool cdm_level(CdmRun& run, const std::vector<const uint8_t*>& It,
         // accumulated field is then unused), as in the reference
         if (cur_smoothing != 0.0f) {
             float* spare = solved == pa ? pb : pa;
-            composed = run.nmod == 1;
-            launch_accumulate_smooth(ctx, cur, solved, lay, k, cur_smoothing, g, spare, Is[0],
-                                     composed ? Js.as<uint8_t>() : nullptr);
+            composed = launch_accumulate_smooth(ctx, cur, solved, lay, k, cur_smoothing, g, spare, Is[0],
+                                                run.nmod == 1 ? Js.as<uint8_t>() : nullptr);
             pa = cur == best ? spare_field : cur;
             pb = solved;
             cur = spare;
