@@ -235,6 +235,8 @@ __global__ __launch_bounds__(256) void ztab_kernel(const float* __restrict__ Ts,
 // crop[k] = {flag, sx, sy, sz}: flag 1 reproduces the CPU resample's exact
 // crop for an integer-shift transform (numerical/resampling.hpp:1244-1262).
 // ---------------------------------------------------------------------------
+constexpr int kCorrThreads = 256;
+
 template <bool ZT>
 __device__ __forceinline__ void corr_sums_body(const Segment& sg, uint32_t L, const float* Ts,
                                                const int4* crop, const float4* __restrict__ ztab,
@@ -254,7 +256,7 @@ __device__ __forceinline__ void corr_sums_body(const Segment& sg, uint32_t L, co
     const __amdgpu_buffer_rsrc_t r8 = make_rsrc(sg.to8, g.to_bytes8);
     const uint32_t lane = threadIdx.x & 63u;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const uint32_t nwaves = blockDim.x >> 6;
+    const uint32_t nwaves = uint32_t(kCorrThreads) / 64u;
     const uint32_t it0 = chunk * g.items_per_block;
     const uint32_t it1 = min(it0 + g.items_per_block, g.items);
     const uint32_t fwh = uint32_t(g.fw) * uint32_t(g.fh);
@@ -316,7 +318,7 @@ __device__ __forceinline__ void corr_sums_body(const Segment& sg, uint32_t L, co
         else
             march(std::false_type{});
     }
-    __shared__ unsigned long long red[3][4];
+    __shared__ unsigned long long red[3][kCorrThreads / 64];
     unsigned long long a = wave_sum_u64(sy), b = wave_sum_u64(syy), c = wave_sum_u64(sxy);
     if (lane == 0) {
         red[0][wave] = a;
@@ -332,7 +334,7 @@ __device__ __forceinline__ void corr_sums_body(const Segment& sg, uint32_t L, co
 }
 
 template <bool ZT>
-__global__ __launch_bounds__(256) void corr_sums_kernel(const Segment* __restrict__ segs,
+__global__ __launch_bounds__(kCorrThreads) void corr_sums_kernel(const Segment* __restrict__ segs,
                                                         uint32_t nseg, uint32_t total_blocks,
                                                         const float* __restrict__ Ts,
                                                         const int4* __restrict__ crop,
@@ -344,23 +346,15 @@ __global__ __launch_bounds__(256) void corr_sums_kernel(const Segment* __restric
     corr_sums_body<ZT>(segs[find_segment(segs, nseg, L, ByBlock{})], L, Ts, crop, ztab, zstride, sums);
 }
 
-// The inputs of a launch over one pair and few candidates, which travel as a
-// kernel argument: no upload, and no wait for one, before the launch.
-constexpr uint32_t kArgK = 56;
-struct ArgBatch {
-    Segment seg;
-    float T[12 * kArgK];
-};
-struct ArgCrops {
-    int4 crop[kArgK];
-};
-static_assert(sizeof(ArgBatch) + sizeof(ArgCrops) + 64 <= 4096, "kernel arguments end at 4 KB");
-
-__global__ __launch_bounds__(256) void corr_sums_arg_kernel(const ArgBatch in, const ArgCrops crops,
-                                                            uint32_t total_blocks,
-                                                            unsigned long long* __restrict__ sums)
+// One pair: its segment travels as a kernel argument, and Ts and crop may lie in
+// mapped host memory (one_pair_cost).
+__global__ __launch_bounds__(kCorrThreads) void corr_sums_one_kernel(const Segment seg,
+                                                                     const float* __restrict__ Ts,
+                                                                     const int4* __restrict__ crop,
+                                                                     uint32_t total_blocks,
+                                                                     unsigned long long* __restrict__ sums)
 {
-    corr_sums_body<false>(in.seg, xcd_remap(blockIdx.x, total_blocks), in.T, crops.crop, nullptr, 0u, sums);
+    corr_sums_body<false>(seg, xcd_remap(blockIdx.x, total_blocks), Ts, crop, nullptr, 0u, sums);
 }
 
 // What the finalizer needs of a candidate's `from` volume.
@@ -456,14 +450,7 @@ __device__ __forceinline__ void mi_hist_body(const Segment& sg, uint32_t L, cons
                                              int* __restrict__ hist, uint32_t* __restrict__ to_hist)
 {
     using Tr = MiTraits<BINS>;
-    // cleared 16 bytes a store: the 256-bin kernel 0.8-1.4% faster at
-    // 182x218x182 with 64 candidates (0.970 -> 0.963 ms), the 64-bin one unchanged
-    static_assert(Tr::kLdsWords % 4 == 0, "the clear stores 16 bytes at a time");
-    __shared__ __align__(16) uint32_t lds[Tr::kLdsWords];
-    for (uint32_t i = threadIdx.x; i < uint32_t(Tr::kLdsWords) / 4u; i += blockDim.x)
-        reinterpret_cast<uint4*>(lds)[i] = make_uint4(0u, 0u, 0u, 0u);
-    __syncthreads();
-
+    // (the transform first: it arrives while the histogram is cleared)
     const BatchGeo g = sg.g;
     const uint32_t local = L - sg.block_begin;
     const uint32_t cand = sg.cand_begin + local % g.K;
@@ -471,12 +458,20 @@ __device__ __forceinline__ void mi_hist_body(const Segment& sg, uint32_t L, cons
     float T[12];
 #pragma unroll
     for (int i = 0; i < 12; ++i) T[i] = Ts[12 * cand + i];
+    // cleared 16 bytes a store: the 256-bin kernel 0.8-1.4% faster at
+    // 182x218x182 with 64 candidates (0.970 -> 0.963 ms), the 64-bin one unchanged
+    static_assert(Tr::kLdsWords % 4 == 0, "the clear stores 16 bytes at a time");
+    __shared__ __align__(16) uint32_t lds[Tr::kLdsWords];
+    for (uint32_t i = threadIdx.x; i < uint32_t(Tr::kLdsWords) / 4u; i += uint32_t(Tr::kThreads))
+        reinterpret_cast<uint4*>(lds)[i] = make_uint4(0u, 0u, 0u, 0u);
+    __syncthreads();
+
     const uint32_t zrow = cand * zstride;
     const __amdgpu_buffer_rsrc_t rf = make_rsrc(sg.from, g.from_bytes);
     const __amdgpu_buffer_rsrc_t r8 = make_rsrc(sg.to8, g.to_bytes8);
     const uint32_t lane = threadIdx.x & 63u;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const uint32_t nwaves = blockDim.x >> 6;
+    const uint32_t nwaves = uint32_t(Tr::kThreads) >> 6;
     const uint32_t it0 = chunk * g.items_per_block;
     const uint32_t it1 = min(it0 + g.items_per_block, g.items);
     const uint32_t fwh = uint32_t(g.fw) * uint32_t(g.fh);
@@ -552,7 +547,7 @@ __device__ __forceinline__ void mi_hist_body(const Segment& sg, uint32_t L, cons
                   "flush layout");
     int* h = hist + size_t(cand) * BINS * BINS;
     uint32_t col_lo = 0, col_hi = 0;
-    for (uint32_t i = threadIdx.x; i < uint32_t(Tr::kWords); i += blockDim.x) {
+    for (uint32_t i = threadIdx.x; i < uint32_t(Tr::kWords); i += uint32_t(Tr::kThreads)) {
         const uint32_t v = lds[(i / kWpr) * uint32_t(Tr::kStride) + (i % kWpr)];
         if constexpr (BINS == 256) {
             col_lo += v & 0xffffu;
@@ -595,11 +590,14 @@ __global__ __launch_bounds__(MiTraits<BINS>::kThreads) void mi_hist_kernel(
     mi_hist_body<BINS, ZT>(segs[find_segment(segs, nseg, L, ByBlock{})], L, Ts, ztab, zstride, hist, to_hist);
 }
 
+// One pair: its segment travels as a kernel argument, and Ts may lie in mapped
+// host memory (one_pair_cost).
 template <int BINS>
-__global__ __launch_bounds__(MiTraits<BINS>::kThreads) void mi_hist_arg_kernel(
-    const ArgBatch in, uint32_t total_blocks, int* __restrict__ hist, uint32_t* __restrict__ to_hist)
+__global__ __launch_bounds__(MiTraits<BINS>::kThreads) void mi_hist_one_kernel(
+    const Segment seg, const float* __restrict__ Ts, uint32_t total_blocks, int* __restrict__ hist,
+    uint32_t* __restrict__ to_hist)
 {
-    mi_hist_body<BINS, false>(in.seg, xcd_remap(blockIdx.x, total_blocks), in.T, nullptr, 0u, hist, to_hist);
+    mi_hist_body<BINS, false>(seg, xcd_remap(blockIdx.x, total_blocks), Ts, nullptr, 0u, hist, to_hist);
 }
 
 // get_mutual_info_mean (reg/linear.hpp:87-104): the sum of
@@ -871,8 +869,11 @@ struct Staged {
     uint32_t zstride = 0;   // the largest `from` depth: rows of the z-product table
     size_t bytes = 0;       // staged bytes (transforms, crop flags, segment table)
     bool grew = false;      // the device staging buffer was reallocated
-    const Segment* host_segs = nullptr;  // the staged inputs in host memory (until the next staging)
-    const float* host_T = nullptr;
+    // the staged inputs in mapped host memory (until the next staging): the
+    // first segment as the host reads it, transforms and crop flags as kernels do
+    const Segment* host_seg = nullptr;
+    const float* mapped_T = nullptr;
+    const int4* mapped_crop = nullptr;
 };
 
 // Launches of at least this many samples get a z-product table: its build
@@ -990,8 +991,10 @@ Staged stage_jobs(tiplhip_ctx* ctx, const std::vector<PairJob>& jobs, const floa
     if (crop) std::memcpy(h + tb, crop, cb);
     std::memcpy(h + tb + cb, segs.data(), sb);
     if (upload) TIPLHIP_CHECK(hipMemcpyAsync(ctx->d_T.p, h, st.bytes, hipMemcpyHostToDevice, ctx->stream));
-    st.host_T = hT;
-    st.host_segs = reinterpret_cast<const Segment*>(h + tb + cb);
+    st.host_seg = reinterpret_cast<const Segment*>(h + tb + cb);
+    const char* m = static_cast<const char*>(ctx->h_T.dev);
+    st.mapped_T = reinterpret_cast<const float*>(m);
+    st.mapped_crop = crop ? reinterpret_cast<const int4*>(m + tb) : nullptr;
     char* d = static_cast<char*>(ctx->d_T.p);
     st.T = reinterpret_cast<const float*>(d);
     st.crop = crop ? reinterpret_cast<const int4*>(d + tb) : nullptr;
@@ -1052,11 +1055,11 @@ void launch_corr_sums(tiplhip_ctx* ctx, const Staged& st)
     // per-lane uint32 sums of squares stay below 2^32 for < 65536 voxels a lane
     timing_begin(ctx);
     if (zt)
-        hipLaunchKernelGGL(corr_sums_kernel<true>, dim3(st.total_blocks), dim3(256), 0, ctx->stream,
+        hipLaunchKernelGGL(corr_sums_kernel<true>, dim3(st.total_blocks), dim3(kCorrThreads), 0, ctx->stream,
                            st.segs, st.nseg, st.total_blocks, st.T, st.crop, zt, st.zstride,
                            ctx->d_sums.as<unsigned long long>());
     else
-        hipLaunchKernelGGL(corr_sums_kernel<false>, dim3(st.total_blocks), dim3(256), 0, ctx->stream,
+        hipLaunchKernelGGL(corr_sums_kernel<false>, dim3(st.total_blocks), dim3(kCorrThreads), 0, ctx->stream,
                            st.segs, st.nseg, st.total_blocks, st.T, st.crop, nullptr, 0u,
                            ctx->d_sums.as<unsigned long long>());
     TIPLHIP_CHECK(hipGetLastError());
@@ -1081,7 +1084,7 @@ uint32_t* to_hist_of(tiplhip_ctx* ctx, const Staged& st, int bins)
     return reinterpret_cast<uint32_t*>(ctx->d_hist.as<int>() + size_t(bins) * bins * size_t(st.K));
 }
 
-// ... then (arg_cost) a ticket per candidate.
+// ... then (one_pair_cost) a ticket per candidate.
 size_t hist_bytes(const Staged& st, int bins)
 {
     return sizeof(int) * (size_t(bins) * bins + size_t(bins)) * size_t(st.K) +
@@ -1191,31 +1194,37 @@ void launch_resample(tiplhip_ctx* ctx, const tiplhip_volume* src, const int* out
     TIPLHIP_CHECK(hipGetLastError());
 }
 
-// The cost launches of one pair and at most kArgK candidates: the inputs are
-// kernel arguments, and a 256-bin launch's slice sums go to host_out, K x
-// slices of them, for the host to combine.  Two launches, where the staged
-// path has an upload and three (correlation: an upload, a clear and two).
-// Such a launch is latency: 33.5 -> 29.4 us a call for ten 48x48x48 candidates
-// at 256 bins, 50.2 -> 45.6 for twelve of 91x109x91.  (kArgK is what 4 KB of
-// arguments hold.)
-void arg_cost(tiplhip_ctx* ctx, const Staged& st, const int4* crop, int cost, int bins, double* host_out)
+// The cost launches of one pair and at most kOneK candidates: the segment is a
+// kernel argument, the transforms are read from mapped host memory, and a
+// 256-bin launch's slice sums go to host_out, K x slices of them, for the host
+// to combine.  Two launches, where the staged path has an upload and three
+// (correlation: an upload, a clear and two).
+// Such a launch is latency: 35.9 -> 32.4 us a call for twelve 48x48x48
+// candidates at 256 bins, 50.4 -> 46.9 at 91x109x91, 64.5 -> 63.1 for 56 of
+// 48x48x48 and 132.4 -> 129.4 for 256, the most that was measured; 64 bins and
+// correlation gain 2 to 3 us at every count, 12 at 256.
+// (Transforms as kernel arguments too are up to 1 us faster again.  But from
+// some 500 bytes of arguments on, the launch call allocates memory in a way that
+// makes the C library merge the free blocks of the whole heap first: 10 to 60 us
+// in one of the first calls after a program has freed many.)
+// The host may stage the next call's inputs as soon as the costs are there: the
+// kernel that reads these has ended before the one that stores the costs began.
+constexpr size_t kOneK = 256;
+
+void one_pair_cost(tiplhip_ctx* ctx, const Staged& st, int cost, int bins, double* host_out)
 {
-    ArgBatch in;
-    in.seg = st.host_segs[0];
-    std::memcpy(in.T, st.host_T, sizeof(float) * 12 * st.K);
+    const Segment& seg = *st.host_seg;
     if (cost == TIPLHIP_COST_CORR) {
-        ArgCrops crops;
-        std::memcpy(crops.crop, crop, sizeof(int4) * st.K);
         make_sums_clean(ctx, st.K);
         ctx->sums_dirty = st.K;
         unsigned long long* sums = ctx->d_sums.as<unsigned long long>();
         timing_begin(ctx);
-        hipLaunchKernelGGL(corr_sums_arg_kernel, dim3(st.total_blocks), dim3(256), 0, ctx->stream, in, crops,
-                           st.total_blocks, sums);
+        hipLaunchKernelGGL(corr_sums_one_kernel, dim3(st.total_blocks), dim3(kCorrThreads), 0, ctx->stream, seg,
+                           st.mapped_T, st.mapped_crop, st.total_blocks, sums);
         TIPLHIP_CHECK(hipGetLastError());
         timing_end(ctx);
         hipLaunchKernelGGL(corr_finalize_kernel, dim3((st.K + 63) / 64), dim3(64), 0, ctx->stream, nullptr,
-                           0u, FromSums{in.seg.sx, in.seg.sxx, in.seg.n}, sums, int(st.K),
+                           0u, FromSums{seg.sx, seg.sxx, seg.n}, sums, int(st.K),
                            ctx->d_costs.as<double>(), host_out, nullptr);
         TIPLHIP_CHECK(hipGetLastError());
         ctx->sums_dirty = 0;
@@ -1229,20 +1238,20 @@ void arg_cost(tiplhip_ctx* ctx, const Staged& st, const int4* crop, int cost, in
     double* costs = ctx->d_costs.as<double>();
     timing_begin(ctx);
     if (bins == 256)
-        hipLaunchKernelGGL(mi_hist_arg_kernel<256>, dim3(st.total_blocks), dim3(1024), 0, ctx->stream, in,
-                           st.total_blocks, h, th);
+        hipLaunchKernelGGL(mi_hist_one_kernel<256>, dim3(st.total_blocks), dim3(MiTraits<256>::kThreads), 0,
+                           ctx->stream, seg, st.mapped_T, st.total_blocks, h, th);
     else
-        hipLaunchKernelGGL(mi_hist_arg_kernel<64>, dim3(st.total_blocks), dim3(256), 0, ctx->stream, in,
-                           st.total_blocks, h, th);
+        hipLaunchKernelGGL(mi_hist_one_kernel<64>, dim3(st.total_blocks), dim3(MiTraits<64>::kThreads), 0,
+                           ctx->stream, seg, st.mapped_T, st.total_blocks, h, th);
     TIPLHIP_CHECK(hipGetLastError());
     timing_end(ctx);
     if (bins == 256)
         hipLaunchKernelGGL(mi_entropy_kernel<256>, dim3(st.K * uint32_t(entropy_slices<256>())),
-                           dim3(kEntropyThreads), 0, ctx->stream, nullptr, 0u, in.seg.from_hist, h, th,
+                           dim3(kEntropyThreads), 0, ctx->stream, nullptr, 0u, seg.from_hist, h, th,
                            tickets_of(ctx, st, bins), host_out, costs, nullptr);
     else
         hipLaunchKernelGGL(mi_entropy_kernel<64>, dim3(st.K), dim3(kEntropyThreads), 0, ctx->stream, nullptr,
-                           0u, in.seg.from_hist, h, th, nullptr, nullptr, costs, host_out);
+                           0u, seg.from_hist, h, th, nullptr, nullptr, costs, host_out);
     TIPLHIP_CHECK(hipGetLastError());
     ctx->hist_dirty = 0;
 }
@@ -1313,7 +1322,7 @@ void cost_jobs(tiplhip_ctx* ctx, std::vector<PairJob> jobs, const float* T, int 
     // copy back, the host only waits for the stream
     const size_t had_hc = ctx->h_costs.bytes;
     // (a small 256-bin launch stores its slice sums, combined by the host)
-    const bool small = !ctx->use_graphs && st.nseg == 1 && K <= kArgK && st.samples < kZTableSamples;
+    const bool small = !ctx->use_graphs && st.nseg == 1 && K <= kOneK && st.samples < kZTableSamples;
     const size_t per_cand = small && mi && bins == 256 ? size_t(entropy_slices<256>()) : 1;
     const size_t nslots = K * per_cand;
     ctx->h_costs.reserve(sizeof(double) * nslots);
@@ -1389,7 +1398,7 @@ void cost_jobs(tiplhip_ctx* ctx, std::vector<PairJob> jobs, const float* T, int 
         }
         TIPLHIP_CHECK(hipGraphLaunch(it->second, ctx->stream));
     } else if (small) {
-        arg_cost(ctx, st, crop.data(), cost, bins, hc);
+        one_pair_cost(ctx, st, cost, bins, hc);
     } else {
         enqueue();
     }
@@ -1545,7 +1554,7 @@ void cost_noalloc(tiplhip_ctx* ctx, const tiplhip_volume* from, const tiplhip_vo
         TIPLHIP_CHECK(hipMemcpyAsync(scr + kNaCrop, crop, sizeof(int4) * size_t(K), hipMemcpyHostToDevice, st));
         unsigned long long* sums = reinterpret_cast<unsigned long long*>(scr + kNaSums);
         zero_u64(ctx, sums, 4 * size_t(K));
-        hipLaunchKernelGGL(corr_sums_kernel<false>, dim3(blocks), dim3(256), 0, st, d_seg, 1u, blocks, d_T,
+        hipLaunchKernelGGL(corr_sums_kernel<false>, dim3(blocks), dim3(kCorrThreads), 0, st, d_seg, 1u, blocks, d_T,
                            d_crop, nullptr, 0u, sums);
         TIPLHIP_CHECK(hipGetLastError());
         hipLaunchKernelGGL(corr_finalize_kernel, dim3((uint32_t(K) + 63) / 64), dim3(64), 0, st, d_seg, 1u,

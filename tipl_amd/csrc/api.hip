@@ -687,8 +687,10 @@ int tiplhip_ctx_create(int device, tiplhip_ctx** out)
         TIPLHIP_REQUIRE(device >= 0 && device < n, "device index out of range");
         auto* c = new tiplhip_ctx();
         c->device = device;
-        // costs written by kernels straight into host memory: uncached on the
-        // device side, so a finished kernel's writes are already visible
+        // costs written by kernels straight into host memory, and transforms
+        // they read from it: uncached on the device side, so a finished kernel's
+        // writes, and the host's before a launch, are already visible
+        c->h_T.flags = hipHostMallocMapped | hipHostMallocCoherent;
         c->h_costs.flags = hipHostMallocMapped | hipHostMallocCoherent;
         c->h_cdm.flags = hipHostMallocMapped | hipHostMallocCoherent;
         try {
