@@ -5,6 +5,7 @@
 #include <condition_variable>
 #include <cstddef>
 #include <cstring>
+#include <memory>
 #include <mutex>
 #include <system_error>
 #include <thread>
@@ -96,5 +97,70 @@ void staged_copy(char* host, size_t bytes, const char* staging, size_t chunk, si
     }
     pool.finished = true;  // the threads leave when every chunk is taken
 }
+
+// Objects that several threads borrow, at most `limit` of them: take() lends an
+// idle one, or one it makes while there are fewer, or none.  An object goes back
+// when its lease ends; all are destroyed with the pool, which outlives them.
+template <class T>
+class BoundedPool {
+public:
+    explicit BoundedPool(size_t limit) : limit_(limit) {}
+    BoundedPool(const BoundedPool&) = delete;
+    BoundedPool& operator=(const BoundedPool&) = delete;
+
+    class Lease {
+    public:
+        Lease() = default;
+        Lease(BoundedPool* pool, std::unique_ptr<T> t) : pool_(pool), t_(std::move(t)) {}
+        Lease(Lease&&) = default;
+        Lease& operator=(Lease&&) = delete;
+        ~Lease()
+        {
+            if (t_) pool_->put(std::move(t_));
+        }
+        explicit operator bool() const { return t_ != nullptr; }
+        T* operator->() const { return t_.get(); }
+
+    private:
+        BoundedPool* pool_ = nullptr;
+        std::unique_ptr<T> t_;
+    };
+
+    // make() returns a unique_ptr<T>; where it throws, the place stays free.
+    template <class Make>
+    Lease take(Make&& make)
+    {
+        {
+            std::lock_guard<std::mutex> lk(mu_);
+            if (!idle_.empty()) {
+                std::unique_ptr<T> t = std::move(idle_.back());
+                idle_.pop_back();
+                return Lease(this, std::move(t));
+            }
+            if (made_ == limit_) return Lease();
+            idle_.reserve(made_ + 1);  // put() never allocates
+            ++made_;
+        }
+        try {
+            return Lease(this, make());
+        } catch (...) {
+            std::lock_guard<std::mutex> lk(mu_);
+            --made_;
+            throw;
+        }
+    }
+
+private:
+    void put(std::unique_ptr<T> t)
+    {
+        std::lock_guard<std::mutex> lk(mu_);
+        idle_.push_back(std::move(t));
+    }
+
+    const size_t limit_;
+    std::mutex mu_;
+    std::vector<std::unique_ptr<T>> idle_;
+    size_t made_ = 0;
+};
 
 }  // namespace tiplhip

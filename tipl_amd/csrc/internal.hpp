@@ -16,6 +16,7 @@
 
 #include "../../include/tiplhip.h"
 #include "errors.hpp"
+#include "host_copy.hpp"
 
 // Every FP32 operation on the bit-exact paths must be a separately rounded
 // IEEE operation in source order (the reference's uint8 truncation after
@@ -142,8 +143,9 @@ struct tiplhip_ctx {
     tiplhip::PinnedBuffer h_out;
     tiplhip::PinnedBuffer h_costs;   // coherent: cost kernels write the K costs here directly
     tiplhip::PinnedBuffer h_cdm;     // coherent: a CDM iteration's per-modality costs
-    tiplhip::PinnedBuffer h_stage;   // staging ring of large copies to the host
-    std::vector<hipEvent_t> stage_events;  // one per slot of it
+    // staging rings of large copies to the host, shared by the process's contexts
+    std::shared_ptr<tiplhip::BoundedPool<tiplhip::PinnedBuffer>> staging;
+    std::vector<hipEvent_t> stage_events;  // one per slot of a ring
     // d_hist once queued work ends: [0, hist_dirty) holds counts no entropy
     // pass consumed, [hist_dirty, hist_zero) is zero
     size_t hist_dirty = 0, hist_zero = 0;
