@@ -24,6 +24,7 @@
 #include "field_limits.hpp"
 #include "host_wait.hpp"
 #include "internal.hpp"
+#include "march_plan.hpp"
 #include "regression.hpp"
 #include "step_gate.hpp"
 
@@ -912,24 +913,10 @@ March march_of(const FieldGeo& g)
     March m;
     m.gx = uint32_t((g.w + 63 - 2 * K) / (64 - 2 * K));
     m.gy = uint32_t((g.h + kMRows - 1 - 2 * K) / (kMRows - 2 * K));
-    // two workgroups run on a CU at a time: the number of z runs with the
-    // fewest steps over all rounds of them
     const uint32_t cols = 3u * m.gx * m.gy;
-    long best = 0;
-    for (int zc = g.d; zc >= 2; --zc) {
-        const uint32_t gz = uint32_t((g.d + zc - 1) / zc);
-        const long rounds = long((uint64_t(cols) * gz + kMarchBlocks - 1) / kMarchBlocks);
-        const long steps = rounds * (zc + 2 * K + 2);
-        if (best && steps >= best) continue;
-        best = steps;
-        m.gz = gz;
-        m.zc = zc;
-        if (rounds > 64) break;
-    }
-    if (!best) {
-        m.gz = 1;
-        m.zc = g.d;
-    }
+    const MarchPlan p = march_plan(cols, g.d, 2 * K + 2, 2, kMarchBlocks);
+    m.gz = p.runs;
+    m.zc = p.planes;
     m.blocks = cols * m.gz;
     return m;
 }

@@ -15,6 +15,7 @@
 // volume, CH = 3 for a vector<3,float> displacement field.
 #include "device.hpp"
 #include "internal.hpp"
+#include "march_plan.hpp"
 
 #include <algorithm>
 #include <cmath>
@@ -178,21 +179,10 @@ GaussMarch gauss_march(const GaussGeo& g, int channels)
     GaussMarch m;
     m.gx = tiles(g.w, 64);
     m.gy = tiles(g.h, kMRows);
-    // the number of z runs with the fewest steps over all rounds of workgroups
     const uint32_t cols = uint32_t(channels) * m.gx * m.gy;
-    long best = 0;
-    for (int zc = g.d; zc >= 1; --zc) {
-        const uint32_t gz = uint32_t((g.d + zc - 1) / zc);
-        const long rounds = long((uint64_t(cols) * gz + kMBlocks - 1) / kMBlocks);
-        const long steps = rounds * (zc + 3 * kMK + 2);
-        if (best && steps >= best) {
-            if (rounds > 64) break;
-            continue;
-        }
-        best = steps;
-        m.gz = gz;
-        m.zc = zc;
-    }
+    const MarchPlan p = march_plan(cols, g.d, 3 * kMK + 2, 1, kMBlocks);
+    m.gz = p.runs;
+    m.zc = p.planes;
     m.blocks = cols * m.gz;
     return m;
 }
