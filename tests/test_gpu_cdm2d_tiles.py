@@ -26,6 +26,20 @@ def test_poisson2d_tile_edges(ctx, oracle, shape):
         assert ml == oracle.max_length2(want)
 
 
+@pytest.mark.parametrize("shape", [(1, 1), (41, 39), (12, 200), (90, 1)])
+def test_poisson2d_signed_zeros(ctx, oracle, shape):
+    """Fields of -0.0, and of -0.0 and +0.0 mixed: a neighbour past either end of
+    the array is dropped, so a -0.0 there must stay one, in the first sweep too."""
+    r = np.random.default_rng(3)
+    for nd in (np.full(shape + (2,), -0.0, np.float32),
+               np.where(r.random(shape + (2,)) < 0.5, -0.0, 0.0).astype(np.float32)):
+        for sweeps in (1, 12, 13):
+            got, _ = ctx.poisson2d(nd, sweeps)
+            want = nd.copy()
+            oracle._c2_poisson(want, oracle._d2(want), sweeps)
+            assert _bits_equal(got, want), sweeps
+
+
 @pytest.mark.parametrize("shape", [(1, 1), (16, 16), (17, 15), (2, 33), (35, 1)])
 def test_gradient2d_tile_edges(ctx, oracle, shape):
     """Images around the 16 x 16 tile, full-range bytes."""

@@ -79,6 +79,19 @@ def test_poisson_marched_tiles(ctx, oracle, shape):
         assert ml == oracle.max_length(want)
 
 
+@pytest.mark.parametrize("shape", [(16, 16, 16), (17, 19, 16), (3, 5, 300), (64, 64, 65), (3, 300, 301), (1, 1, 5000)])
+def test_poisson_signed_zeros(ctx, oracle, shape):
+    """Fields of -0.0, and of -0.0 and +0.0 mixed: a neighbour past either end of
+    the array is dropped, so a -0.0 there must stay one, in the first sweep too,
+    in the launch that takes every sweep, the tiled and the marched one."""
+    r = np.random.default_rng(3)
+    for nd in (np.full(shape + (3,), -0.0, np.float32),
+               np.where(r.random(shape + (3,)) < 0.5, -0.0, 0.0).astype(np.float32)):
+        for sweeps in (4, 12, 13):
+            out, _ = ctx.poisson(nd, sweeps)
+            assert _bits_equal(out, oracle.poisson(nd, sweeps)), sweeps
+
+
 @pytest.mark.parametrize("speed", [0.3, 4.0])
 @pytest.mark.parametrize("shape", [(21, 30, 27), (61, 67, 71), (130, 2, 1100), (1, 33, 9), (9, 1, 33), (40, 9, 1)])
 def test_level_iterations_by_size(ctx, oracle, shape, speed):

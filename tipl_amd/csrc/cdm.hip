@@ -773,8 +773,8 @@ __global__ __launch_bounds__(kQX * kQY) void poisson2_kernel(const float* __rest
 // planes.  A sweep spoils one layer of the grown tile, so after four the
 // 8 x 8 x 8 core is exact.  Offsets are flat-index offsets as in
 // poisson2_kernel (row and plane wrap included); positions outside [0, n)
-// read 0 through the buffer's range check and are kept 0, which is the
-// reference's dropped neighbour.
+// read 0 through the buffer's range check and are kept +0.0, which is the
+// reference's dropped neighbour (x - (+0.0) is x, -0.0 included).
 // What bounds it is latency -- one round of loads, four barriers -- where
 // poisson2_kernel chains a barrier pair and a load per plane.  Twelve sweeps:
 // 44 -> 17 us at 32x32x32 and below, 45 -> 21 at 40x48x40; at 80x96x80 the
@@ -815,18 +815,23 @@ __device__ __forceinline__ void poisson4_body(const float* __restrict__ nd, cons
     float r[kCL], v[kCL];
 #pragma unroll
     for (int k = 0; k < kCL; ++k) r[k] = load(rn, k);
-    if constexpr (FIRST) {
-#pragma unroll
-        for (int k = 0; k < kCL; ++k) v[k] = r[k] * kInvD2;
-    } else {
-#pragma unroll
-        for (int k = 0; k < kCL; ++k) v[k] = load(ra, k);
-    }
-    // tiles that reach past either end of the array keep those positions 0
+    // tiles that reach past either end of the array keep those positions +0.0
     const bool ends = q0 < 0 || q0 + (kCL - 1) * (1 + w + wh) >= n;
     uint32_t inside = 0;
 #pragma unroll
     for (int k = 0; k < kCL; ++k) inside |= uint32_t(q + k * wh >= 0 && q + k * wh < n) << k;
+    if constexpr (FIRST) {
+#pragma unroll
+        for (int k = 0; k < kCL; ++k) v[k] = r[k] * kInvD2;
+        if (ends) {
+            // (the factor is negative: 0 read there has become -0.0)
+#pragma unroll
+            for (int k = 0; k < kCL; ++k) v[k] = (inside >> k) & 1u ? v[k] : 0.0f;
+        }
+    } else {
+#pragma unroll
+        for (int k = 0; k < kCL; ++k) v[k] = load(ra, k);
+    }
 #pragma unroll
     for (int s = 1; s <= kCH; ++s) {
         float(*pl)[kCL + 2][kCL] = plane[s & 1];
@@ -992,6 +997,13 @@ __global__ __launch_bounds__(kMThreads, 4) void poisson_march_kernel(const float
                 for (int j = 0; j < kMR; ++j) {
                     r[u][j] = in[u][j];
                     in[u][j] = in[u][j] * kInvD2;
+                }
+                if (ends) {
+                    // positions outside the array hold +0.0 (0 read there has
+                    // become -0.0)
+#pragma unroll
+                    for (int j = 0; j < kMR; ++j)
+                        in[u][j] = uint32_t(qm + j * w) < uint32_t(n) ? in[u][j] : 0.0f;
                 }
             }
             __syncthreads();

@@ -397,7 +397,7 @@ __global__ __launch_bounds__(kThreads2) void cost2_final_kernel(const CostReduce
 // (DPP wave shift), p -+ w the thread's other rows, or, at a wave's first and
 // last row, a value the neighbouring wave left in LDS: one barrier a sweep.
 // Offsets are flat-index offsets (row wrap included); positions outside
-// [0, n) read 0 through the buffer's range check and are kept 0, which
+// [0, n) read 0 through the buffer's range check and are kept +0.0, which
 // changes nothing where the reference drops the neighbour (x - (+0) == x).  A
 // sweep spoils one layer of the grown tile, so up to twelve leave the core
 // exact.  Latency bounds it: twelve sweeps of 109x91 in one launch of 6.4 us
@@ -442,13 +442,14 @@ __global__ __launch_bounds__(64 * kP2Waves) void poisson2d_tile_kernel(const flo
     for (int j = 0; j < kP2Rows; ++j)
         v[j] = __uint_as_float(
             __builtin_amdgcn_raw_buffer_load_b32(rs, (q0 + j * w) * 8 + int(comp) * 4, 0, 0));
-    if (first) {
-#pragma unroll
-        for (int j = 0; j < kP2Rows; ++j) v[j] = v[j] * inv_d2;
-    }
     bool in[kP2Rows];
 #pragma unroll
     for (int j = 0; j < kP2Rows; ++j) in[j] = uint32_t(q0 + j * w) < uint32_t(n);
+    if (first) {
+        // (0 read outside would become -0.0: the factor is negative)
+#pragma unroll
+        for (int j = 0; j < kP2Rows; ++j) v[j] = in[j] ? v[j] * inv_d2 : 0.0f;
+    }
     for (int s = 0; s < sweeps; ++s) {
         edge[s & 1][wv + 1][0][lane] = v[0];
         edge[s & 1][wv + 1][1][lane] = v[kP2Rows - 1];
