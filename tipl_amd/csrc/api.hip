@@ -230,8 +230,11 @@ template <>
 __device__ inline int value_key<int16_t>(int16_t v) { return int(v); }
 
 // Min and max of the input (minmax_value, used by normalize_upper_lower2).
-// (one pair of atomics a workgroup: 194 us with a pair a wave at 182x218x182
-// float, 22 now; 188 and 8 at 96x96x96 int16)
+// One pair of atomics a workgroup: 194 us with a pair a wave at 182x218x182
+// float, 22 with this; 188 and 8 at 96x96x96 int16.  With one workgroup a CU a
+// thread needs several loads in flight where memory bounds it: the upload of
+// 800x800x800 int16 from device memory took 2.14 ms with one, 1.94 when 2048
+// workgroups ran, 1.56 with four (182x218x182: 0.091 -> 0.087).
 template <class T>
 __global__ __launch_bounds__(kOnceThreads) void minmax_kernel(const T* __restrict__ in, size_t n,
                                                               int* __restrict__ mm)
@@ -240,11 +243,20 @@ __global__ __launch_bounds__(kOnceThreads) void minmax_kernel(const T* __restric
     __shared__ int part[2][kWaves];
     int lo = 0x7fffffff, hi = int(0x80000000);
     const size_t stride = size_t(gridDim.x) * blockDim.x;
-    for (size_t i = size_t(blockIdx.x) * blockDim.x + threadIdx.x; i < n; i += stride) {
-        const int k = value_key<T>(in[i]);
+    auto take = [&](T v) {
+        const int k = value_key<T>(v);
         lo = min(lo, k);
         hi = max(hi, k);
+    };
+    size_t i = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
+    for (; i + 3 * stride < n; i += 4 * stride) {
+        const T a = in[i], b = in[i + stride], c = in[i + 2 * stride], d = in[i + 3 * stride];
+        take(a);
+        take(b);
+        take(c);
+        take(d);
     }
+    for (; i < n; i += stride) take(in[i]);
     for (int off = 32; off > 0; off >>= 1) {
         lo = min(lo, __shfl_xor(lo, off, 64));
         hi = max(hi, __shfl_xor(hi, off, 64));
