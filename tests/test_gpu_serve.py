@@ -308,3 +308,27 @@ def test_cdm_batching_one_lane_full_batches(ctx, cdm_mix, monkeypatch):
     for a, b in zip(got, plain):
         _same(a, b)
     assert st["cdm_fields"] >= 3 * st["cdm_steps"]
+
+
+def test_cdm_batching_of_every_level(ctx, cdm_mix, monkeypatch):
+    """Levels of up to 2^25 voxels batched (TIPLHIP_CDM_BATCH_VOXELS): the finest
+    ones, of 262144 to 552960 voxels, take the large tiles of the gradient and of
+    the field update, beside fields on the small tiles in the same step, both
+    directions at a time.  Every iteration goes out as a batched step, and every
+    result equals the plain path's bit for bit."""
+    import tipl_amd
+    monkeypatch.setenv("TIPLHIP_CDM_BATCH_VOXELS", str(1 << 25))
+    monkeypatch.setenv("TIPLHIP_CDM_LANES", "2")
+    sel = [cdm_mix[i] for i in (5, 1, 0, 3)]
+    kw = dict(nonlinear=True, reverse=True, outputs=("f2t", "to2from", "from2to", "warped"))
+    plain = [tipl_amd.register(ctx, f, m, **kw) for f, m in sel]
+    with tipl_amd.Server(0, slots=4, hbm_budget=16 << 30) as srv:
+        ts = [srv.submit(f, m, **kw) for f, m in sel]
+        got = [srv.wait(t) for t in ts]
+        st = srv.stats()
+    for a, b in zip(got, plain):
+        _same(a, b)
+    iters = sum(p["cdm_iterations"] for p in plain)
+    print(f"batched CDM: {st['cdm_fields']} fields in {st['cdm_steps']} steps, {iters} forward iterations")
+    assert st["cdm_fields"] > iters  # the forward ones, and the reverse ones of the other direction
+    assert st["cdm_fields"] >= 1.3 * st["cdm_steps"]

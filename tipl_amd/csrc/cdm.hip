@@ -99,84 +99,28 @@ __global__ __launch_bounds__(256) void compose_kernel(const uint8_t* __restrict_
 }
 
 // ---------------------------------------------------------------------------
-// cdm_get_gradient.  'r': local linear regression of Js onto It over the
-// border-clipped 5x5x5 window (exact integer sums, then FP64 as in
-// linear_regression), gradient scaled by r2*(a*Js+b-It) where a > 0.
-// 'd': SSD gradient.  accumulate = 0 writes nd = 0 + g (a fresh field);
-// accumulate = 1 adds a further modality: nd = nd + (0 + g).
-// Per-block FP64 partial sums of the cost map go to `partials`.
+// cdm_get_gradient 'd' (SSD): the gradient of Js scaled by Js - It.
+// accumulate = 0 writes nd = 0 + g (a fresh field); accumulate = 1 adds a
+// further modality: nd = nd + (0 + g).  Per-block FP64 partial sums of the cost
+// map go to `partials`.
 // ---------------------------------------------------------------------------
-template <char TYPE>
-__global__ __launch_bounds__(256) void gradient_kernel(const uint8_t* __restrict__ Js,
-                                                       const uint8_t* __restrict__ It, FieldGeo g,
-                                                       int accumulate, float* __restrict__ nd, Lay lay,
-                                                       double* __restrict__ partials)
+__global__ __launch_bounds__(256) void gradient_d_kernel(const uint8_t* __restrict__ Js,
+                                                         const uint8_t* __restrict__ It, FieldGeo g,
+                                                         int accumulate, float* __restrict__ nd, Lay lay,
+                                                         double* __restrict__ partials)
 {
     const Vox v = this_voxel(g);
-    float3 gr = make_float3(0.0f, 0.0f, 0.0f);
     float cost = 0.0f;
     if (v.ok) {
-        const uint32_t js = Js[v.p], it = It[v.p];
-        bool active;
-        float s = 0.0f;
-        if (TYPE == 'd') {
-            const int dif = int(js) - int(it);
-            s = float(dif);
-            cost = float(dif * dif);
-            active = true;
-        } else {
-            active = false;
-            if (js != 0u && it != 0u) {
-                const int x0 = max(v.x - 2, 0), x1 = min(v.x + 2, g.w - 1);
-                const int y0 = max(v.y - 2, 0), y1 = min(v.y + 2, g.h - 1);
-                const int z0 = max(v.z - 2, 0), z1 = min(v.z + 2, g.d - 1);
-                const __amdgpu_buffer_rsrc_t rj = make_rsrc(Js, g.n);
-                const __amdgpu_buffer_rsrc_t ri = make_rsrc(It, g.n);
-                uint32_t sx = 0, sxx = 0, sy = 0, syy = 0, sxy = 0;
-                for (int zz = z0; zz <= z1; ++zz)
-                    for (int yy = y0; yy <= y1; ++yy) {
-                        const uint32_t row = uint32_t(zz) * g.wh + uint32_t(yy) * uint32_t(g.w);
-                        for (int xx = x0; xx <= x1; ++xx) {
-                            const uint32_t a = load_u8(rj, row + uint32_t(xx), 0);
-                            const uint32_t b = load_u8(ri, row + uint32_t(xx), 0);
-                            sx += a;
-                            sxx += a * a;
-                            sy += b;
-                            syy += b * b;
-                            sxy += a * b;
-                        }
-                    }
-                const double dn = double((x1 - x0 + 1) * (y1 - y0 + 1) * (z1 - z0 + 1));
-                const double mean_x = double(sx) / dn;
-                const double mean_y = double(sy) / dn;
-                const double x_var = double(sxx) / dn - mean_x * mean_x;
-                const double y_var = double(syy) / dn - mean_y * mean_y;
-                if (!(x_var == 0.0 || y_var == 0.0)) {
-                    const double cov = double(sxy) / dn - mean_x * mean_y;
-                    const float a = float(cov / x_var);
-                    if (a > 0.0f) {
-                        const float b = float(mean_y - double(a) * mean_x);
-                        const float r2 = float(cov * cov / x_var / y_var);
-                        s = float(js) * a;
-                        s = s + b;
-                        s = s - float(it);
-                        s = r2 * s;
-                        cost = -r2;
-                        active = true;
-                    }
-                }
-            }
-        }
-        if (active) {
-            // gradient_at: central differences, 0 on the first/last slab.
-            const uint32_t w = uint32_t(g.w);
-            const float gx = (v.x + 1 < g.w && v.x) ? float(int(Js[v.p + 1]) - int(Js[v.p - 1])) : 0.0f;
-            const float gy = (v.y + 1 < g.h && v.y) ? float(int(Js[v.p + w]) - int(Js[v.p - w])) : 0.0f;
-            const float gz = (v.z + 1 < g.d && v.z) ? float(int(Js[v.p + g.wh]) - int(Js[v.p - g.wh])) : 0.0f;
-            gr.x = 0.0f + gx * s;
-            gr.y = 0.0f + gy * s;
-            gr.z = 0.0f + gz * s;
-        }
+        const int dif = int(Js[v.p]) - int(It[v.p]);
+        const float s = float(dif);
+        cost = float(dif * dif);
+        // gradient_at: central differences, 0 on the first/last slab.
+        const uint32_t w = uint32_t(g.w);
+        const float gx = (v.x + 1 < g.w && v.x) ? float(int(Js[v.p + 1]) - int(Js[v.p - 1])) : 0.0f;
+        const float gy = (v.y + 1 < g.h && v.y) ? float(int(Js[v.p + w]) - int(Js[v.p - w])) : 0.0f;
+        const float gz = (v.z + 1 < g.d && v.z) ? float(int(Js[v.p + g.wh]) - int(Js[v.p - g.wh])) : 0.0f;
+        const float3 gr = make_float3(0.0f + gx * s, 0.0f + gy * s, 0.0f + gz * s);
         if (accumulate) {
             float3 o = ld_lay(nd, v.p, lay);
             o.x = o.x + gr.x;
@@ -197,7 +141,10 @@ __global__ __launch_bounds__(256) void gradient_kernel(const uint8_t* __restrict
 }
 
 // ---------------------------------------------------------------------------
-// cdm_get_gradient 'r' with the window sums done as box filters.  A block
+// cdm_get_gradient 'r': local linear regression of Js onto It over the
+// border-clipped 5x5x5 window (exact integer sums, then FP64 as in
+// linear_regression), the gradient scaled by r2*(a*Js+b-It) where a > 0, with
+// the window sums done as box filters.  accumulate and partials as above.  A block
 // owns 16 x TY x TZ outputs.  It stages the bytes of Js and It with a 2-voxel
 // halo (zero outside the volume) in LDS, aligned dwords as they lie in
 // memory, and forms the 5-tap sums along x, then y, then z, one pass over LDS
@@ -1688,8 +1635,8 @@ CostReduce launch_gradient(tiplhip_ctx* ctx, const uint8_t* Js, const uint8_t* I
 {
     uint32_t parts;
     if (type == 'd') {
-        hipLaunchKernelGGL(gradient_kernel<'d'>, tile_grid(g), dim3(kTX, kTY), 0, ctx->stream, Js,
-                           It, g, accumulate, nd, lay, partials);
+        hipLaunchKernelGGL(gradient_d_kernel, tile_grid(g), dim3(kTX, kTY), 0, ctx->stream, Js, It, g,
+                           accumulate, nd, lay, partials);
         const dim3 tg = tile_grid(g);
         parts = tg.x * tg.y * tg.z;
     } else {
