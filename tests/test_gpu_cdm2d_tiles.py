@@ -64,3 +64,24 @@ def test_cdm2d_update_across_tiles(ctx, oracle, shape, speed):
     rc, got, m = ctx.cdm2d(It, Is, ctx.cdm_param(speed=speed))
     assert ok and rc == 0 and n == m
     assert float(np.sqrt(((got - want) ** 2).sum(-1).mean())) <= 0.01
+
+
+@pytest.mark.parametrize("iterations", [2, 3, 5])
+@pytest.mark.parametrize("shape,seed", [((16, 16), 0), ((15, 17), 0), ((17, 16), 0), ((33, 31), 0), ((16, 50), 0),
+                                        ((49, 15), 0), ((2, 35), 3), ((35, 2), 20), ((1, 40), 0), ((40, 1), 0)])
+def test_cdm2d_first_iterations_bit_exact(ctx, oracle, shape, seed, iterations):
+    """The fused field update (accumulate, smooth, next composition) on images
+    around its 16 x 16 tile and narrower, and the best field taken from among the
+    rotating ones: the oracle's field after the first iterations, bit for bit, for
+    one modality and for two (which compose apart).  On these images every
+    iteration improves, so the last but one's update is in the result; images one
+    pixel wide, where no sample is inside, keep a zero field."""
+    It = image2(shape, seed, sigma=1.0, background=False)
+    Is = np.roll(It, (1, -1), (0, 1))
+    kw = dict(min_dimension=1000, max_iterations=iterations, speed=1.2)
+    for a, b in ((It, Is), ([It, It], [Is, Is])):
+        ok, want, n = oracle.cdm2(a, b, **kw)
+        rc, got, m = ctx.cdm2d(a, b, ctx.cdm_param(**kw))
+        assert ok and rc == 0 and n == m == iterations
+        assert want.any() or min(shape) == 1
+        assert _bits_equal(got, want)
