@@ -404,9 +404,10 @@ __device__ __forceinline__ void max_reduce_body(const float* __restrict__ parts,
 
 __global__ __launch_bounds__(1024) void max_reduce_kernel(const float* __restrict__ parts,
                                                           uint32_t count,
-                                                          unsigned int* __restrict__ out)
+                                                          unsigned int* __restrict__ out,
+                                                          unsigned int* __restrict__ host_out)
 {
-    max_reduce_body(parts, count, out, nullptr);
+    max_reduce_body(parts, count, out, host_out);
 }
 
 // ---------------------------------------------------------------------------
@@ -1412,10 +1413,11 @@ dim3 acc_grid(const FieldGeo& g)
 template <bool LARGE>
 __global__ __launch_bounds__(AccTile<LARGE>::kThreads, 4) void accumulate_smooth_kernel(
     const float* __restrict__ cur, const float* __restrict__ nd, Lay lay, float k, float w_6, float w_1,
-    FieldGeo g, float* __restrict__ out, const uint8_t* __restrict__ Is, uint8_t* __restrict__ Js)
+    FieldGeo g, float* __restrict__ out, const uint8_t* __restrict__ Is, uint8_t* __restrict__ Js,
+    float* __restrict__ keep)
 {
     using T = AccTile<LARGE>;
-    accumulate_smooth_body<T::kX, T::kY, T::kZ, T::kThreads, LARGE>(cur, nd, lay, k, w_6, w_1, g, out, nullptr, Is,
+    accumulate_smooth_body<T::kX, T::kY, T::kZ, T::kThreads, LARGE>(cur, nd, lay, k, w_6, w_1, g, out, keep, Is,
                                                              Js, logical_block());
 }
 
@@ -1614,28 +1616,28 @@ uint32_t block_count(const FieldGeo& g)
     return std::max(t.x * t.y * t.z, b.x * b.y * b.z);
 }
 
-void launch_compose(tiplhip_ctx* ctx, const uint8_t* Is, const float* d, const FieldGeo& g,
+void launch_compose(hipStream_t stream, const uint8_t* Is, const float* d, const FieldGeo& g,
                     uint8_t* Js)
 {
-    hipLaunchKernelGGL(compose_kernel, tile_grid(g), dim3(kTX, kTY), 0, ctx->stream, Is, d, g, Js);
+    hipLaunchKernelGGL(compose_kernel, tile_grid(g), dim3(kTX, kTY), 0, stream, Is, d, g, Js);
     TIPLHIP_CHECK(hipGetLastError());
 }
 
 // Queues the sum of a gradient's cost partials.
-void launch_cost_reduce(tiplhip_ctx* ctx, const CostReduce& r)
+void launch_cost_reduce(hipStream_t stream, const CostReduce& r)
 {
-    hipLaunchKernelGGL(cost_reduce_kernel, dim3(1), dim3(kReduceThreads), 0, ctx->stream, r);
+    hipLaunchKernelGGL(cost_reduce_kernel, dim3(1), dim3(kReduceThreads), 0, stream, r);
     TIPLHIP_CHECK(hipGetLastError());
 }
 
 // Queues the gradient; the sum of its cost partials is left to the caller.
-CostReduce launch_gradient(tiplhip_ctx* ctx, const uint8_t* Js, const uint8_t* It, const FieldGeo& g,
+CostReduce launch_gradient(hipStream_t stream, const uint8_t* Js, const uint8_t* It, const FieldGeo& g,
                      char type, int accumulate, float* nd, Lay lay, double* partials, float* cost_out,
                      float* host_cost = nullptr)
 {
     uint32_t parts;
     if (type == 'd') {
-        hipLaunchKernelGGL(gradient_d_kernel, tile_grid(g), dim3(kTX, kTY), 0, ctx->stream, Js, It, g,
+        hipLaunchKernelGGL(gradient_d_kernel, tile_grid(g), dim3(kTX, kTY), 0, stream, Js, It, g,
                            accumulate, nd, lay, partials);
         const dim3 tg = tile_grid(g);
         parts = tg.x * tg.y * tg.z;
@@ -1643,10 +1645,10 @@ CostReduce launch_gradient(tiplhip_ctx* ctx, const uint8_t* Js, const uint8_t* I
         const dim3 bg = box_grid(g);
         if (grad_large(g))
             hipLaunchKernelGGL(gradient_r_box_kernel<true>, bg, dim3(GradTile<true>::kThreads), 0,
-                               ctx->stream, Js, It, g, accumulate, nd, lay, partials);
+                               stream, Js, It, g, accumulate, nd, lay, partials);
         else
             hipLaunchKernelGGL(gradient_r_box_kernel<false>, bg, dim3(GradTile<false>::kThreads), 0,
-                               ctx->stream, Js, It, g, accumulate, nd, lay, partials);
+                               stream, Js, It, g, accumulate, nd, lay, partials);
         parts = bg.x * bg.y * bg.z;
     }
     TIPLHIP_CHECK(hipGetLastError());
@@ -1660,9 +1662,9 @@ CostReduce launch_gradient(tiplhip_ctx* ctx, const uint8_t* Js, const uint8_t* I
 // and one (the z-marching sweep).  Returns the buffer holding the result.  With maxlen, per-block maxima of the displacement length (from the
 // last launch, or a pass of their own after a four-sweep one) are reduced by
 // max_reduce_kernel.
-float* launch_poisson(tiplhip_ctx* ctx, const float* nd, float* a, float* b, const FieldGeo& g, Lay lay,
+float* launch_poisson(hipStream_t stream, const float* nd, float* a, float* b, const FieldGeo& g, Lay lay,
                       int sweeps, unsigned int* maxlen, float* maxparts,
-                      const CostReduce& cost = CostReduce{})
+                      const CostReduce& cost = CostReduce{}, unsigned int* host_maxlen = nullptr)
 {
     // a gradient's cost partials, when given, are summed by one more workgroup
     // of the first launch
@@ -1674,13 +1676,13 @@ float* launch_poisson(tiplhip_ctx* ctx, const float* nd, float* a, float* b, con
     while (done < sweeps) {
         const bool first = done == 0;
         if (poisson_whole_fits(g)) {
-            hipLaunchKernelGGL(poisson_whole_kernel, dim3(3u + extra), dim3(kWThreads), 0, ctx->stream, nd,
+            hipLaunchKernelGGL(poisson_whole_kernel, dim3(3u + extra), dim3(kWThreads), 0, stream, nd,
                                g, lay, sweeps, dst, cost);
             TIPLHIP_CHECK(hipGetLastError());
             done = sweeps;
             if (maxlen) {
                 last_blocks = std::min(kMaxLenBlocks, block_count(g));
-                hipLaunchKernelGGL(max_length_kernel, dim3(last_blocks), dim3(256), 0, ctx->stream, dst,
+                hipLaunchKernelGGL(max_length_kernel, dim3(last_blocks), dim3(256), 0, stream, dst,
                                    g.n, lay, maxparts);
                 TIPLHIP_CHECK(hipGetLastError());
             }
@@ -1691,16 +1693,16 @@ float* launch_poisson(tiplhip_ctx* ctx, const float* nd, float* a, float* b, con
             const dim3 block(kCThreads);
             const uint32_t blocks = poisson4_blocks(g);
             if (first)
-                hipLaunchKernelGGL(poisson4_kernel<true>, dim3(blocks + extra), block, 0, ctx->stream, nd,
+                hipLaunchKernelGGL(poisson4_kernel<true>, dim3(blocks + extra), block, 0, stream, nd,
                                    src, g, lay, dst, cost);
             else
-                hipLaunchKernelGGL(poisson4_kernel<false>, dim3(blocks), block, 0, ctx->stream, nd, src, g,
+                hipLaunchKernelGGL(poisson4_kernel<false>, dim3(blocks), block, 0, stream, nd, src, g,
                                    lay, dst, CostReduce{});
             TIPLHIP_CHECK(hipGetLastError());
             done += kCH;
             if (done == sweeps && maxlen) {
                 last_blocks = std::min(kMaxLenBlocks, block_count(g));
-                hipLaunchKernelGGL(max_length_kernel, dim3(last_blocks), dim3(256), 0, ctx->stream, dst,
+                hipLaunchKernelGGL(max_length_kernel, dim3(last_blocks), dim3(256), 0, stream, dst,
                                    g.n, lay, maxparts);
                 TIPLHIP_CHECK(hipGetLastError());
             }
@@ -1712,22 +1714,22 @@ float* launch_poisson(tiplhip_ctx* ctx, const float* nd, float* a, float* b, con
             const dim3 block(kMThreads);
             if (first)
                 hipLaunchKernelGGL((poisson_march_kernel<kMK, true>), dim3(mg.blocks + extra), block, 0,
-                                   ctx->stream, nd, src, g, mg, lay, dst, cost);
+                                   stream, nd, src, g, mg, lay, dst, cost);
             else
                 hipLaunchKernelGGL((poisson_march_kernel<kMK, false>), dim3(mg.blocks), block, 0,
-                                   ctx->stream, nd, src, g, mg, lay, dst, CostReduce{});
+                                   stream, nd, src, g, mg, lay, dst, CostReduce{});
             TIPLHIP_CHECK(hipGetLastError());
             done += kMK;
             if (done == sweeps && maxlen) {
                 last_blocks = std::min(kMaxLenBlocks, block_count(g));
-                hipLaunchKernelGGL(max_length_kernel, dim3(last_blocks), dim3(256), 0, ctx->stream, dst,
+                hipLaunchKernelGGL(max_length_kernel, dim3(last_blocks), dim3(256), 0, stream, dst,
                                    g.n, lay, maxparts);
                 TIPLHIP_CHECK(hipGetLastError());
             }
             std::swap(src, dst);
             continue;
         }
-        if (first && extra) launch_cost_reduce(ctx, cost);
+        if (first && extra) launch_cost_reduce(stream, cost);
         TIPLHIP_REQUIRE(lay.ps == 3u, "one- and two-sweep launches take packed fields");
         const bool pair = sweeps - done >= 2;
         const bool last = done + (pair ? 2 : 1) == sweeps && maxlen;
@@ -1735,32 +1737,32 @@ float* launch_poisson(tiplhip_ctx* ctx, const float* nd, float* a, float* b, con
             const int zq = poisson2_zq(g);
             const dim3 grid = poisson2_grid(g, zq), block(kQX, kQY);
             if (first && last)
-                hipLaunchKernelGGL((poisson2_kernel<true, true>), grid, block, 0, ctx->stream, nd, src,
+                hipLaunchKernelGGL((poisson2_kernel<true, true>), grid, block, 0, stream, nd, src,
                                    g, zq, dst, maxparts);
             else if (first)
-                hipLaunchKernelGGL((poisson2_kernel<true, false>), grid, block, 0, ctx->stream, nd,
+                hipLaunchKernelGGL((poisson2_kernel<true, false>), grid, block, 0, stream, nd,
                                    src, g, zq, dst, maxparts);
             else if (last)
-                hipLaunchKernelGGL((poisson2_kernel<false, true>), grid, block, 0, ctx->stream, nd,
+                hipLaunchKernelGGL((poisson2_kernel<false, true>), grid, block, 0, stream, nd,
                                    src, g, zq, dst, maxparts);
             else
-                hipLaunchKernelGGL((poisson2_kernel<false, false>), grid, block, 0, ctx->stream, nd,
+                hipLaunchKernelGGL((poisson2_kernel<false, false>), grid, block, 0, stream, nd,
                                    src, g, zq, dst, maxparts);
             last_blocks = grid.x * grid.y * grid.z;
             done += 2;
         } else {
             const dim3 grid = poisson_grid(g), block(kTX, kPTY);
             if (first && last)
-                hipLaunchKernelGGL((poisson_zm_kernel<true, true>), grid, block, 0, ctx->stream, nd,
+                hipLaunchKernelGGL((poisson_zm_kernel<true, true>), grid, block, 0, stream, nd,
                                    src, g, dst, maxparts);
             else if (first)
-                hipLaunchKernelGGL((poisson_zm_kernel<true, false>), grid, block, 0, ctx->stream, nd,
+                hipLaunchKernelGGL((poisson_zm_kernel<true, false>), grid, block, 0, stream, nd,
                                    src, g, dst, maxparts);
             else if (last)
-                hipLaunchKernelGGL((poisson_zm_kernel<false, true>), grid, block, 0, ctx->stream, nd,
+                hipLaunchKernelGGL((poisson_zm_kernel<false, true>), grid, block, 0, stream, nd,
                                    src, g, dst, maxparts);
             else
-                hipLaunchKernelGGL((poisson_zm_kernel<false, false>), grid, block, 0, ctx->stream, nd,
+                hipLaunchKernelGGL((poisson_zm_kernel<false, false>), grid, block, 0, stream, nd,
                                    src, g, dst, maxparts);
             last_blocks = grid.x * grid.y * grid.z;
             done += 1;
@@ -1769,26 +1771,28 @@ float* launch_poisson(tiplhip_ctx* ctx, const float* nd, float* a, float* b, con
         std::swap(src, dst);
     }
     if (maxlen) {
-        hipLaunchKernelGGL(max_reduce_kernel, dim3(1), dim3(1024), 0, ctx->stream, maxparts,
-                           last_blocks, maxlen);
+        hipLaunchKernelGGL(max_reduce_kernel, dim3(1), dim3(1024), 0, stream, maxparts,
+                           last_blocks, maxlen, host_maxlen);
         TIPLHIP_CHECK(hipGetLastError());
     }
     return src;
 }
 
-void launch_accumulate(tiplhip_ctx* ctx, const float* cur, const float* nd, Lay lay, float k,
+void launch_accumulate(hipStream_t stream, const float* cur, const float* nd, Lay lay, float k,
                        const FieldGeo& g, float* out, Lay out_lay)
 {
-    hipLaunchKernelGGL(accumulate_kernel, tile_grid(g), dim3(kTX, kTY), 0, ctx->stream, cur, nd, lay, k, g,
+    hipLaunchKernelGGL(accumulate_kernel, tile_grid(g), dim3(kTX, kTY), 0, stream, cur, nd, lay, k, g,
                        out, out_lay);
     TIPLHIP_CHECK(hipGetLastError());
 }
 
-void launch_smooth(tiplhip_ctx* ctx, const float* d, float* dd, float smoothing, const FieldGeo& g)
+// cdm_smooth's weight of a neighbour.
+inline float smooth_w6(float smoothing) { return smoothing / float(2.0f * 3.0f); }
+
+void launch_smooth(hipStream_t stream, const float* d, float* dd, float smoothing, const FieldGeo& g)
 {
-    const float w_6 = smoothing / float(2.0f * 3.0f);
-    const float w_1 = 1.0f - smoothing;
-    hipLaunchKernelGGL(smooth_kernel, tile_grid(g), dim3(kTX, kTY), 0, ctx->stream, d, dd, w_6, w_1, g);
+    const float w_6 = smooth_w6(smoothing), w_1 = 1.0f - smoothing;
+    hipLaunchKernelGGL(smooth_kernel, tile_grid(g), dim3(kTX, kTY), 0, stream, d, dd, w_6, w_1, g);
     TIPLHIP_CHECK(hipGetLastError());
 }
 
@@ -1797,30 +1801,30 @@ void launch_smooth(tiplhip_ctx* ctx, const float* d, float* dd, float smoothing,
 // set; returns whether it did.  That kernel addresses the packed field in 32
 // bits: a field of 2^32 bytes and more takes the two kernels it replaces, whose
 // addresses are 64 bits wide, and nd (packed there) is overwritten.
-bool launch_accumulate_smooth(tiplhip_ctx* ctx, const float* cur, float* nd, Lay lay, float k,
-                              float smoothing, const FieldGeo& g, float* out, const uint8_t* Is, uint8_t* Js)
+bool launch_accumulate_smooth(hipStream_t stream, const float* cur, float* nd, Lay lay, float k,
+                              float smoothing, const FieldGeo& g, float* out, const uint8_t* Is, uint8_t* Js,
+                              float* keep = nullptr)
 {
     if (!field_fits_32(g.n)) {
-        launch_accumulate(ctx, cur, nd, lay, k, g, nd, lay);
-        launch_smooth(ctx, nd, out, smoothing, g);
+        launch_accumulate(stream, cur, nd, lay, k, g, nd, lay);
+        launch_smooth(stream, nd, out, smoothing, g);
         return false;
     }
-    const float w_6 = smoothing / float(2.0f * 3.0f);
-    const float w_1 = 1.0f - smoothing;
+    const float w_6 = smooth_w6(smoothing), w_1 = 1.0f - smoothing;
     if (acc_large(g))
         hipLaunchKernelGGL(accumulate_smooth_kernel<true>, acc_grid(g), dim3(AccTile<true>::kThreads), 0,
-                           ctx->stream, cur, nd, lay, k, w_6, w_1, g, out, Is, Js);
+                           stream, cur, nd, lay, k, w_6, w_1, g, out, Is, Js, keep);
     else
         hipLaunchKernelGGL(accumulate_smooth_kernel<false>, acc_grid(g), dim3(AccTile<false>::kThreads), 0,
-                           ctx->stream, cur, nd, lay, k, w_6, w_1, g, out, Is, Js);
+                           stream, cur, nd, lay, k, w_6, w_1, g, out, Is, Js, keep);
     TIPLHIP_CHECK(hipGetLastError());
     return Js != nullptr;
 }
 
-void launch_upsample(tiplhip_ctx* ctx, const float* in, const FieldGeo& gi, const FieldGeo& go,
+void launch_upsample(hipStream_t stream, const float* in, const FieldGeo& gi, const FieldGeo& go,
                      float* out)
 {
-    hipLaunchKernelGGL(upsample_kernel, tile_grid(go), dim3(kTX, kTY), 0, ctx->stream, in, gi, go, out);
+    hipLaunchKernelGGL(upsample_kernel, tile_grid(go), dim3(kTX, kTY), 0, stream, in, gi, go, out);
     TIPLHIP_CHECK(hipGetLastError());
 }
 
@@ -1876,10 +1880,10 @@ struct CdmJob : GateSlot {
     // set) or plain copies, then the iteration body on cur
     bool smooth = false;
     const float* s_src = nullptr;
-    const float* s_nd = nullptr;
+    float* s_nd = nullptr;
     float* s_out = nullptr;
     float* s_keep = nullptr;
-    float k = 0.0f, w_6 = 0.0f, w_1 = 0.0f;
+    float k = 0.0f, smoothing = 0.0f;
     bool copy_best = false;   // without smoothing: best <- cur, then
     bool restore = false;     // cur <- best
     bool need_theta = false;  // the last Jacobi launch forms max_len
@@ -1899,6 +1903,25 @@ void set_grids(CdmStep& st, CdmJob* const* J, int n, dim3 CdmJob::*grid)
         total = uint32_t(t);
     }
     st.total = total;
+}
+
+// The step of a job that is alone in its batch (its copies are queued): the
+// launches cdm_level makes, on packed fields.  Three to five of them instead of
+// nine, whose sweeps take half the time (17 against 44 us at 32x32x32); most
+// batches have one field unless the slots outnumber the lanes several times.
+void launch_cdm_step_alone(hipStream_t stream, CdmJob& j)
+{
+    const Lay lay = packed_layout();
+    if (j.smooth)
+        launch_accumulate_smooth(stream, j.s_src, j.s_nd, lay, j.k, j.smoothing, j.g, j.s_out, j.Is, j.Js,
+                                 j.s_keep);
+    else
+        launch_compose(stream, j.Is, j.cur, j.g, j.Js);
+    const CostReduce reduce =
+        launch_gradient(stream, j.Js, j.It, j.g, 'r', 0, j.nd, lay, j.partials, j.d_cost, j.h_cost);
+    const float* solved = launch_poisson(stream, j.nd, j.pa, j.pb, j.g, lay, 12,
+                                         j.need_theta ? j.d_maxlen : nullptr, j.maxparts, reduce, j.h_maxlen);
+    if (solved != j.pa) std::swap(j.pa, j.pb);  // (the next step reads pa)
 }
 
 // Queues one step of every job in J (at most kMaxSegs) on `stream`, in the
@@ -1922,6 +1945,10 @@ void launch_cdm_steps(hipStream_t stream, CdmJob* const* J, int n)
         if (j.restore)
             TIPLHIP_CHECK(hipMemcpyAsync(j.cur, j.best, fb, hipMemcpyDeviceToDevice, stream));
     }
+    if (n == 1) {
+        launch_cdm_step_alone(stream, *J[0]);
+        return;
+    }
     // the field update of the jobs that have one, compose_displacement
     // included; one launch per tile shape among them
     for (const bool large : {false, true}) {
@@ -1937,14 +1964,14 @@ void launch_cdm_steps(hipStream_t stream, CdmJob* const* J, int n)
             const CdmJob& j = *sm[s];
             st.g[s] = j.g;
             st.cur[s] = j.s_src;
-            st.nd[s] = const_cast<float*>(j.s_nd);
+            st.nd[s] = j.s_nd;
             st.dst[s] = j.s_out;
             st.keep[s] = j.s_keep;
             st.Is[s] = j.Is;
             st.Js[s] = j.Js;
             st.k[s] = j.k;
-            st.w_6[s] = j.w_6;
-            st.w_1[s] = j.w_1;
+            st.w_6[s] = smooth_w6(j.smoothing);
+            st.w_1[s] = 1.0f - j.smoothing;
         }
         if (large)
             hipLaunchKernelGGL(accumulate_smooth_seg_kernel<true>, dim3(st.total),
@@ -2055,19 +2082,19 @@ void launch_cdm_steps(hipStream_t stream, CdmJob* const* J, int n)
 // (at most kMaxSegs fields a batch, kGatherUs); a job keeps the lane it
 // joined (the one with the fewest members), whose stream orders its steps.
 // Levels above max_voxels run unbatched on their owner's stream: a batch is
-// held to the pace of its largest field, and only a field of its own stream
-// takes the four-sweep Jacobi launches and the planar gradient field.
-// Measured on 32 uneven affine+CDM pairs served on 16 slots with 4 lanes
-// (pairs/s): every level batched 79.6-80.5, up to 2^18 voxels 83.7-87.3, up to
-// 4096 87.7-91.3, none 86.7-88.6; with four-sweep launches in the batched
-// steps 78.5-79.9.  The line is where a field alone would march.  Lanes, while every level was batched and took
-// two sweeps a launch alone as well: 1 lane 56.1-58.0, 2 62.3-64.3, 3
-// 64.6-65.6, 4 65.6-68.8, 6 62.3, 8 61.6-61.9, 16 58.9-61.3, unbatched
-// 57.6-61.2.
+// held to the pace of its largest field, and only a field of its own stream has
+// the planar gradient field of the marched sweeps, which larger levels take.
+// Measured on 32 uneven affine+CDM pairs (pairs/s, medians of six runs, which
+// spread by 3 to 5), unbatched, then up to 2^18 voxels on 2, 3 and 4 lanes:
+// 4 slots 71.0, 70.4, 70.6, 71.9; 8 slots 85.8, 84.8, 85.0, 84.2; 16 slots
+// 89.7, 90.3, 91.1, 89.5; 32 slots 85.6, 84.2, 85.2, 85.5; 6 slots with both
+// directions 53.4, 53.7, 55.2, 54.3.  Lines at 4096 and 70000 voxels on 16 slots
+// and 4 lanes: 91.3, 88.4 (2^18: 91.2).  While a batch of one field took the
+// batch's launches too, 4 lanes gave 64.4 on 4 slots, 78.0 on 8 and 87.6 on 16.
 class CdmBatcher {
 public:
     static constexpr int kGatherUs = 300;
-    static constexpr int kDefaultLanes = 4;
+    static constexpr int kDefaultLanes = 3;
     static constexpr size_t kDefaultMaxVoxels = size_t(1) << 18;
 
     CdmBatcher(int device, int lanes, size_t max_voxels) : device_(device), max_voxels_(max_voxels)
@@ -2308,8 +2335,7 @@ bool cdm_iterate_batched(CdmRun& run, const uint8_t* It, const uint8_t* Is, cons
             job.s_nd = job.pa;
             job.s_out = job.pb;
             job.k = k;
-            job.w_6 = cur_smoothing / float(2.0f * 3.0f);
-            job.w_1 = 1.0f - cur_smoothing;
+            job.smoothing = cur_smoothing;
             float* spare = job.pb;
             job.pb = job.pa;
             job.pa = job.cur;
@@ -2386,7 +2412,7 @@ bool cdm_level(CdmRun& run, const std::vector<const uint8_t*>& It,
         DevMem rbest(ctx, sizeof(float) * 3 * rn);
         zero(ctx, rbest.p, sizeof(float) * 3 * rn);
         if (!cdm_level(run, rIt, rIs, rd, rbest.as<float>(), resolution / 2.0f)) return false;
-        launch_upsample(ctx, rbest.as<float>(), field_geo(rd), g, best_d);
+        launch_upsample(ctx->stream, rbest.as<float>(), field_geo(rd), g, best_d);
         if (resolution > 1.0f) return true;
     }
     if (run.stopped) return true;
@@ -2442,16 +2468,16 @@ bool cdm_level(CdmRun& run, const std::vector<const uint8_t*>& It,
         CostReduce reduce;
         for (int i = 0; i < run.nmod; ++i) {
             // (of a single modality the field update has composed Js)
-            if (!composed) launch_compose(ctx, Is[size_t(i)], cur, g, Js.as<uint8_t>());
+            if (!composed) launch_compose(ctx->stream, Is[size_t(i)], cur, g, Js.as<uint8_t>());
             const char type = run.param.gradient_type[std::min(i, 7)] == 'd' ? 'd' : 'r';
-            reduce = launch_gradient(ctx, Js.as<uint8_t>(), It[size_t(i)], g, type, i > 0 ? 1 : 0,
+            reduce = launch_gradient(ctx->stream, Js.as<uint8_t>(), It[size_t(i)], g, type, i > 0 ? 1 : 0,
                                      nd.as<float>(), lay, partials.as<double>(), d_cost + i, h_cost + i);
             // the last modality's sum rides on the first Poisson launch
-            if (i + 1 < run.nmod) launch_cost_reduce(ctx, reduce);
+            if (i + 1 < run.nmod) launch_cost_reduce(ctx->stream, reduce);
         }
         composed = false;
         const bool need_theta = theta == 0.0f;
-        float* solved = launch_poisson(ctx, nd.as<float>(), pa, pb, g, lay, 12,
+        float* solved = launch_poisson(ctx->stream, nd.as<float>(), pa, pb, g, lay, 12,
                                        need_theta ? d_maxlen : nullptr, maxparts.as<float>(), reduce);
         wait_for_slots(static_cast<const volatile uint32_t*>(slots), size_t(run.nmod), kCostPending,
                        std::chrono::microseconds(kCostSpinUs),
@@ -2490,7 +2516,7 @@ bool cdm_level(CdmRun& run, const std::vector<const uint8_t*>& It,
         // accumulated field is then unused), as in the reference
         if (cur_smoothing != 0.0f) {
             float* spare = solved == pa ? pb : pa;
-            composed = launch_accumulate_smooth(ctx, cur, solved, lay, k, cur_smoothing, g, spare, Is[0],
+            composed = launch_accumulate_smooth(ctx->stream, cur, solved, lay, k, cur_smoothing, g, spare, Is[0],
                                                 run.nmod == 1 ? Js.as<uint8_t>() : nullptr);
             pa = cur == best ? spare_field : cur;
             pb = solved;
@@ -2531,7 +2557,7 @@ void cdm_fixed(CdmRun& run, const std::vector<const uint8_t*>& It,
         }
         cdm_fixed(run, rIt, rIs, rd, rfield.as<float>(), levels - 1);
         zero(ctx, field, fb);  // far-edge slabs of the upsampled field stay 0
-        launch_upsample(ctx, rfield.as<float>(), field_geo(rd), g, field);
+        launch_upsample(ctx->stream, rfield.as<float>(), field_geo(rd), g, field);
     } else {
         zero(ctx, field, fb);
     }
@@ -2551,14 +2577,14 @@ void cdm_fixed(CdmRun& run, const std::vector<const uint8_t*>& It,
         }
         ++run.iterations;
         for (int i = 0; i < run.nmod; ++i) {
-            launch_compose(ctx, Is[size_t(i)], field, g, Js.as<uint8_t>());
+            launch_compose(ctx->stream, Is[size_t(i)], field, g, Js.as<uint8_t>());
             const char type = run.param.gradient_type[std::min(i, 7)] == 'd' ? 'd' : 'r';
             // (the fixed schedule does not look at the cost)
-            launch_gradient(ctx, Js.as<uint8_t>(), It[size_t(i)], g, type, i > 0 ? 1 : 0,
+            launch_gradient(ctx->stream, Js.as<uint8_t>(), It[size_t(i)], g, type, i > 0 ? 1 : 0,
                             nd.as<float>(), lay, partials.as<double>(), d_cost + i);
         }
         const bool need_theta = theta == 0.0f;
-        float* solved = launch_poisson(ctx, nd.as<float>(), pa.as<float>(), pb.as<float>(), g, lay, 12,
+        float* solved = launch_poisson(ctx->stream, nd.as<float>(), pa.as<float>(), pb.as<float>(), g, lay, 12,
                                        need_theta ? d_maxlen : nullptr, maxparts.as<float>());
         if (need_theta) {
             unsigned int bits = 0;
@@ -2569,13 +2595,13 @@ void cdm_fixed(CdmRun& run, const std::vector<const uint8_t*>& It,
         float* spare = solved == pa.as<float>() ? pb.as<float>() : pa.as<float>();
         // (the gaussian reads a planar field where it marches four rounds a launch)
         const bool planar = gaussian_takes_planar(dim, unsigned(run.param.field_bandwidth));
-        launch_accumulate(ctx, field, solved, lay, run.param.speed / theta, g, spare,
+        launch_accumulate(ctx->stream, field, solved, lay, run.param.speed / theta, g, spare,
                           planar ? Lay{1u, g.n} : packed_layout());
         if (run.param.field_bandwidth > 0) {
             launch_gaussian_to(ctx, spare, field, solved, dim, 3, unsigned(run.param.field_bandwidth), planar);
         } else if (run.param.smoothing != 0.0f) {
             // cdm_smooth with weight 0 leaves the field untouched, as in the reference
-            launch_smooth(ctx, spare, field, run.param.smoothing, g);
+            launch_smooth(ctx->stream, spare, field, run.param.smoothing, g);
         }
     }
     TIPLHIP_CHECK(hipStreamSynchronize(ctx->stream));
@@ -2710,7 +2736,7 @@ int tiplhip_compose_displacement(tiplhip_ctx* ctx, const uint8_t* Is, const int 
         DevMem dI(ctx, g.n), dD(ctx, sizeof(float) * 3 * g.n), dJ(ctx, g.n);
         TIPLHIP_CHECK(hipMemcpyAsync(dI.p, Is, g.n, hipMemcpyHostToDevice, ctx->stream));
         TIPLHIP_CHECK(hipMemcpyAsync(dD.p, d, sizeof(float) * 3 * g.n, hipMemcpyHostToDevice, ctx->stream));
-        launch_compose(ctx, dI.as<uint8_t>(), dD.as<float>(), g, dJ.as<uint8_t>());
+        launch_compose(ctx->stream, dI.as<uint8_t>(), dD.as<float>(), g, dJ.as<uint8_t>());
         TIPLHIP_CHECK(hipMemcpyAsync(Js, dJ.p, g.n, hipMemcpyDeviceToHost, ctx->stream));
         TIPLHIP_CHECK(hipStreamSynchronize(ctx->stream));
     });
@@ -2730,7 +2756,7 @@ int tiplhip_cdm_gradient(tiplhip_ctx* ctx, const uint8_t* Js, const uint8_t* It,
         DevMem part(ctx, sizeof(double) * block_count(g)), dc(ctx, sizeof(float));
         TIPLHIP_CHECK(hipMemcpyAsync(dJ.p, Js, g.n, hipMemcpyHostToDevice, ctx->stream));
         TIPLHIP_CHECK(hipMemcpyAsync(dI.p, It, g.n, hipMemcpyHostToDevice, ctx->stream));
-        launch_cost_reduce(ctx, launch_gradient(ctx, dJ.as<uint8_t>(), dI.as<uint8_t>(), g, type, 0,
+        launch_cost_reduce(ctx->stream, launch_gradient(ctx->stream, dJ.as<uint8_t>(), dI.as<uint8_t>(), g, type, 0,
                                                 dN.as<float>(), packed_layout(), part.as<double>(),
                                                 dc.as<float>()));
         TIPLHIP_CHECK(hipMemcpyAsync(new_d, dN.p, sizeof(float) * 3 * g.n, hipMemcpyDeviceToHost, ctx->stream));
@@ -2754,7 +2780,7 @@ int tiplhip_cdm_poisson(tiplhip_ctx* ctx, float* new_d, const int dim[3], int sw
         const size_t fb = sizeof(float) * 3 * g.n;
         DevMem dN(ctx, fb), a(ctx, fb), b(ctx, fb), ml(ctx, sizeof(unsigned int)), mp(ctx, sizeof(float) * block_count(g));
         TIPLHIP_CHECK(hipMemcpyAsync(dN.p, new_d, fb, hipMemcpyHostToDevice, ctx->stream));
-        float* out = launch_poisson(ctx, dN.as<float>(), a.as<float>(), b.as<float>(), g, packed_layout(), sweeps,
+        float* out = launch_poisson(ctx->stream, dN.as<float>(), a.as<float>(), b.as<float>(), g, packed_layout(), sweeps,
                                     ml.as<unsigned int>(), mp.as<float>());
         TIPLHIP_CHECK(hipMemcpyAsync(new_d, out, fb, hipMemcpyDeviceToHost, ctx->stream));
         unsigned int bits = 0;
@@ -2777,7 +2803,7 @@ int tiplhip_accumulate_displacement(tiplhip_ctx* ctx, const float* cur, float* n
         DevMem dC(ctx, fb), dN(ctx, fb);
         TIPLHIP_CHECK(hipMemcpyAsync(dC.p, cur, fb, hipMemcpyHostToDevice, ctx->stream));
         TIPLHIP_CHECK(hipMemcpyAsync(dN.p, new_d, fb, hipMemcpyHostToDevice, ctx->stream));
-        launch_accumulate(ctx, dC.as<float>(), dN.as<float>(), packed_layout(), scale, g, dN.as<float>(),
+        launch_accumulate(ctx->stream, dC.as<float>(), dN.as<float>(), packed_layout(), scale, g, dN.as<float>(),
                           packed_layout());
         TIPLHIP_CHECK(hipMemcpyAsync(new_d, dN.p, fb, hipMemcpyDeviceToHost, ctx->stream));
         TIPLHIP_CHECK(hipStreamSynchronize(ctx->stream));
@@ -2796,7 +2822,7 @@ int tiplhip_cdm_smooth(tiplhip_ctx* ctx, const float* d, float* dd, const int di
         const size_t fb = sizeof(float) * 3 * g.n;
         DevMem dD(ctx, fb), dO(ctx, fb);
         TIPLHIP_CHECK(hipMemcpyAsync(dD.p, d, fb, hipMemcpyHostToDevice, ctx->stream));
-        launch_smooth(ctx, dD.as<float>(), dO.as<float>(), smoothing, g);
+        launch_smooth(ctx->stream, dD.as<float>(), dO.as<float>(), smoothing, g);
         TIPLHIP_CHECK(hipMemcpyAsync(dd, dO.p, fb, hipMemcpyDeviceToHost, ctx->stream));
         TIPLHIP_CHECK(hipStreamSynchronize(ctx->stream));
     });
@@ -2814,7 +2840,7 @@ int tiplhip_upsample_field(tiplhip_ctx* ctx, const float* in, const int in_dim[3
         const FieldGeo gi = field_geo(in_dim), go = field_geo(out_dim);
         DevMem dI(ctx, sizeof(float) * 3 * gi.n), dO(ctx, sizeof(float) * 3 * go.n);
         TIPLHIP_CHECK(hipMemcpyAsync(dI.p, in, sizeof(float) * 3 * gi.n, hipMemcpyHostToDevice, ctx->stream));
-        launch_upsample(ctx, dI.as<float>(), gi, go, dO.as<float>());
+        launch_upsample(ctx->stream, dI.as<float>(), gi, go, dO.as<float>());
         TIPLHIP_CHECK(hipMemcpyAsync(out, dO.p, sizeof(float) * 3 * go.n, hipMemcpyDeviceToHost, ctx->stream));
         TIPLHIP_CHECK(hipStreamSynchronize(ctx->stream));
     });
