@@ -605,9 +605,10 @@ __global__ __launch_bounds__(MiTraits<BINS>::kThreads) void mi_hist_one_kernel(
 // float(BINS*BINS) and negated (reg/linear.hpp:201).  to_h comes from the
 // histogram kernel.  Each candidate's bins are split into slices of 4096
 // (16 per thread), one workgroup per slice, so even a single candidate
-// fills many CUs; the slice sums of 256-bin histograms are combined by
-// mi_entropy_final_kernel in a fixed tree (a 64-bin histogram is one slice).  Each wave first packs its non-zero bins (a ballot and a
-// lane rank per bin slot) so the FP64 log terms run on dense lanes only.
+// fills many CUs; the slice sums of 256-bin histograms are combined in a fixed
+// tree by mi_entropy_final_kernel, or by the host (a 64-bin histogram is one
+// slice).  Each wave first packs its non-zero bins (a ballot and a lane rank per
+// bin slot) so the FP64 log terms run on dense lanes only.
 // The result is deterministic (the reference's sum is sequential in
 // row-major order; the two agree to rounding).
 constexpr int kEntropyThreads = 256;

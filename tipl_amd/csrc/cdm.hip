@@ -1103,8 +1103,9 @@ __global__ __launch_bounds__(256) void max_length_kernel(const float* __restrict
 
 // ---------------------------------------------------------------------------
 // new_d *= k, then accumulate_displacement(cur, new_d) into out (which may be
-// new_d itself where that is packed): new(x) = m(x + new(x)) - x with m(y) = cur(y) + y by trilinear
-// interpolation; cur(x) where new(x) == 0 or the sample is outside.
+// new_d itself where that is packed): new(x) = m(x + new(x)) - x with
+// m(y) = cur(y) + y by trilinear interpolation; cur(x) where new(x) == 0 or the
+// sample is outside.
 // ---------------------------------------------------------------------------
 // The accumulated displacement at voxel p = (x, y, z).
 __device__ inline float3 accumulated(const float* __restrict__ cur, const float* __restrict__ nd,
@@ -1164,9 +1165,10 @@ __device__ inline float3 ld3_rsrc(__amdgpu_buffer_rsrc_t r, uint32_t p)
 // compose_displacement in one pass: out = smooth(acc), acc = the accumulated
 // field of accumulate_kernel, and Js(x) = Is(x + out(x)) where Js is given.
 // A block owns TX x TY x TZ outputs, evaluates acc on them and on the six
-// faces around them, keeps it in LDS, and smooths behind one barrier.  Offsets are flat-index offsets:
-// a cell past the end of its row or plane is the next row's or plane's first
-// voxel, as smooth's neighbours p-+1, p-+w, p-+wh are.  A position outside
+// faces around them, keeps it in LDS, and smooths behind one barrier.  Offsets
+// are flat-index offsets: a cell past the end of its row or plane is the next
+// row's or plane's first voxel, as smooth's neighbours p-+1, p-+w, p-+wh are.
+// Byte offsets into the field have 32 bits (field_fits_32).  A position outside
 // [0, n) holds +0.0, which adds nothing to the neighbour sum (that sum starts
 // at +0.0 and is never -0.0), as the reference drops it.  HBM traffic per
 // voxel: new_d read, cur gathered, out written (36 B), Is gathered and Js
@@ -1657,10 +1659,11 @@ CostReduce launch_gradient(hipStream_t stream, const uint8_t* Js, const uint8_t*
 
 // `sweeps` Jacobi sweeps: all in one launch for the smallest volumes
 // (poisson_whole_kernel), four per launch else (poisson4_kernel for small
-// volumes, poisson_march_kernel for large ones); of a packed field also the remainder,
-// and all of a volume whose byte offsets pass 2^31, by two (poisson2_kernel)
-// and one (the z-marching sweep).  Returns the buffer holding the result.  With maxlen, per-block maxima of the displacement length (from the
-// last launch, or a pass of their own after a four-sweep one) are reduced by
+// volumes, poisson_march_kernel for large ones); of a packed field also the
+// remainder, and all of a volume whose byte offsets pass 2^31, by two
+// (poisson2_kernel) and one (the z-marching sweep).  Returns the buffer holding
+// the result.  With maxlen, per-block maxima of the displacement length (from
+// the last launch, or a pass of their own after a four-sweep one) are reduced by
 // max_reduce_kernel.
 float* launch_poisson(hipStream_t stream, const float* nd, float* a, float* b, const FieldGeo& g, Lay lay,
                       int sweeps, unsigned int* maxlen, float* maxparts,

@@ -5,11 +5,12 @@
 // 2^(-2*bandwidth*3) (bandwidth b has variance b/2 per axis).  Each pass of
 // the reference writes a float array, so every intermediate value is rounded
 // to float; one launch here runs one whole round (three passes), or four
-// (gaussian_march_kernel), and keeps those roundings.  In the single round the x pass of a tile (with a one-voxel halo) is written to
-// LDS, the y pass of it stays in registers, and the z pass combines three
-// consecutive y-pass planes while the block marches along z.  HBM traffic per
-// round is one read (plus halo) and one write of the image instead of the
-// reference's three of each.
+// (gaussian_march_kernel), and keeps those roundings.  In the single round the
+// x pass of a tile (with a one-voxel halo) is written to LDS, the y pass of it
+// stays in registers, and the z pass combines three consecutive y-pass planes
+// while the block marches along z.  HBM traffic per launch is one read (plus
+// halo) and one write of the image instead of the reference's three of each a
+// round.
 //
 // Works on float images of CH interleaved channels: CH = 1 for a scalar
 // volume, CH = 3 for a vector<3,float> displacement field.
