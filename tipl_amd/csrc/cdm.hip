@@ -910,9 +910,10 @@ __global__ __launch_bounds__(kMThreads, 4) void poisson_march_kernel(const float
         for (int j = 0; j < kMR; ++j)
             dst[j] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rs, at + j * row, 0, 0));
     };
-    const int lo = y0 * w + x0 + (z0 - K) * wh;
-    const int hi = (y0 + kMRows - 1) * w + x0 + 63 + (z1 - 1 + K) * wh;
-    const bool ends = lo < 0 || hi >= n;
+    // the tile's first and last position in plane 0, and whether any of its
+    // planes reaches past the array
+    const int first_q = y0 * w + x0, last_q = (y0 + kMRows - 1) * w + x0 + 63;
+    const bool ends = first_q + (z0 - K) * wh < 0 || last_q + (z1 - 1 + K) * wh >= n;
     float in[kMUnroll][kMR], r[kMUnroll][kMR], st[K][3][kMR];
 #pragma unroll
     for (int t = 1; t < K; ++t)
@@ -946,7 +947,7 @@ __global__ __launch_bounds__(kMThreads, 4) void poisson_march_kernel(const float
                     r[u][j] = in[u][j];
                     in[u][j] = in[u][j] * kInvD2;
                 }
-                if (ends) {
+                if (ends && (first_q + m * wh < 0 || last_q + m * wh >= n)) {
                     // positions outside the array hold +0.0 (0 read there has
                     // become -0.0)
 #pragma unroll

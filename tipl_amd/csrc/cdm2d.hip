@@ -407,9 +407,10 @@ constexpr int kP2Halo = 12, kP2Rows = 4, kP2Waves = 16, kP2Side = kP2Rows * kP2W
 constexpr int kP2Core = kP2Side - 2 * kP2Halo;
 static_assert(kP2Side == 64, "a tile row is one wave");
 
+template <bool FIRST>
 __global__ __launch_bounds__(64 * kP2Waves) void poisson2d_tile_kernel(const float* __restrict__ nd,
                                                                        const float* __restrict__ src,
-                                                                       Geo2 g, int first, int sweeps,
+                                                                       Geo2 g, int sweeps,
                                                                        float* __restrict__ dst,
                                                                        const CostReduce2 cost)
 {
@@ -432,23 +433,24 @@ __global__ __launch_bounds__(64 * kP2Waves) void poisson2d_tile_kernel(const flo
     const int w = g.w, n = int(g.n);
     const int q0 = (y0 + wv * kP2Rows) * w + x0 + lane;
     const __amdgpu_buffer_rsrc_t rn = make_rsrc(nd, g.n * 8u);
-    const __amdgpu_buffer_rsrc_t rs = make_rsrc(first ? nd : src, g.n * 8u);
     float r[kP2Rows], v[kP2Rows];
 #pragma unroll
     for (int j = 0; j < kP2Rows; ++j)
         r[j] = __uint_as_float(
             __builtin_amdgcn_raw_buffer_load_b32(rn, (q0 + j * w) * 8 + int(comp) * 4, 0, 0));
-#pragma unroll
-    for (int j = 0; j < kP2Rows; ++j)
-        v[j] = __uint_as_float(
-            __builtin_amdgcn_raw_buffer_load_b32(rs, (q0 + j * w) * 8 + int(comp) * 4, 0, 0));
     bool in[kP2Rows];
 #pragma unroll
     for (int j = 0; j < kP2Rows; ++j) in[j] = uint32_t(q0 + j * w) < uint32_t(n);
-    if (first) {
+    if constexpr (FIRST) {
         // (0 read outside would become -0.0: the factor is negative)
 #pragma unroll
-        for (int j = 0; j < kP2Rows; ++j) v[j] = in[j] ? v[j] * inv_d2 : 0.0f;
+        for (int j = 0; j < kP2Rows; ++j) v[j] = in[j] ? r[j] * inv_d2 : 0.0f;
+    } else {
+        const __amdgpu_buffer_rsrc_t rs = make_rsrc(src, g.n * 8u);
+#pragma unroll
+        for (int j = 0; j < kP2Rows; ++j)
+            v[j] = __uint_as_float(
+                __builtin_amdgcn_raw_buffer_load_b32(rs, (q0 + j * w) * 8 + int(comp) * 4, 0, 0));
     }
     for (int s = 0; s < sweeps; ++s) {
         edge[s & 1][wv + 1][0][lane] = v[0];
@@ -762,9 +764,13 @@ float* launch_poisson2(tiplhip_ctx* ctx, const float* nd, float* a, float* b, co
             const CostReduce2 c = done == 0 ? cost : CostReduce2{};
             const uint32_t blocks = 2u * uint32_t((g.w + kP2Core - 1) / kP2Core) *
                                     uint32_t((g.h + kP2Core - 1) / kP2Core);
-            hipLaunchKernelGGL(poisson2d_tile_kernel, dim3(blocks + (c.part ? 1u : 0u)),
-                               dim3(64 * kP2Waves), 0, ctx->stream, nd, src, g, done == 0 ? 1 : 0, run,
-                               dst, c);
+            const dim3 grid(blocks + (c.part ? 1u : 0u)), block(64 * kP2Waves);
+            if (done == 0)
+                hipLaunchKernelGGL(poisson2d_tile_kernel<true>, grid, block, 0, ctx->stream, nd, src, g, run,
+                                   dst, c);
+            else
+                hipLaunchKernelGGL(poisson2d_tile_kernel<false>, grid, block, 0, ctx->stream, nd, src, g, run,
+                                   dst, c);
             done += run;
         } else {
             hipLaunchKernelGGL(poisson2d_kernel, grid2(g), dim3(kBX, kBY), 0, ctx->stream, nd, src, g,
