@@ -845,8 +845,10 @@ __global__ __launch_bounds__(kCThreads) void poisson4_kernel(const float* __rest
 // and last row go through LDS, written in one step and read in the next, so
 // a step has one barrier for its K sweeps.  Rings of planes are indexed by
 // the unrolled step, so no value is moved.
-// FP32 issue bounds it (about 160 vector instructions a step for 16 updates a
-// thread).  Twelve sweeps, against six poisson2_kernel launches: 350 -> 204 us
+// Issue (about 160 vector instructions a step for 16 updates a thread) and the
+// chain within a step bound it, at the four waves a SIMD that its registers
+// leave: at 182x218x182 waves issue 37 to 40% of their cycles, wait to issue 21%
+// and for data 40%.  Twelve sweeps, against six poisson2_kernel launches: 350 -> 204 us
 // at 182x218x182, 245 -> 120 at 160x192x160, 75 -> 39 at 80x96x80.
 // ---------------------------------------------------------------------------
 constexpr int kMWaves = 8, kMR = 4, kMThreads = 64 * kMWaves, kMRows = kMWaves * kMR;
@@ -1179,7 +1181,9 @@ __device__ inline float3 ld3_rsrc(__amdgpu_buffer_rsrc_t r, uint32_t p)
 // The eight 12-byte corner gathers bind the address unit (a quad of lanes a
 // cycle or two), so large volumes stage cur on the tile grown by 2 in LDS and
 // gather there; a sample that leaves it (a displacement of a voxel or more, a
-// wrapped neighbour) is evaluated again from memory.  Then vector issue binds.
+// wrapped neighbour) is evaluated again from memory.  Then it is issue and the
+// latency of three phases at four waves a SIMD (issuing 33%, waiting to issue 22%
+// and for data 45% of the wave cycles, address unit 53% busy at 182x218x182).
 // Against the z-marching kernel without compose and compose_kernel after it:
 // 12.4 -> 5.1 us at 32x32x32, 24 -> 20 at 80x96x80, 177 -> 152 at
 // 182x218x182 (164 unstaged).
